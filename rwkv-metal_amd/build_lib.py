@@ -45,6 +45,8 @@ def _units():
         # result with VALU fmas, so accumulator registers only add copies
         units.append(("rq_qmv.hip", [f"-DRQ_BITS={b}", "-mllvm", "-amdgpu-mfma-vgpr-form=1"],
                       f"rq_qmv_b{b}.o"))
+        units.append(("rq_mid.hip", [f"-DRQ_BITS={b}", "-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+                      f"rq_mid_b{b}.o"))
         units.append(("rq_qmm.hip", [f"-DRQ_BITS={b}"], f"rq_qmm_b{b}.o"))
     return units
 

@@ -1,0 +1,525 @@
+// rq_mid.hip -- GEMMs on group-affine packed weights for batches of activation
+// rows that give the large-tile GEMMs (rq_qmm.hip) too few tiles to fill the
+// chip: short prompts, batched decode beyond the GEMV, short QLoRA batches.
+//
+//   qmm_t_mid : y[m, r] = sum_k x[m, k] * ŵ[r, k]     (transpose=True)
+//
+// (mx.quantized_matmul, rwkv_metal/lora/rwkvq_native.py:120-122, QuantizedLinear
+// inside LoRALinear, rwkv_metal/lora/lora.py:58-59.)
+//
+// Such a product moves a few MB and does well under a microsecond of matrix
+// work, so its time is memory round trips and the length of the longest serial
+// chain.  A block is one tile of 16*TM activation rows x 16*TN weight rows; its
+// waves (up to 16) each take a contiguous slice of the contraction, so that a
+// wave walks one to a few 128-element spans however long K is, and add their
+// fp32 tiles through LDS at the end, in wave order (deterministic).  Nothing is
+// shared before that: no barrier precedes the MFMAs.
+//  * A span is 128 codes of the 16 rows of an MFMA tile.  Lane L loads run L/16
+//    (32 codes, whole words at every bit width) of row L%16; lane groups 0 and
+//    1 load the span's scales and biases of row L%16 in one load and swaps hand
+//    them to all four.  The MFMAs contract k = 64 h + 16 (L/16) + 8 j .. +7 (half
+//    h, j = 0, 1): the packed words are spread over the lane groups with
+//    v_permlane16_swap / v_permlane32_swap (two swaps per pair of words) and
+//    dequantized there (ŵ = bf16(fma(scale, code, bias)), as the large GEMMs).
+//  * Activations go through a wave-private LDS tile, half a span at a time.  A
+//    load instruction whose neighbouring lanes read different rows costs one
+//    address cycle per lane; eight lanes per 128-byte line cost a quarter of
+//    it.  (Activations loaded straight in the MFMA operand's layout: [2048,
+//    2048] at M = 77 9.4 us against 7.2, [16384, 4096] 56 against 40.)
+//  * The weight fragment is the MFMA's A operand, so a lane ends with four
+//    consecutive outputs of one activation row.
+#include "rq_common.h"
+#include "rq_dequant.h"
+#include "rq_launch.h"
+
+#ifndef RQ_BITS
+#error "compile rq_mid.hip once per bit width with -DRQ_BITS=<bits>"
+#endif
+
+namespace {
+
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+typedef const __attribute__((address_space(1))) u32x4_t* gvec_t;
+typedef const __attribute__((address_space(1))) uint32_t* gword_t;
+typedef const __attribute__((address_space(1))) uint16_t* ghalf_t;
+typedef const __attribute__((address_space(1))) uint8_t* gbyte_t;
+// loads of less than their natural alignment
+typedef uint32_t u32_a2_t __attribute__((aligned(2)));
+typedef uint32_t u32x2_a2_t __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t u32x2_a4_t __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t u32x4_a4_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef const __attribute__((address_space(1))) u32_a2_t* gword_a2_t;
+typedef const __attribute__((address_space(1))) u32x2_a2_t* gvec2_a2_t;
+typedef const __attribute__((address_space(1))) u32x2_a4_t* gvec2_a4_t;
+typedef const __attribute__((address_space(1))) u32x4_a4_t* gvec_a4_t;
+
+struct MidArgs {
+    const uint8_t* x;
+    const uint32_t* wq;
+    const void* scales;
+    const void* biases;
+    void* y;
+    int64_t M, R, K;
+    int gs_shift, sb_f16, x_f16, y_dt, y_vec;
+    int tiles_m, tiles_n;
+    int spw;  // spans per wave
+    rq::LoraArgs lora;
+};
+
+// LDS bytes per wave
+__host__ __device__ constexpr int mid_wave_bytes(int tm, int tn) {
+    return (tn > 2 ? tm * tn : 2 * tm) * 1024;
+}
+
+// Swap of the odd lane groups of a with the even ones of b, then of lane
+// groups 2, 3 of a with 0, 1 of b.  With a, b the lower and upper half of each
+// lane group's piece list (group g: pieces 2g, 2g + 1), a ends with piece g and
+// b with piece 4 + g.
+RQ_DEV void spread_pieces(uint32_t& a, uint32_t& b) {
+    const auto r0 = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    const auto r1 = __builtin_amdgcn_permlane32_swap(r0[0], r0[1], false, false);
+    a = r1[0];
+    b = r1[1];
+}
+
+// One 16-row weight tile's span: the lane's run of codes, and in lane groups
+// 0 / 1 the raw scales / biases of the span's groups of row lr.
+template <int BITS, bool SB32>
+struct SpanRegs {
+    static constexpr int NW = SB32 ? 4 : 2;  // words of one array: up to four groups
+    uint32_t w[BITS];
+    uint32_t sb[NW];
+
+    RQ_DEV void load_codes(const uint8_t* wq, uint32_t off) {
+        const gbyte_t p = (gbyte_t)wq + off;
+        if constexpr (BITS == 4 || BITS == 8) {
+#pragma unroll
+            for (int i = 0; i < BITS / 4; ++i) {
+                const u32x4_t v = ((gvec_t)p)[i];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) w[4 * i + e] = v[e];
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < BITS; ++i) w[i] = ((gword_t)p)[i];
+        }
+    }
+    // ng: groups of this span in the row; 4 >> gsh unless the row ends in it.
+    // One load of all of them (rows of an odd number of groups are 2-byte
+    // aligned), element by element where the row ends.
+    RQ_DEV void load_sb(gbyte_t p, int gsh, int ng) {
+        if (ng == (4 >> gsh)) {
+            if constexpr (SB32) {
+                if (gsh == 0) {
+                    const u32x4_t v = *(gvec_a4_t)p;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sb[e] = v[e];
+                } else if (gsh == 1) {
+                    const u32x2_t v = *(gvec2_a4_t)p;
+                    sb[0] = v[0];
+                    sb[1] = v[1];
+                } else {
+                    sb[0] = *(gword_t)p;
+                }
+            } else {
+                if (gsh == 0) {
+                    const u32x2_t v = *(gvec2_a2_t)p;
+                    sb[0] = v[0];
+                    sb[1] = v[1];
+                } else if (gsh == 1) {
+                    sb[0] = *(gword_a2_t)p;
+                } else {
+                    sb[0] = *(ghalf_t)p;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < NW; ++i) {
+                sb[i] = 0;  // a weight past the row's end is 0
+                if constexpr (SB32) {
+                    if (i < ng) sb[i] = ((gword_t)p)[i];
+                } else {
+                    if (2 * i < ng) sb[i] = ((ghalf_t)p)[2 * i];
+                    if (2 * i + 1 < ng) sb[i] |= (uint32_t)((ghalf_t)p)[2 * i + 1] << 16;
+                }
+            }
+        }
+    }
+    // The weights as the fragments of four MFMAs: frag[2 h + j] holds, in lane
+    // (lg, lr), k = 64 h + 16 lg + 8 j .. +7 of row lr.
+    RQ_DEV void fragments(int gsh, int lg, bool f16, u32x4_t* frag) {
+        // the scales to every lane group, then the biases
+        uint32_t sv[NW], bv[NW];
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            const auto r0 = __builtin_amdgcn_permlane32_swap(sb[i], sb[i], false, false);
+            const auto r1 = __builtin_amdgcn_permlane16_swap(r0[0], r0[0], false, false);
+            sv[i] = r1[0];
+            bv[i] = r1[1];
+        }
+        if constexpr (BITS % 2 == 0) {
+            // 16 codes are BITS / 2 whole words: spread the packed words, then
+            // dequantize; group of the lane's codes of half h: (2 h + lg / 2) >> gsh
+            constexpr int HW = BITS / 2;
+            uint32_t p[2][HW];
+#pragma unroll
+            for (int i = 0; i < HW; ++i) {
+                p[0][i] = w[i];
+                p[1][i] = w[HW + i];
+                spread_pieces(p[0][i], p[1][i]);
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                uint32_t d[8];
+                const float s = value(sv, gsh, h, lg >> 1, f16), b = value(bv, gsh, h, lg >> 1, f16);
+                dequant_half_run<BITS>(p[h], s, b, d);
+                frag[2 * h] = u32x4_t{d[0], d[1], d[2], d[3]};
+                frag[2 * h + 1] = u32x4_t{d[4], d[5], d[6], d[7]};
+            }
+        } else {
+            // odd widths: dequantize the lane's own run (group lg >> gsh), then
+            // spread its 16 bf16 pairs
+            uint32_t d[16];
+            const float s0 = value(sv, gsh, 0, lg & 1, f16), s1 = value(sv, gsh, 1, lg & 1, f16);
+            const float b0 = value(bv, gsh, 0, lg & 1, f16), b1 = value(bv, gsh, 1, lg & 1, f16);
+            dequant_run_bf16<BITS>(w, lg < 2 ? s0 : s1, lg < 2 ? b0 : b1, d);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) spread_pieces(d[i], d[8 + i]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) frag[j] = u32x4_t{d[4 * j], d[4 * j + 1], d[4 * j + 2], d[4 * j + 3]};
+        }
+    }
+    // Value of run 2 h + o of the span (h wave-uniform, o per lane).
+    RQ_DEV static float value(const uint32_t* v, int gsh, int h, int o, bool f16) {
+        if constexpr (SB32) {
+            const uint32_t r = o ? v[2 * h + 1] : v[2 * h];
+            return __uint_as_float(gsh == 0 ? r : (gsh == 1 ? v[h] : v[0]));
+        } else {
+            const int sh = gsh == 0 ? 16 * o : (gsh == 1 ? 16 * h : 0);
+            const uint32_t r = ((gsh == 0 && h) ? v[1] : v[0]) >> sh;
+            return f16 ? f16_bits_to_f32(r & 0xffffu) : bf16_bits_to_f32(r);
+        }
+    }
+};
+
+// Eight consecutive activations of one row, as they are loaded.  XF: fp32
+// ones, rounded to bf16 (RNE) on their way to LDS; else 16-bit ones, f16
+// converted when `f16`.
+template <bool XF>
+struct XPiece {
+    u32x4_t v[XF ? 2 : 1];
+    RQ_DEV void load(const uint8_t* base, uint32_t off) {
+        const gbyte_t p = (gbyte_t)base + off;
+        v[0] = *(gvec_t)p;
+        if constexpr (XF) v[1] = *((gvec_t)p + 1);
+    }
+    RQ_DEV u32x4_t bf16(bool f16) const {
+        if constexpr (XF) {
+            return u32x4_t{pack_bf16x2(__uint_as_float(v[0][0]), __uint_as_float(v[0][1])),
+                           pack_bf16x2(__uint_as_float(v[0][2]), __uint_as_float(v[0][3])),
+                           pack_bf16x2(__uint_as_float(v[1][0]), __uint_as_float(v[1][1])),
+                           pack_bf16x2(__uint_as_float(v[1][2]), __uint_as_float(v[1][3]))};
+        } else {
+            u32x4_t r = v[0];
+            if (f16) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    r[e] = pack_bf16x2(f16_bits_to_f32(r[e] & 0xffffu), f16_bits_to_f32(r[e] >> 16));
+            }
+            return r;
+        }
+    }
+};
+
+// Four consecutive outputs of row m at columns n.. (rows >= M and columns >=
+// ld are not written).
+RQ_DEV void store_out4(const MidArgs& a, int64_t m, int64_t n, int64_t ld, f32x4_t v) {
+    if (m >= a.M) return;
+    const int64_t o = m * ld + n;
+    if (a.y_vec && n + 4 <= ld) {
+        if (a.y_dt == RQ_F32)
+            *(f32x4_t*)((float*)a.y + o) = v;
+        else
+            *(u32x2_t*)((uint16_t*)a.y + o) =
+                u32x2_t{pack2_dt(a.y_dt, v[0], v[1]), pack2_dt(a.y_dt, v[2], v[3])};
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (n + e < ld) store_dt(a.y, a.y_dt, o + e, v[e]);
+}
+
+// The QLoRA low-rank term of one 16x16 tile (outputs n0 + 4 lg .. +3 of row
+// m0 + lr): v += scale * z . L^T, z [M, rank] and L [ncols, rank] bf16.
+RQ_DEV f32x4_t add_lora(const rq::LoraArgs& lo, f32x4_t v, int64_t M, int64_t ncols, int64_t m0,
+                        int64_t n0, int lane) {
+    const int lg = lane >> 4, lr = lane & 15;
+    const int64_t m = m0 + lr, n = n0 + lr;
+    f32x4_t t = {0.f, 0.f, 0.f, 0.f};
+    for (int j0 = 0; j0 < lo.rank; j0 += 32) {
+        const int j = j0 + 8 * lg;
+        u32x4_t zf = {0u, 0u, 0u, 0u}, lf = zf;
+        if (j < lo.rank && m < M) zf = *(const u32x4_t*)((const uint16_t*)lo.z + m * lo.rank + j);
+        if (j < lo.rank && n < ncols) lf = *(const u32x4_t*)((const uint16_t*)lo.l + n * lo.rank + j);
+        t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, lf),
+                                                    __builtin_bit_cast(bf16x8_t, zf), t, 0, 0, 0);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = fmaf(lo.scale, t[e], v[e]);
+    return v;
+}
+
+// XD: halves of a span (64 k) of activations in flight ahead of the MFMAs.
+template <int BITS, bool SB32, bool XF, int TM, int TN, int MAXW, int XD>
+__global__ __launch_bounds__(64 * MAXW) void qmm_t_mid(const MidArgs a) {
+    // per wave: its activation tile of 64 k (2 KB per 16 rows), later its
+    // fp32 output tile [tile][lane]
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    constexpr int T = TM * TN;
+    constexpr int ES = XF ? 4 : 2;
+    constexpr int WB = mid_wave_bytes(TM, TN);
+    const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lg = lane >> 4, lr = lane & 15;
+    // consecutive blocks go to different XCDs: each XCD takes a contiguous
+    // range of tiles, the row tiles of one weight panel next to each other
+    const int nt = a.tiles_m * a.tiles_n, per = (nt + 7) >> 3;
+    const int t0 = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (t0 >= nt) return;
+    const int64_t n0 = (int64_t)(t0 / a.tiles_m) * (16 * TN), m0 = (int64_t)(t0 % a.tiles_m) * (16 * TM);
+
+    const int runs = (int)(a.K >> 5);
+    const int sp0 = wave * a.spw, nspan = (runs + 3) >> 2;
+    const int sp1 = sp0 + a.spw < nspan ? sp0 + a.spw : nspan;
+    const int64_t wpr = (int64_t)runs * BITS, G = a.K >> a.gs_shift;
+    const int gsh = a.gs_shift - 5;
+    constexpr int SBS = SB32 ? 4 : 2;
+
+    const uint8_t* wbase = (const uint8_t*)(a.wq + n0 * wpr);
+    uint32_t woff[TN];  // this lane's weight rows, the last row for those past it
+    gbyte_t sbp[TN];    // and their scales (even lane groups) or biases
+#pragma unroll
+    for (int b = 0; b < TN; ++b) {
+        const int left = a.R - n0 < 16 * TN ? (int)(a.R - n0) : 16 * TN;
+        const int nr = 16 * b + lr < left ? 16 * b + lr : left - 1;
+        woff[b] = (uint32_t)nr * (uint32_t)wpr * 4;
+        sbp[b] = (gbyte_t)((lg & 1) ? a.biases : a.scales) + ((n0 + nr) * G + ((4 * sp0) >> gsh)) * SBS;
+    }
+    SpanRegs<BITS, SB32> cur[TN], nxt[TN];
+    auto load_span = [&](SpanRegs<BITS, SB32>(&r)[TN], int sp) {
+        // a run past the row's end reads the last one; its k-steps are not run
+        const int run = 4 * sp + lg < runs ? 4 * sp + lg : runs - 1;
+#pragma unroll
+        for (int b = 0; b < TN; ++b) r[b].load_codes(wbase, woff[b] + run * BITS * 4);
+        if (lg < 2) {
+            const int left = (runs - 4 * sp + (1 << gsh) - 1) >> gsh, ng = 4 >> gsh;
+#pragma unroll
+            for (int b = 0; b < TN; ++b)
+                r[b].load_sb(sbp[b] + (int64_t)((4 * (sp - sp0)) >> gsh) * SBS, gsh, left < ng ? left : ng);
+        }
+    };
+    // Activations: load q covers rows 8q .. 8q+7 of the tile, 64 k (one whole
+    // 128-byte line a row in 16 bits): eight consecutive lanes read one row.
+    // Groups of rows past M repeat the last one.
+    const int qlast = (a.M - m0 < 16 * TM ? (int)(a.M - m0) - 1 : 16 * TM - 1) >> 3;
+    const int rem = a.M - m0 - 8 * qlast < 8 ? (int)(a.M - m0) - 8 * qlast : 8;
+    const int xr = lane >> 3, xc = lane & 7;
+    const uint32_t xfull = (uint32_t)xr * (uint32_t)a.K * ES;
+    const uint32_t xpart = (uint32_t)(xr < rem ? xr : rem - 1) * (uint32_t)a.K * ES;
+    const uint8_t* xbase = a.x + m0 * a.K * ES;
+    XPiece<XF> xv[XD][2 * TM];
+    auto load_x = [&](XPiece<XF>(&v)[2 * TM], int half) {  // half: index of the 64 k
+        // a k past the row's end reads the half's first 32 (never used)
+        const int c = 64 * half + 8 * xc < a.K ? xc : xc & 3;
+        const uint32_t ko = (64 * half + 8 * c) * ES;
+#pragma unroll
+        for (int q = 0; q < 2 * TM; ++q) {
+            const int qe = q < qlast ? q : qlast;
+            v[q].load(xbase + (int64_t)(8 * qe) * a.K * ES, (qe == qlast ? xpart : xfull) + ko);
+        }
+    };
+    // LDS tile: 16-byte chunk c of row r at (c ^ (r & 7)), 128 bytes a row
+    uint8_t* xs = lds + wave * WB;
+    uint8_t* xw = xs + xr * 128 + ((xc ^ xr) << 4);
+    const uint32_t xrd = wave * WB + lr * 128 + (((2 * lg) ^ (lr & 7)) << 4);
+
+    f32x4_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int b = 0; b < TN; ++b) acc[i][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    const int h1 = 2 * sp1 < (runs + 1) >> 1 ? 2 * sp1 : (runs + 1) >> 1;  // halves of the slice end here
+    load_span(cur, sp0);
+#pragma unroll
+    for (int d = 0; d < XD; ++d)
+        if (2 * sp0 + d < h1) load_x(xv[d], 2 * sp0 + d);
+    for (int sp = sp0; sp < sp1; ++sp) {
+        if (sp + 1 < sp1) load_span(nxt, sp + 1);
+        u32x4_t wf[TN][4];
+#pragma unroll
+        for (int b = 0; b < TN; ++b) cur[b].fragments(gsh, lg, a.sb_f16, wf[b]);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int half = 2 * sp + h;
+            if (half < h1) {
+                // x past the row's end is 0
+                if (64 * half + 64 > a.K && xc >= 4) {
+#pragma unroll
+                    for (int q = 0; q < 2 * TM; ++q) *(u32x4_t*)(xw + q * 1024) = u32x4_t{0u, 0u, 0u, 0u};
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 2 * TM; ++q) *(u32x4_t*)(xw + q * 1024) = xv[h % XD][q].bf16(a.x_f16);
+                }
+                if (half + XD < h1) load_x(xv[h % XD], half + XD);
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) {
+                        const bf16x8_t xf = __builtin_bit_cast(
+                            bf16x8_t, *(const u32x4_t*)(lds + (xrd ^ (16 * j)) + i * 2048));
+#pragma unroll
+                        for (int b = 0; b < TN; ++b)
+                            acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                __builtin_bit_cast(bf16x8_t, wf[b][2 * h + j]), xf, acc[i][b], 0, 0, 0);
+                    }
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < TN; ++b) cur[b] = nxt[b];
+    }
+
+    if (nw > 1) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int b = 0; b < TN; ++b)
+                *(f32x4_t*)(xs + ((i * TN + b) * 64 + lane) * 16) = acc[i][b];
+        __syncthreads();
+        for (int t = wave; t < T; t += nw) {
+            const uint8_t* p = lds + (t * 64 + lane) * 16;
+            f32x4_t v = *(const f32x4_t*)p;
+            for (int w = 1; w < nw; ++w) {
+                const f32x4_t u = *(const f32x4_t*)(p + w * WB);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] += u[e];
+            }
+            const int64_t m = m0 + 16 * (t / TN), n = n0 + 16 * (t % TN);
+            if (a.lora.z) v = add_lora(a.lora, v, a.M, a.R, m, n, lane);
+            store_out4(a, m + lr, n + 4 * lg, a.R, v);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int b = 0; b < TN; ++b) {
+                const int64_t m = m0 + 16 * i, n = n0 + 16 * b;
+                f32x4_t v = acc[i][b];
+                if (a.lora.z) v = add_lora(a.lora, v, a.M, a.R, m, n, lane);
+                store_out4(a, m + lr, n + 4 * lg, a.R, v);
+            }
+    }
+}
+
+}  // namespace
+
+namespace rq {
+
+#define RQ_CAT2(a, b) a##b
+#define RQ_CAT(a, b) RQ_CAT2(a, b)
+
+// Tiles: 16*tm activation rows x 16*tn weight rows, `waves` at most, and the
+// measured time per 128-wide span of a CU that runs one block of it (us; 4-bit
+// codes, bf16 activations, from [2048, 2048] against [2048, 8192]).  A wave
+// dequantizes tn weight tiles and stages tm activation tiles per span, so wide
+// tiles do less per output, and small ones fill the chip.
+struct MidTile {
+    int tm, tn, waves;
+    double span_us;
+};
+static constexpr MidTile kMidTiles[] = {{1, 1, 16, 0.123}, {2, 1, 16, 0.177}, {3, 1, 16, 0.204},
+                                        {2, 2, 16, 0.233}, {4, 2, 8, 0.305},  {3, 4, 8, 0.43},
+                                        {4, 4, 8, 0.479}};
+
+// The tile with the least rounds x spans x time per span, plus the launch and
+// the sum over the waves (3 + 0.2 us per 16x16 tile of the block).
+static int mid_pick(int64_t m, int64_t n_out, int64_t k, double* us) {
+    int best = 0;
+    double bt = 1e30;
+    for (int i = 0; i < (int)(sizeof(kMidTiles) / sizeof(kMidTiles[0])); ++i) {
+        const MidTile& t = kMidTiles[i];
+        const int64_t blocks = ((m + 16 * t.tm - 1) / (16 * t.tm)) * ((n_out + 16 * t.tn - 1) / (16 * t.tn));
+        const double c = 3.0 + 0.2 * t.tm * t.tn +
+                         (double)((blocks + 255) / 256) * (double)((k + 127) / 128) * t.span_us;
+        if (c < bt) {
+            bt = c;
+            best = i;
+        }
+    }
+    if (us) *us = bt;
+    return best;
+}
+
+template <bool SB32, bool XF, int TM, int TN, int MAXW>
+static hipError_t launch_mid_t(MidArgs& a, hipStream_t stream) {
+    a.tiles_m = (int)((a.M + 16 * TM - 1) / (16 * TM));
+    a.tiles_n = (int)((a.R + 16 * TN - 1) / (16 * TN));
+    const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
+    const int nspan = (int)((a.K + 127) / 128);
+    // about MAXW waves a CU, at least 4 a block ([16384, 4096] at M = 128, two
+    // 4x4 blocks a CU: 38 us with 4 waves, 42 with 8; [8192, 2048] at M = 200
+    // 21 against 25)
+    const int q = (int)((tiles + 255) / 256);
+    const int maxw = MAXW / q > 4 ? MAXW / q : 4;
+    a.spw = (nspan + maxw - 1) / maxw;
+    const int nw = (nspan + a.spw - 1) / a.spw;
+    // activations in flight: two halves of a span where the registers allow
+    constexpr int XD = !XF && TN == 1 ? 2 : 1;
+    hipLaunchKernelGGL((qmm_t_mid<RQ_BITS, SB32, XF, TM, TN, MAXW, XD>),
+                       dim3((unsigned)(((tiles + 7) / 8) * 8)), dim3(64 * nw),
+                       nw * mid_wave_bytes(TM, TN), stream, a);
+    return hipGetLastError();
+}
+
+template <bool SB32, bool XF>
+static hipError_t launch_mid_t_tile(MidArgs& a, int tile, hipStream_t stream) {
+    switch (tile) {
+        case 0: return launch_mid_t<SB32, XF, 1, 1, 16>(a, stream);
+        case 1: return launch_mid_t<SB32, XF, 2, 1, 16>(a, stream);
+        case 2: return launch_mid_t<SB32, XF, 3, 1, 16>(a, stream);
+        case 3: return launch_mid_t<SB32, XF, 2, 2, 16>(a, stream);
+        case 4: return launch_mid_t<SB32, XF, 4, 2, 8>(a, stream);
+        case 5: return launch_mid_t<SB32, XF, 3, 4, 8>(a, stream);
+        default: return launch_mid_t<SB32, XF, 4, 4, 8>(a, stream);
+    }
+}
+
+hipError_t RQ_CAT(launch_qmm_t_mid_b, RQ_BITS)(const void* x, int x_dt, const uint32_t* wq,
+                                          const void* scales, const void* biases, int sb_dt,
+                                          int64_t m, int64_t rows, int64_t cols, int gs, void* y,
+                                          int y_dt, hipStream_t stream, const LoraArgs* lora) {
+    MidArgs a{};
+    a.x = (const uint8_t*)x;
+    a.wq = wq;
+    a.scales = scales;
+    a.biases = biases;
+    a.y = y;
+    a.M = m;
+    a.R = rows;
+    a.K = cols;
+    a.gs_shift = __builtin_ctz(gs);
+    a.sb_f16 = sb_dt == RQ_F16;
+    a.x_f16 = x_dt == RQ_F16;
+    a.y_dt = y_dt;
+    const int ysz = y_dt == RQ_F32 ? 16 : 8;  // four outputs
+    a.y_vec = ((uintptr_t)y & (ysz - 1)) == 0 && rows % 4 == 0;
+    if (lora) a.lora = *lora;
+    const int tile = mid_pick(m, rows, cols, nullptr);
+    if (sb_dt == RQ_F32)
+        return x_dt == RQ_F32 ? launch_mid_t_tile<true, true>(a, tile, stream)
+                              : launch_mid_t_tile<true, false>(a, tile, stream);
+    return x_dt == RQ_F32 ? launch_mid_t_tile<false, true>(a, tile, stream)
+                          : launch_mid_t_tile<false, false>(a, tile, stream);
+}
+
+}  // namespace rq

@@ -8,22 +8,21 @@
 // w.r.t. x, which MLX autograd emits for the QLoRA backward
 // (rwkv_metal/lora/finetune.py:141).
 //
-// Design: block tile BM x 128 outputs, 64 contraction elements per stage,
-// 4 waves in a 2x2 arrangement, v_mfma_f32_16x16x32_bf16 with fp32
-// accumulators.  Packed weights are dequantized ONCE per block per stage in
-// registers (ŵ = bf16(fma(scale, code, bias))) and written to LDS as bf16;
-// the activation tile is converted to bf16 on its way to LDS.  LDS is double
-// buffered and the next stage's global loads are issued before the current
-// stage's MFMAs.
+// Fewer than 256 activation rows of a forward product run rq_mid.hip.
 //
-//  * qmm_t: the packed axis K is the contraction axis, so a thread's 32-code
-//    run lands as one 64-byte row segment of the B tile (row-major [n][k]).
-//  * qmm_n: the contraction runs over the weight rows, so the B tile is
-//    stored transposed ([k][r]); a thread dequantizes the same run of two
-//    adjacent rows and writes (row, row+1) pairs as one dword per k.
+// qmm_n (qmm_n_kernel) covers the transposed products outside the 64-wide-stage
+// kernels below: block tile BM x 128 outputs, 64 weight rows per stage, 4 waves
+// in a 2x2 arrangement, v_mfma_f32_16x16x32_bf16 with fp32 accumulators.  Packed
+// weights are dequantized once per block per stage in registers (ŵ =
+// bf16(fma(scale, code, bias))) and written to LDS as bf16, transposed ([k][r]):
+// the contraction runs over the weight rows, and a thread dequantizes the same
+// run of two adjacent rows and writes (row, row+1) pairs as one dword per k.
+// LDS is double buffered and the next stage's global loads are issued before
+// the current stage's MFMAs.
 #include <type_traits>
 
 #include "rq_common.h"
+#include "rq_dequant.h"
 #include "rq_launch.h"
 
 #ifndef RQ_BITS
@@ -37,21 +36,8 @@ constexpr int BK = 64;        // contraction elements per stage
 constexpr int LDS_LD = BK + 8;  // LDS row stride in bf16 elements (144 B)
 constexpr int BN = 128;       // output columns per block
 
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-
 RQ_DEV bf16x8_t lds_frag(const uint16_t* p) {
     return __builtin_bit_cast(bf16x8_t, *(const u32x4_t*)p);
-}
-
-// One run of 32 codes -> 16 dwords of bf16 pairs, ŵ = bf16(scale*code + bias).
-template <int BITS>
-RQ_DEV void dequant_run_bf16(const uint32_t* words, float s, float b, uint32_t* out) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const float lo = fmaf(s, (float)run_code<BITS>(words, 2 * i), b);
-        const float hi = fmaf(s, (float)run_code<BITS>(words, 2 * i + 1), b);
-        out[i] = pack_bf16x2(lo, hi);
-    }
 }
 
 // Load 32 activations x[row][col0 .. col0+31] (row length ld elements) as 16
@@ -92,112 +78,6 @@ RQ_DEV void store_16dw(uint16_t* lds, const uint32_t* d) {
     u32x4_t* p = (u32x4_t*)lds;
 #pragma unroll
     for (int q = 0; q < 4; ++q) p[q] = u32x4_t{d[4 * q], d[4 * q + 1], d[4 * q + 2], d[4 * q + 3]};
-}
-
-// ----------------------------------------------------------------- qmm_t
-
-template <int BITS, int XDT, int BM>
-__global__ __launch_bounds__(kBlock) void qmm_t_kernel(
-    const void* __restrict__ x, const uint32_t* __restrict__ wq, const void* __restrict__ scales,
-    const void* __restrict__ biases, int sb_dt, int64_t M, int64_t R, int64_t K, int gs_shift,
-    void* __restrict__ y, int y_dt) {
-    constexpr int TM = BM / 32;  // 16-row MFMA tiles per wave along m (wave covers BM/2)
-    constexpr int TN = 4;        // wave covers 64 output columns
-    constexpr int AR = BM / 128; // activation rows loaded per thread per stage
-    __shared__ __attribute__((aligned(16))) uint16_t As[2][BM * LDS_LD];
-    __shared__ __attribute__((aligned(16))) uint16_t Bs[2][BN * LDS_LD];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int lg = lane >> 4, lr = lane & 15;
-    const int64_t m0 = (int64_t)blockIdx.y * BM, n0 = (int64_t)blockIdx.x * BN;
-    const int64_t runs_per_row = K >> 5, wpr = runs_per_row * BITS, G = K >> gs_shift;
-    const int nst = (int)((runs_per_row + 1) >> 1);
-    const int half = tid & 1;           // which run of the stage this thread loads
-    const int64_t brow = n0 + (tid >> 1);
-
-    uint32_t cw[BITS];
-    float sc = 0.f, bi = 0.f;
-    uint32_t xa[AR][16];
-
-    auto gload = [&](int st) {
-        const int64_t run = 2 * (int64_t)st + half;
-        const bool run_ok = run < runs_per_row;
-        if (run_ok && brow < R) {
-            load_run<BITS>(wq + brow * wpr + run * BITS, cw);
-            const int64_t gi = brow * G + (run >> (gs_shift - 5));
-            sc = load_dt(scales, sb_dt, gi);
-            bi = load_dt(biases, sb_dt, gi);
-        } else {
-#pragma unroll
-            for (int w = 0; w < BITS; ++w) cw[w] = 0u;
-            sc = 0.f;
-            bi = 0.f;
-        }
-#pragma unroll
-        for (int i = 0; i < AR; ++i) {
-            const int64_t arow = m0 + (tid >> 1) + 128 * i;
-            if (run_ok && arow < M) {
-                load_act_run<XDT>(x, arow, K, run * 32, K, true, xa[i]);
-            } else {
-#pragma unroll
-                for (int q = 0; q < 16; ++q) xa[i][q] = 0u;
-            }
-        }
-    };
-    auto swrite = [&](int buf) {
-        uint32_t d[16];
-        dequant_run_bf16<BITS>(cw, sc, bi, d);
-        store_16dw(&Bs[buf][(tid >> 1) * LDS_LD + half * 32], d);
-#pragma unroll
-        for (int i = 0; i < AR; ++i)
-            store_16dw(&As[buf][((tid >> 1) + 128 * i) * LDS_LD + half * 32], xa[i]);
-    };
-
-    f32x4_t acc[TM][TN];
-#pragma unroll
-    for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int b = 0; b < TN; ++b) acc[a][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-    gload(0);
-    swrite(0);
-    __syncthreads();
-    for (int st = 0; st < nst; ++st) {
-        const int buf = st & 1;
-        if (st + 1 < nst) gload(st + 1);
-#pragma unroll
-        for (int ks = 0; ks < BK / 32; ++ks) {
-            bf16x8_t af[TM], bf[TN];
-#pragma unroll
-            for (int a = 0; a < TM; ++a)
-                af[a] = lds_frag(&As[buf][(wm * (BM / 2) + a * 16 + lr) * LDS_LD + ks * 32 + lg * 8]);
-#pragma unroll
-            for (int b = 0; b < TN; ++b)
-                bf[b] = lds_frag(&Bs[buf][(wn * 64 + b * 16 + lr) * LDS_LD + ks * 32 + lg * 8]);
-#pragma unroll
-            for (int a = 0; a < TM; ++a)
-#pragma unroll
-                for (int b = 0; b < TN; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bf[b], acc[a][b],
-                                                                        0, 0, 0);
-        }
-        if (st + 1 < nst) swrite(buf ^ 1);
-        __syncthreads();
-    }
-
-    // D[4*lg + i][lr] of each 16x16 tile: rows are m, columns are n.
-#pragma unroll
-    for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int b = 0; b < TN; ++b) {
-            const int64_t n = n0 + wn * 64 + b * 16 + lr;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int64_t m = m0 + wm * (BM / 2) + a * 16 + 4 * lg + i;
-                if (m < M && n < R) store_dt(y, y_dt, m * R + n, acc[a][b][i]);
-            }
-        }
 }
 
 // ----------------------------------------------------------------- qmm_n
@@ -338,54 +218,6 @@ __global__ __launch_bounds__(kBlock) void qmm_n_kernel(
 // stage's global loads are issued before the current stage's MFMAs.
 // Blocks are assigned to tiles so that each XCD works on a contiguous run of
 // tiles (shared activation rows and weight rows stay in that XCD's L2).
-
-// Eight 4-bit codes of one word -> 4 dwords of bf16 pairs (codes 0,1 .. 6,7),
-// ŵ = bf16(s*code + b).  gfx950's v_cvt_scalef32_pk_f32_fp8 turns two bytes
-// into two fp32 values in one instruction: an e4m3 byte 0x0q is exactly
-// q / 512 (its subnormals and first binade are evenly spaced, 2^-9 apart),
-// and the conversion applies only the exponent of its scale (measured on
-// the box), so a scale of 512 gives q exactly.  Per 8 codes: 3 mask ops, 4
-// converts, 8 fmas, 4 packs (byte converts took 8 converts).
-RQ_DEV void dequant_word4(uint32_t word, float s, float b, uint32_t* out) {
-    typedef float f32x2_t __attribute__((ext_vector_type(2)));
-    const uint32_t lo = word & 0x0F0F0F0Fu;         // codes 0,2,4,6
-    const uint32_t hi = (word >> 4) & 0x0F0F0F0Fu;  // codes 1,3,5,7
-    const f32x2_t l0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 512.f, false);
-    const f32x2_t l1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 512.f, true);
-    const f32x2_t h0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 512.f, false);
-    const f32x2_t h1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 512.f, true);
-    out[0] = pack_bf16x2(fmaf(s, l0[0], b), fmaf(s, h0[0], b));
-    out[1] = pack_bf16x2(fmaf(s, l0[1], b), fmaf(s, h0[1], b));
-    out[2] = pack_bf16x2(fmaf(s, l1[0], b), fmaf(s, h1[0], b));
-    out[3] = pack_bf16x2(fmaf(s, l1[1], b), fmaf(s, h1[1], b));
-}
-
-// One run of 32 codes -> 16 dwords of bf16 pairs, ŵ = bf16(scale*code + bias):
-// 4-bit codes by dequant_word4, 8-bit ones by byte converts
-// (v_cvt_f32_ubyte0..3; the bytes are hidden from the optimiser by an empty
-// asm, otherwise it folds each byte select into a bit-field extract, a second
-// VALU op per code in front of a v_cvt_f32_ubyte0).
-template <int BITS>
-RQ_DEV void dequant_run_fast(const uint32_t* words, float s, float b, uint32_t* out) {
-    if constexpr (BITS == 4) {
-#pragma unroll
-        for (int w = 0; w < 4; ++w) dequant_word4(words[w], s, b, out + 4 * w);
-    } else if constexpr (BITS == 8) {
-#pragma unroll
-        for (int w = 0; w < 8; ++w) {
-            uint32_t v = words[w];
-            asm("" : "+v"(v));
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const float c0 = (float)(uint8_t)(v >> (16 * i));
-                const float c1 = (float)(uint8_t)(v >> (16 * i + 8));
-                out[2 * w + i] = pack_bf16x2(fmaf(s, c0, b), fmaf(s, c1, b));
-            }
-        }
-    } else {
-        dequant_run_bf16<BITS>(words, s, b, out);
-    }
-}
 
 template <int BITS, int XDT, int BN>
 __global__ __launch_bounds__(kBlock, 1) void qmm_t_big(
@@ -896,11 +728,6 @@ __global__ __launch_bounds__(kWsBlock, 1) void qmm_t_ws(
         }
 }
 
-
-// Two outputs of dtype dt (bf16 or f16) packed in one dword, RNE.
-RQ_DEV uint32_t pack2_dt(int dt, float lo, float hi) {
-    return dt == RQ_BF16 ? pack_bf16x2(lo, hi) : (f32_to_f16_bits(lo) | (f32_to_f16_bits(hi) << 16));
-}
 
 // Store one wave's 128 x WN output tile of a k64 GEMM.  The MFMAs ran with
 // the weight fragment as the A operand, so lane (lg = lane / 16, lr =
@@ -1942,10 +1769,23 @@ namespace rq {
 #define RQ_CAT2(a, b) a##b
 #define RQ_CAT(a, b) RQ_CAT2(a, b)
 
+// rq_mid.hip
+hipError_t RQ_CAT(launch_qmm_t_mid_b, RQ_BITS)(const void* x, int x_dt, const uint32_t* wq,
+                                          const void* scales, const void* biases, int sb_dt,
+                                          int64_t m, int64_t rows, int64_t cols, int gs, void* y,
+                                          int y_dt, hipStream_t stream, const LoraArgs* lora);
+
 hipError_t RQ_CAT(launch_qmm_t_b, RQ_BITS)(const void* x, int x_dt, const uint32_t* wq,
                                       const void* scales, const void* biases, int sb_dt,
                                       int64_t m, int64_t rows, int64_t cols, int gs, void* y,
                                       int y_dt, hipStream_t stream, const LoraArgs* lora) {
+    // Fewer than 256 rows: small tiles, the contraction split over the waves of
+    // a block.  (128 x 128 tiles of the same dequantization, one block walking
+    // all of K, took 58 us on [2048, 2048] and 220 on [2048, 8192] at M = 77,
+    // on 16 CUs; these take 7 and 17.)  Offsets inside a tile are 32-bit.
+    if (m < 256 && cols <= kMidMaxCols && !lora)
+        return RQ_CAT(launch_qmm_t_mid_b, RQ_BITS)(x, x_dt, wq, scales, biases, sb_dt, m, rows, cols,
+                                              gs, y, y_dt, stream, lora);
     const int gs_shift = __builtin_ctz(gs);
     const LoraArgs lo = lora ? *lora : LoraArgs{nullptr, nullptr, 0, 0.f};
     // bf16 or fp32 activations (fp32 rounded to bf16 as the producers stage them)
@@ -2067,7 +1907,7 @@ hipError_t RQ_CAT(launch_qmm_t_b, RQ_BITS)(const void* x, int x_dt, const uint32
 #undef RQ_DMA
         return hipGetLastError();
     }
-    if (m >= 256) {
+    {
         // weight-row tile: whole rounds over 256 CUs at M=4096 for the RWKV-7 shapes
         const int bn = rows % 160 == 0 ? 160 : 128;
         const int tm = (int)((m + 255) / 256);
@@ -2081,12 +1921,6 @@ hipError_t RQ_CAT(launch_qmm_t_b, RQ_BITS)(const void* x, int x_dt, const uint32
 #undef RQ_BIG
         return hipGetLastError();
     }
-    constexpr int BM = 128;
-    const dim3 grid((unsigned)((rows + BN - 1) / BN), (unsigned)((m + BM - 1) / BM));
-    RQ_DISPATCH_DT(x_dt, XD,
-        hipLaunchKernelGGL((qmm_t_kernel<RQ_BITS, XD, BM>), grid, dim3(kBlock), 0, stream, x, wq,
-                           scales, biases, sb_dt, m, rows, cols, gs_shift, y, y_dt));
-    return hipGetLastError();
 }
 
 // Split-K form of the 64-wide-stage GEMM (transpose=1; the caller checked the
