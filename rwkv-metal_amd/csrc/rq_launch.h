@@ -135,8 +135,8 @@ hipError_t launch_lora_grads(const void* x, const void* u, const void* dy, const
                              void* db, const LoraGradPlan& p, void* work, hipStream_t stream,
                              bool xdy_f32 = false);
 
-// The short-batch GEMMs (rq_mid.hip) take contractions up to this length.
-constexpr int64_t kMidMaxCols = 1 << 25;
+// The short-batch GEMMs (rq_mid.hip) take weights of up to this many rows and columns.
+constexpr int64_t kMidMaxCols = 1 << 26;
 
 // MFMA GEMM, transpose=True: y[m, rows] = x[m, cols] . W^T.
 hipError_t launch_qmm_t(const void* x, int x_dt, const uint32_t* wq, const void* scales,

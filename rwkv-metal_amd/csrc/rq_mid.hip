@@ -3,9 +3,11 @@
 // chip: short prompts, batched decode beyond the GEMV, short QLoRA batches.
 //
 //   qmm_t_mid : y[m, r] = sum_k x[m, k] * ŵ[r, k]     (transpose=True)
+//   qmm_n_mid : y[m, k] = sum_r x[m, r] * ŵ[r, k]     (transpose=False, dX = dY·W)
 //
 // (mx.quantized_matmul, rwkv_metal/lora/rwkvq_native.py:120-122, QuantizedLinear
-// inside LoRALinear, rwkv_metal/lora/lora.py:58-59.)
+// inside LoRALinear, rwkv_metal/lora/lora.py:58-59, and its VJP w.r.t. x,
+// rwkv_metal/lora/finetune.py:141.)
 //
 // Such a product moves a few MB and does well under a microsecond of matrix
 // work, so its time is memory round trips and the length of the longest serial
@@ -52,6 +54,8 @@ typedef const __attribute__((address_space(1))) u32_a2_t* gword_a2_t;
 typedef const __attribute__((address_space(1))) u32x2_a2_t* gvec2_a2_t;
 typedef const __attribute__((address_space(1))) u32x2_a4_t* gvec2_a4_t;
 typedef const __attribute__((address_space(1))) u32x4_a4_t* gvec_a4_t;
+typedef uint32_t u32x4_a2_t __attribute__((ext_vector_type(4), aligned(2)));
+typedef const __attribute__((address_space(1))) u32x4_a2_t* gvec_a2_t;
 
 struct MidArgs {
     const uint8_t* x;
@@ -210,8 +214,22 @@ struct XPiece {
     u32x4_t v[XF ? 2 : 1];
     RQ_DEV void load(const uint8_t* base, uint32_t off) {
         const gbyte_t p = (gbyte_t)base + off;
-        v[0] = *(gvec_t)p;
-        if constexpr (XF) v[1] = *((gvec_t)p + 1);
+        v[0] = *(gvec_a2_t)p;
+        if constexpr (XF) v[1] = *((gvec_a2_t)p + 1);
+    }
+    // the first n of them (n < 8), zeros beyond
+    RQ_DEV void load_part(const uint8_t* base, uint32_t off, int n) {
+        const gbyte_t p = (gbyte_t)base + off;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if constexpr (XF) {
+                v[0][e] = e < n ? ((gword_t)p)[e] : 0u;
+                v[1][e] = 4 + e < n ? ((gword_t)p)[4 + e] : 0u;
+            } else {
+                v[0][e] = (2 * e < n ? (uint32_t)((ghalf_t)p)[2 * e] : 0u) |
+                          (2 * e + 1 < n ? (uint32_t)((ghalf_t)p)[2 * e + 1] << 16 : 0u);
+            }
+        }
     }
     RQ_DEV u32x4_t bf16(bool f16) const {
         if constexpr (XF) {
@@ -421,6 +439,282 @@ __global__ __launch_bounds__(64 * MAXW) void qmm_t_mid(const MidArgs a) {
     }
 }
 
+// ------------------------------------------------------------- qmm_n_mid
+//
+// y[m, k] = sum_r x[m, r] * ŵ[r, k].  The contraction runs over the weight
+// rows, the packed codes along k.  The MFMA's output index along k is free to
+// be any permutation of the tile's columns, so no transpose is needed: lane
+// (lg, lr) holds the NC (8 or 4) codes at columns NC lr .. of the rows 8 lg ..
+// +7 of a 32-row step, and the c-th of NC MFMAs contracts those 32 rows for the
+// columns {NC lr + c}, its operand the c-th code of the lane's eight rows.  A
+// block is a tile of 16*TM activation rows x 16*NC columns; its waves take
+// contiguous slices of the weight rows and add their tiles through LDS in wave
+// order.  A load instruction reads 4 rows x 16*NC codes.  (The codes loaded as
+// whole row segments and read back through LDS: the same times; what bounds it
+// is the ~2.5 VALU instructions per code, and with few columns the number of
+// blocks, since a block dequantizes all rows of its columns.)
+// The step's scales and biases (32 rows x the tile's groups) come in one load
+// and go through wave-private LDS as fp32 pairs; activations are staged as in
+// qmm_t_mid, 64 weight rows at a time.
+
+// NC (4 or 8) consecutive codes of one row in one load: the bytes they fill at
+// 2, 4 and 8 bits, else two words of the run shifted so that they start at bit 0.
+template <int BITS, int NC>
+struct Codes {
+    static constexpr int NB = BITS * NC;  // bits
+    static constexpr bool SH = BITS == 3 || BITS >= 5 && BITS < 8;
+    static constexpr int NW = SH || NB > 32 ? 2 : 1;
+    uint32_t w[NW];
+    // piece p of a run: byte offset of the load within the run, and the shift
+    RQ_DEV static int offset(int p) {
+        if constexpr (!SH) return p * (NB / 8);
+        const int o = (p * NB) >> 5;
+        return 4 * (o < BITS - 2 ? o : BITS - 2);
+    }
+    RQ_DEV static int shift(int p) {
+        if constexpr (!SH) return 0;
+        return p * NB - 8 * offset(p);
+    }
+    RQ_DEV void load(const uint8_t* base, uint32_t off) {
+        const gbyte_t p = (gbyte_t)base + off;
+        if constexpr (NW == 2) {
+            const u32x2_t v = *(gvec2_a4_t)p;
+            w[0] = v[0];
+            w[1] = v[1];
+        } else if constexpr (NB == 32) {
+            w[0] = *(gword_t)p;
+        } else if constexpr (NB == 16) {
+            w[0] = *(ghalf_t)p;
+        } else {
+            static_assert(NB == 8, "");
+            w[0] = *p;
+        }
+    }
+    // scale * code + bias, fp32
+    RQ_DEV void values(int sh, float s, float b, float* out) const {
+        if constexpr (BITS == 4) {
+            typedef float f32x2_t __attribute__((ext_vector_type(2)));
+            const uint32_t lo = w[0] & 0x0F0F0F0Fu, hi = (w[0] >> 4) & 0x0F0F0F0Fu;
+#pragma unroll
+            for (int i = 0; i < NC / 4; ++i) {
+                const f32x2_t l = i ? __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 512.f, true)
+                                    : __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 512.f, false);
+                const f32x2_t h = i ? __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 512.f, true)
+                                    : __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 512.f, false);
+                out[4 * i] = fmaf(s, l[0], b);
+                out[4 * i + 1] = fmaf(s, h[0], b);
+                out[4 * i + 2] = fmaf(s, l[1], b);
+                out[4 * i + 3] = fmaf(s, h[1], b);
+            }
+        } else if constexpr (BITS == 8) {
+#pragma unroll
+            for (int h = 0; h < NC / 4; ++h) {
+                uint32_t v = w[h];
+                asm("" : "+v"(v));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) out[4 * h + i] = fmaf(s, (float)(uint8_t)(v >> (8 * i)), b);
+            }
+        } else if constexpr (BITS == 2) {
+#pragma unroll
+            for (int i = 0; i < NC; ++i) out[i] = fmaf(s, (float)((w[0] >> (2 * i)) & 3u), b);
+        } else {
+            const uint64_t v = (((uint64_t)w[1] << 32) | w[0]) >> sh;
+            const uint32_t d[2] = {(uint32_t)v, (uint32_t)(v >> 32)};
+#pragma unroll
+            for (int i = 0; i < NC; ++i) out[i] = fmaf(s, (float)run_code<BITS>(d, i), b);
+        }
+    }
+};
+
+// LDS of a wave: activations (2 KB per 16 rows) and the (scale, bias) pairs of
+// a step (256 B per group); later 16x16 tiles of its fp32 output, `pass` row
+// tiles at a time.
+__host__ __device__ constexpr int mid_n_pass(int tm, int nc) { return tm * nc <= 16 ? tm : 16 / nc; }
+__host__ __device__ constexpr int mid_n_wave_bytes(int tm, int nc) {
+    const int in = 2048 * tm + 256 * (nc / 2), out = 1024 * nc * mid_n_pass(tm, nc);
+    return in > out ? in : out;
+}
+// fp32 row stride of the block's output tile
+__host__ __device__ constexpr int mid_n_out_row(int nc) { return 16 * nc + 4; }
+__host__ __device__ constexpr int mid_n_out_bytes(int tm, int nc) {
+    return 16 * mid_n_pass(tm, nc) * mid_n_out_row(nc) * 4;
+}
+
+template <int BITS, bool SB32, bool XF, int TM, int NC, int MAXW>
+__global__ __launch_bounds__(64 * MAXW) void qmm_n_mid(const MidArgs a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    constexpr int ES = XF ? 4 : 2, SBS = SB32 ? 4 : 2, CT = 16 * NC;
+    constexpr int WB = mid_n_wave_bytes(TM, NC), TP = mid_n_pass(TM, NC);
+    const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lg = lane >> 4, lr = lane & 15;
+    const int nt = a.tiles_m * a.tiles_n, per = (nt + 7) >> 3;
+    const int t0 = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (t0 >= nt) return;
+    const int64_t c0 = (int64_t)(t0 / a.tiles_m) * CT, m0 = (int64_t)(t0 % a.tiles_m) * (16 * TM);
+
+    const int64_t wpr = (a.K >> 5) * BITS, G = a.K >> a.gs_shift;
+    const int gsh = a.gs_shift - 5;
+    const int nhalf = (int)((a.R + 63) >> 6);  // 64 weight rows each
+    const int h0 = wave * a.spw, h1 = h0 + a.spw < nhalf ? h0 + a.spw : nhalf;
+
+    // codes: piece lr of the tile, the last piece of the row for those past it
+    constexpr int PR = 32 / NC;  // pieces of a run
+    const int pieces = a.K - c0 < CT ? (int)(a.K - c0) / NC : 16;
+    const int pc = lr < pieces ? lr : pieces - 1;
+    const uint8_t* wbase = (const uint8_t*)a.wq + (c0 >> 5) * (BITS * 4);
+    const uint32_t wcol = (uint32_t)(pc / PR) * (BITS * 4) + Codes<BITS, NC>::offset(pc % PR);
+    const uint32_t woff = (uint32_t)(8 * lg) * (uint32_t)wpr * 4 + wcol;
+    const int csh = Codes<BITS, NC>::shift(pc % PR);
+    // scales (lanes 0-31) and biases (lanes 32-63) of row lane % 32 of a step;
+    // the tile's groups are those of a 128-wide span of twice the group size at NC = 4
+    const int gst = NC == 8 ? gsh : (gsh < 2 ? gsh + 1 : 2);
+    const int ngf = 4 >> gst, ngl = (int)(G - (c0 >> a.gs_shift)), ng = ngl < ngf ? ngl : ngf;
+    const gbyte_t sbp = (gbyte_t)(lane < 32 ? a.scales : a.biases) + (c0 >> a.gs_shift) * SBS;
+
+    Codes<BITS, NC> cw[2][8];
+    SpanRegs<BITS, SB32> sbr[2];  // only its scale words are used
+    auto load_step = [&](Codes<BITS, NC>(&c)[8], SpanRegs<BITS, SB32>& sb, int step) {
+        const int64_t r0 = 32 * (int64_t)step;
+        if (r0 + 32 <= a.R) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) c[i].load(wbase + (r0 + i) * wpr * 4, woff);
+        } else {  // rows past the end repeat the last one (x is 0 there)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int64_t r = r0 + 8 * lg + i < a.R ? r0 + 8 * lg + i : a.R - 1;
+                c[i].load(wbase + r * wpr * 4, wcol);
+            }
+        }
+        const int64_t sr = r0 + (lane & 31) < a.R ? r0 + (lane & 31) : a.R - 1;
+        sb.load_sb(sbp + sr * G * SBS, gst, ng);
+    };
+    // activations: as in qmm_t_mid, k -> weight row
+    const int qlast = (a.M - m0 < 16 * TM ? (int)(a.M - m0) - 1 : 16 * TM - 1) >> 3;
+    const int rem = a.M - m0 - 8 * qlast < 8 ? (int)(a.M - m0) - 8 * qlast : 8;
+    const int xr = lane >> 3, xc = lane & 7;
+    const uint32_t xfull = (uint32_t)xr * (uint32_t)a.R * ES;
+    const uint32_t xpart = (uint32_t)(xr < rem ? xr : rem - 1) * (uint32_t)a.R * ES;
+    const uint8_t* xbase = a.x + m0 * a.R * ES;
+    XPiece<XF> xv[2 * TM];
+    auto load_x = [&](int half) {
+        const uint32_t ko = (uint32_t)(64 * half + 8 * xc) * ES;
+        if (64 * (int64_t)half + 64 <= a.R) {
+#pragma unroll
+            for (int q = 0; q < 2 * TM; ++q) {
+                const int qe = q < qlast ? q : qlast;
+                xv[q].load(xbase + (int64_t)(8 * qe) * a.R * ES, (qe == qlast ? xpart : xfull) + ko);
+            }
+        } else {
+            const int left = (int)(a.R - 64 * (int64_t)half) - 8 * xc;  // zeros past the last row
+#pragma unroll
+            for (int q = 0; q < 2 * TM; ++q) {
+                const int qe = q < qlast ? q : qlast;
+                xv[q].load_part(xbase + (int64_t)(8 * qe) * a.R * ES, (qe == qlast ? xpart : xfull) + ko,
+                                left < 8 ? left : 8);
+            }
+        }
+    };
+    uint8_t* xs = lds + wave * WB;
+    uint8_t* xw = xs + xr * 128 + ((xc ^ xr) << 4);
+    const uint32_t xrd = wave * WB + lr * 128 + ((lg ^ (lr & 7)) << 4);
+    // (scale, bias) pairs of a step: [group][row] behind the activations
+    uint8_t* sbw = xs + TM * 2048 + (lane & 31) * 8 + (lane >> 5) * 4;
+    const uint8_t* sbrd = xs + TM * 2048 + ((NC * lr) >> a.gs_shift) * 256 + lg * 64;
+
+    f32x4_t acc[TM][NC];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[i][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    const int nstep = (int)((a.R + 31) >> 5), s1 = 2 * h1 < nstep ? 2 * h1 : nstep;
+    load_step(cw[0], sbr[0], 2 * h0);
+    load_x(h0);
+    for (int half = h0; half < h1; ++half) {
+#pragma unroll
+        for (int q = 0; q < 2 * TM; ++q) *(u32x4_t*)(xw + q * 1024) = xv[q].bf16(a.x_f16);
+        if (half + 1 < h1) load_x(half + 1);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int step = 2 * half + j;
+            if (step < s1) {
+                if (step + 1 < s1) load_step(cw[j ^ 1], sbr[j ^ 1], step + 1);
+#pragma unroll
+                for (int g = 0; g < NC / 2; ++g) {
+                    if (g < ngf) {
+                        float v;
+                        if constexpr (SB32) {
+                            v = __uint_as_float(sbr[j].sb[g]);
+                        } else {
+                            const uint32_t h = (g & 1) ? sbr[j].sb[g >> 1] >> 16 : sbr[j].sb[g >> 1] & 0xffffu;
+                            v = a.sb_f16 ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
+                        }
+                        *(float*)(sbw + g * 256) = v;
+                    }
+                }
+                f32x4_t sb[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sb[i] = *(const f32x4_t*)(sbrd + 16 * i);
+                uint32_t wf[NC][4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    float v0[NC], v1[NC];
+                    cw[j][2 * i].values(csh, sb[i][0], sb[i][1], v0);
+                    cw[j][2 * i + 1].values(csh, sb[i][2], sb[i][3], v1);
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) wf[c][i] = pack_bf16x2(v0[c], v1[c]);
+                }
+#pragma unroll
+                for (int i = 0; i < TM; ++i) {
+                    const bf16x8_t xf =
+                        __builtin_bit_cast(bf16x8_t, *(const u32x4_t*)(lds + (xrd ^ (64 * j)) + i * 2048));
+#pragma unroll
+                    for (int c = 0; c < NC; ++c)
+                        acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            __builtin_bit_cast(bf16x8_t, u32x4_t{wf[c][0], wf[c][1], wf[c][2], wf[c][3]}), xf,
+                            acc[i][c], 0, 0, 0);
+                }
+            }
+        }
+    }
+
+    // D element (row 4 lg + e, column lr) of MFMA c: column NC (4 lg + e) + c of
+    // row lr.  TP row tiles a pass: the waves' tiles, their sums into the
+    // block's tile [16 TP][CT], then its 16x16 pieces.
+    constexpr int OR = mid_n_out_row(NC);
+    float* out = (float*)(lds + nw * WB);
+#pragma unroll
+    for (int p = 0; p < TM; p += TP) {
+        if (p) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < TP; ++i)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) *(f32x4_t*)(xs + ((i * NC + c) * 64 + lane) * 16) = acc[p + i][c];
+        __syncthreads();
+        for (int t = wave; t < NC * TP; t += nw) {
+            const uint8_t* q = lds + (t * 64 + lane) * 16;
+            f32x4_t v = *(const f32x4_t*)q;
+            for (int w = 1; w < nw; ++w) {
+                const f32x4_t u = *(const f32x4_t*)(q + w * WB);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] += u[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                out[(16 * (t / NC) + lr) * OR + NC * (4 * lg + e) + t % NC] = v[e];
+        }
+        __syncthreads();
+        for (int t = wave; t < NC * TP; t += nw) {
+            const int64_t m = m0 + 16 * (p + t / NC), n = c0 + 16 * (t % NC);
+            if (m >= a.M || n >= a.K) continue;
+            f32x4_t v = *(const f32x4_t*)(out + (16 * (t / NC) + lr) * OR + 16 * (t % NC) + 4 * lg);
+            if (a.lora.z) v = add_lora(a.lora, v, a.M, a.K, m, n, lane);
+            store_out4(a, m + lr, n + 4 * lg, a.K, v);
+        }
+    }
+}
+
 }  // namespace
 
 namespace rq {
@@ -494,10 +788,9 @@ static hipError_t launch_mid_t_tile(MidArgs& a, int tile, hipStream_t stream) {
     }
 }
 
-hipError_t RQ_CAT(launch_qmm_t_mid_b, RQ_BITS)(const void* x, int x_dt, const uint32_t* wq,
-                                          const void* scales, const void* biases, int sb_dt,
-                                          int64_t m, int64_t rows, int64_t cols, int gs, void* y,
-                                          int y_dt, hipStream_t stream, const LoraArgs* lora) {
+static MidArgs mid_args(const void* x, int x_dt, const uint32_t* wq, const void* scales,
+                        const void* biases, int sb_dt, int64_t m, int64_t rows, int64_t cols, int gs,
+                        void* y, int y_dt, int64_t n_out, const LoraArgs* lora) {
     MidArgs a{};
     a.x = (const uint8_t*)x;
     a.wq = wq;
@@ -512,14 +805,83 @@ hipError_t RQ_CAT(launch_qmm_t_mid_b, RQ_BITS)(const void* x, int x_dt, const ui
     a.x_f16 = x_dt == RQ_F16;
     a.y_dt = y_dt;
     const int ysz = y_dt == RQ_F32 ? 16 : 8;  // four outputs
-    a.y_vec = ((uintptr_t)y & (ysz - 1)) == 0 && rows % 4 == 0;
+    a.y_vec = ((uintptr_t)y & (ysz - 1)) == 0 && n_out % 4 == 0;
     if (lora) a.lora = *lora;
+    return a;
+}
+
+hipError_t RQ_CAT(launch_qmm_t_mid_b, RQ_BITS)(const void* x, int x_dt, const uint32_t* wq,
+                                          const void* scales, const void* biases, int sb_dt,
+                                          int64_t m, int64_t rows, int64_t cols, int gs, void* y,
+                                          int y_dt, hipStream_t stream, const LoraArgs* lora) {
+    MidArgs a = mid_args(x, x_dt, wq, scales, biases, sb_dt, m, rows, cols, gs, y, y_dt, rows, lora);
     const int tile = mid_pick(m, rows, cols, nullptr);
     if (sb_dt == RQ_F32)
         return x_dt == RQ_F32 ? launch_mid_t_tile<true, true>(a, tile, stream)
                               : launch_mid_t_tile<true, false>(a, tile, stream);
     return x_dt == RQ_F32 ? launch_mid_t_tile<false, true>(a, tile, stream)
                           : launch_mid_t_tile<false, false>(a, tile, stream);
+}
+
+// qmm_n_mid tiles: 16*tm activation rows x 16*nc columns, the time per 64 weight
+// rows as above (us; [2048, 2048] against [8192, 2048]).
+static constexpr MidTile kMidNTiles[] = {{1, 4, 16, 0.22}, {2, 4, 8, 0.282}, {3, 4, 8, 0.29},
+                                         {4, 4, 8, 0.322}, {2, 8, 8, 0.322}};
+
+static int mid_n_pick(int64_t m, int64_t n_out, int64_t r) {
+    int best = 0;
+    double bt = 1e30;
+    for (int i = 0; i < (int)(sizeof(kMidNTiles) / sizeof(kMidNTiles[0])); ++i) {
+        const MidTile& t = kMidNTiles[i];
+        const int64_t blocks = ((m + 16 * t.tm - 1) / (16 * t.tm)) * ((n_out + 16 * t.tn - 1) / (16 * t.tn));
+        const double c = 3.0 + 0.12 * t.tm * t.tn +
+                         (double)((blocks + 255) / 256) * (double)((r + 63) / 64) * t.span_us;
+        if (c < bt) {
+            bt = c;
+            best = i;
+        }
+    }
+    return best;
+}
+
+template <bool SB32, bool XF, int TM, int NC, int MAXW>
+static hipError_t launch_mid_n(MidArgs& a, hipStream_t stream) {
+    a.tiles_m = (int)((a.M + 16 * TM - 1) / (16 * TM));
+    a.tiles_n = (int)((a.K + 16 * NC - 1) / (16 * NC));
+    const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
+    const int nhalf = (int)((a.R + 63) / 64);
+    const int q = (int)((tiles + 255) / 256);
+    const int maxw = MAXW / q > 4 ? MAXW / q : 4;
+    a.spw = (nhalf + maxw - 1) / maxw;
+    const int nw = (nhalf + a.spw - 1) / a.spw;
+    hipLaunchKernelGGL((qmm_n_mid<RQ_BITS, SB32, XF, TM, NC, MAXW>),
+                       dim3((unsigned)(((tiles + 7) / 8) * 8)), dim3(64 * nw),
+                       nw * mid_n_wave_bytes(TM, NC) + mid_n_out_bytes(TM, NC), stream, a);
+    return hipGetLastError();
+}
+
+template <bool SB32, bool XF>
+static hipError_t launch_mid_n_tile(MidArgs& a, int tile, hipStream_t stream) {
+    switch (tile) {
+        case 0: return launch_mid_n<SB32, XF, 1, 4, 16>(a, stream);
+        case 1: return launch_mid_n<SB32, XF, 2, 4, 8>(a, stream);
+        case 2: return launch_mid_n<SB32, XF, 3, 4, 8>(a, stream);
+        case 3: return launch_mid_n<SB32, XF, 4, 4, 8>(a, stream);
+        default: return launch_mid_n<SB32, XF, 2, 8, 8>(a, stream);
+    }
+}
+
+hipError_t RQ_CAT(launch_qmm_n_mid_b, RQ_BITS)(const void* x, int x_dt, const uint32_t* wq,
+                                          const void* scales, const void* biases, int sb_dt,
+                                          int64_t m, int64_t rows, int64_t cols, int gs, void* y,
+                                          int y_dt, hipStream_t stream, const LoraArgs* lora) {
+    MidArgs a = mid_args(x, x_dt, wq, scales, biases, sb_dt, m, rows, cols, gs, y, y_dt, cols, lora);
+    const int tile = mid_n_pick(m, cols, rows);
+    if (sb_dt == RQ_F32)
+        return x_dt == RQ_F32 ? launch_mid_n_tile<true, true>(a, tile, stream)
+                              : launch_mid_n_tile<true, false>(a, tile, stream);
+    return x_dt == RQ_F32 ? launch_mid_n_tile<false, true>(a, tile, stream)
+                          : launch_mid_n_tile<false, false>(a, tile, stream);
 }
 
 }  // namespace rq

@@ -1770,6 +1770,10 @@ namespace rq {
 #define RQ_CAT(a, b) RQ_CAT2(a, b)
 
 // rq_mid.hip
+hipError_t RQ_CAT(launch_qmm_n_mid_b, RQ_BITS)(const void* x, int x_dt, const uint32_t* wq,
+                                          const void* scales, const void* biases, int sb_dt,
+                                          int64_t m, int64_t rows, int64_t cols, int gs, void* y,
+                                          int y_dt, hipStream_t stream, const LoraArgs* lora);
 hipError_t RQ_CAT(launch_qmm_t_mid_b, RQ_BITS)(const void* x, int x_dt, const uint32_t* wq,
                                           const void* scales, const void* biases, int sb_dt,
                                           int64_t m, int64_t rows, int64_t cols, int gs, void* y,
@@ -2033,6 +2037,14 @@ hipError_t RQ_CAT(launch_qmm_n_b, RQ_BITS)(const void* x, int x_dt, const uint32
     }
 #undef RQ_NK64
     if (lora) return hipErrorNotSupported;  // the low-rank term rides on the k64 kernels only
+    // Everything else: small tiles over wave slices of the contraction.  (128 x
+    // 128 tiles, one block walking all weight rows, took 44 us on [768, 768] at
+    // M = 200, on 12 CUs, and 3.6 us per 64 rows and round at any size; these
+    // take 5.9, and 0.32 per 64 rows of a 64 x 64 tile.)  Offsets inside a tile
+    // are 32-bit.
+    if (rows <= kMidMaxCols && cols <= kMidMaxCols)
+        return RQ_CAT(launch_qmm_n_mid_b, RQ_BITS)(x, x_dt, wq, scales, biases, sb_dt, m, rows, cols,
+                                              gs, y, y_dt, stream, nullptr);
     constexpr int BM = 128;
     const dim3 grid((unsigned)((cols + BN - 1) / BN), (unsigned)((m + BM - 1) / BM));
     const int gs_shift = __builtin_ctz(gs);

@@ -99,3 +99,58 @@ def test_mid_forward_infinite_rows_stay_in_their_row(rq, dev):
     assert torch.equal(torch.isinf(y), torch.isinf(ref))
     assert torch.isfinite(y[[i for i in range(m) if i != 3]]).all()
     assert torch.equal(y[3].sign(), ref[3].sign().float())
+
+
+# m, rows, cols of the transposed product: each tile, contractions (rows) that
+# are no multiple of 64, 32 or 8, columns that end inside a tile
+N_TILES = [(1, 1, 32), (17, 7, 64), (255, 33, 96), (130, 2049, 2080), (200, 515, 2048),
+           (200, 1000, 4128), (60, 203, 8192), (60, 1000, 16384), (77, 130, 16416),
+           (250, 1000, 2080), (300, 77, 800)]
+
+
+@pytest.mark.parametrize("xdt,sdt", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32),
+                                     (torch.float32, torch.bfloat16), (torch.float16, torch.float16),
+                                     (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("m,R,K", N_TILES)
+def test_mid_transposed_tiles(rq, dev, m, R, K, xdt, sdt):
+    gs = 32
+    (wq, s, b), w = packed(rq, dev, R, K, gs, 4, sdt, m + R)
+    x = torch.randn(m, R, generator=torch.Generator().manual_seed(m)).to(xdt).to(dev)
+    print("mid transposed", m, R, K, xdt, sdt, flush=True)
+    y = rq.quantized_matmul(x, wq, s, b, False, gs, 4)
+    check(y, (x.bfloat16().double() @ w, out_dtype(xdt, sdt)), R, "mid transposed")
+
+
+@pytest.mark.parametrize("sdt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("groups", [1, 2, 3, 5, 8])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("bits", [2, 3, 4, 5, 6, 8])
+def test_mid_transposed_groups(rq, dev, bits, gs, groups, sdt):
+    K = groups * gs
+    for m, R in ((37, 77), (100, 640)):
+        (wq, s, b), w = packed(rq, dev, R, K, gs, bits, sdt, bits + groups)
+        x = torch.randn(m, R, generator=torch.Generator().manual_seed(gs)).to(dev)
+        print("mid transposed groups", bits, gs, groups, sdt, flush=True)
+        y = rq.quantized_matmul(x, wq, s, b, False, gs, bits)
+        check(y, (x.bfloat16().double() @ w, torch.float32), R, "mid transposed groups")
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 5, 6, 8])
+def test_mid_transposed_wide_tiles(rq, dev, bits):
+    """The 128-column tile of every bit width."""
+    m, R, K = 77, 130, 16384 + 32
+    (wq, s, b), w = packed(rq, dev, R, K, 32, bits, torch.bfloat16, bits)
+    x = torch.randn(m, R, generator=torch.Generator().manual_seed(3)).to(dev)
+    y = rq.quantized_matmul(x, wq, s, b, False, 32, bits)
+    check(y, (x.bfloat16().double() @ w, torch.float32), R, "mid transposed 128")
+
+
+def test_mid_transposed_infinite_rows_stay_in_their_row(rq, dev):
+    m, R, K = 20, 45, 96
+    (wq, s, b), w = packed(rq, dev, R, K, 32, 4, torch.bfloat16, 9)
+    x = torch.randn(m, R, generator=torch.Generator().manual_seed(1))
+    x[3, R - 1] = float("inf")
+    y = rq.quantized_matmul(x.to(dev), wq, s, b, False, 32, 4)
+    ref = x.to(dev).double() @ w
+    assert torch.equal(torch.isinf(y), torch.isinf(ref))
+    assert torch.isfinite(y[[i for i in range(m) if i != 3]]).all()
