@@ -14,6 +14,7 @@
 
 #include "../../include/rwkvq.h"
 #include "rq_launch.h"
+#include "rq_mid.h"
 
 namespace rq {
 
@@ -298,6 +299,11 @@ static SplitKPlan splitk_plan(int64_t m, int64_t rows, int64_t cols, int gs, int
             }
         }
     }
+    // the short-batch tiles split the contraction inside a block ([768, 3072] at
+    // M = 512 15.3 -> 11.4 us; [2048, 8192] stays split, 33 against 36)
+    double mid;
+    rq::mid_pick(m, rows, cols, bits, &mid);
+    if (mid < 0.9 * (bt + 2.8)) best.splits = 1;
     return best;
 }
 
@@ -527,6 +533,29 @@ static bool qlora_two_launch(int x_dt, int bits, int64_t rank, int64_t m, int64_
            m >= 256 && n_in % 32 == 0 && n_out >= 4096 && n_out >= 2 * n_in;
 }
 
+// Products that the in-kernel down-projection does not cover (fewer than 256
+// rows, other ranks and bit widths) as two launches where the GEMM takes the
+// term: z (fp32 x not rounded first), then the GEMM with the term in its output
+// stage.  `stored`: the adapters as rq_qlora_dx has them.
+static hipError_t qlora_two_pass(int transpose, const void* x, int x_dt, const uint32_t* w_q,
+                                 const void* scales, const void* biases, int sb_dt, int64_t m,
+                                 int64_t rows, int64_t cols, int gs, int bits, const void* a,
+                                 const void* lora, int rank, float scale, void* z, void* y, int y_dt,
+                                 bool stored, hipStream_t stream) {
+    const int64_t n_in = transpose ? cols : rows;
+    if (!z || n_in % 32 || (x_dt != RQ_BF16 && x_dt != RQ_F32)) return hipErrorNotSupported;
+    if (cols > rq::kMidMaxCols || (!transpose && rows > rq::kMidMaxCols)) return hipErrorNotSupported;
+    rq::LoraArgs lo{z, lora, rank, scale};
+    lo.stored = stored;
+    lo.l_ld = cols;
+    lo.mid = true;
+    const hipError_t e =
+        rq::launch_lora_down(x, m, n_in, a, rank, z, stream, stored, x_dt == RQ_F32 ? 2 : 0);
+    if (e != hipSuccess) return e;
+    return rq::launch_qmm(transpose, x, x_dt, w_q, scales, biases, sb_dt, m, rows, cols, gs, bits, y,
+                          y_dt, stream, &lo);
+}
+
 int rq_qlora(const void* x, rq_dtype x_dt, const uint32_t* w_q, const void* scales,
              const void* biases, rq_dtype sb_dt, int64_t m, int64_t rows, int64_t cols,
              int group_size, int bits, int transpose, const void* a, const void* lora,
@@ -546,7 +575,7 @@ int rq_qlora(const void* x, rq_dtype x_dt, const uint32_t* w_q, const void* scal
     hipError_t e;
     if (z_out && qlora_two_launch(x_dt, bits, rank, m, n_in, n_out)) {
         e = rq::launch_lora_down(x, m, n_in, a, (int)rank, z_out, (hipStream_t)stream,
-                                 /*a_t=*/false, x_dt == RQ_F32);
+                                 /*a_t=*/false, x_dt == RQ_F32 ? 1 : 0);
         rq::LoraArgs lo{z_out, lora, (int)rank, scale};
         if (e == hipSuccess)
             e = rq::launch_qmm(transpose, x, x_dt, w_q, scales, biases, sb_dt, m, rows, cols,
@@ -560,11 +589,13 @@ int rq_qlora(const void* x, rq_dtype x_dt, const uint32_t* w_q, const void* scal
                            group_size, bits, y, y_dt, (hipStream_t)stream, &lo);
     }
     if (e == hipErrorNotSupported)
+        e = qlora_two_pass(transpose, x, x_dt, w_q, scales, biases, sb_dt, m, rows, cols, group_size,
+                           bits, a, lora, (int)rank, scale, z_out, y, y_dt, false, (hipStream_t)stream);
+    if (e == hipErrorNotSupported)
         return fail(RQ_EUNSUPPORTED,
-                    "rq_qlora: the in-kernel down-projection covers rank 16 with 4- or 8-bit codes "
-                    "on the 64-wide-stage GEMMs (bf16 or fp32 x, m >= 256, 16-bit 16-byte aligned scales; "
-                    "transpose=1: cols a multiple of 8 groups; transpose=0: rows %% 64 == 0, "
-                    "cols %% 128 == 0); use rq_lora_down and rq_qmm_lora");
+                    "rq_qlora: needs bf16 or fp32 x and, outside the in-kernel down-projection (rank 16, "
+                    "4- or 8-bit codes, m >= 256, the 64-wide-stage GEMMs), z_out and a contraction "
+                    "that is a multiple of 32; use rq_lora_down and rq_qmm_lora");
     return launch_status(e, "rq_qlora");
 }
 
@@ -591,7 +622,7 @@ int rq_qlora_dx(const void* dy, rq_dtype dy_dt, const uint32_t* w_q, const void*
     hipError_t e;
     if (u_out && qlora_two_launch(dy_dt, bits, rank, m, rows, cols)) {
         e = rq::launch_lora_down(dy, m, rows, lora_b, (int)rank, u_out, (hipStream_t)stream,
-                                 /*a_t=*/true, dy_dt == RQ_F32);
+                                 /*a_t=*/true, dy_dt == RQ_F32 ? 1 : 0);
         rq::LoraArgs lo{u_out, lora_a, (int)rank, scale};
         lo.stored = true;
         lo.l_ld = cols;
@@ -609,11 +640,14 @@ int rq_qlora_dx(const void* dy, rq_dtype dy_dt, const uint32_t* w_q, const void*
                            bits, dx, dx_dt, (hipStream_t)stream, &lo);
     }
     if (e == hipErrorNotSupported)
+        e = qlora_two_pass(0, dy, dy_dt, w_q, scales, biases, sb_dt, m, rows, cols, group_size, bits,
+                           lora_b, lora_a, (int)rank, scale, u_out, dx, dx_dt, true,
+                           (hipStream_t)stream);
+    if (e == hipErrorNotSupported)
         return fail(RQ_EUNSUPPORTED,
-                    "rq_qlora_dx: the in-kernel down-projection covers rank 16 with 4- or 8-bit "
-                    "codes on the 64-wide-stage transposed GEMM (bf16 or fp32 dy, m >= 256, "
-                    "16-bit 16-byte aligned scales, rows %% 64 == 0, cols %% 128 == 0); use "
-                    "rq_lora_down and rq_qmm_lora");
+                    "rq_qlora_dx: needs bf16 or fp32 dy and, outside the in-kernel down-projection "
+                    "(rank 16, 4- or 8-bit codes, m >= 256, the 64-wide-stage transposed GEMM), u_out "
+                    "and rows %% 32 == 0; use rq_lora_down and rq_qmm_lora");
     return launch_status(e, "rq_qlora_dx");
 }
 

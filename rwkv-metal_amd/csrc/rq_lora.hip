@@ -23,8 +23,12 @@
 //    from two gfx950 ds_read_b64_tr_b16 (source lane 4 s + c of a 16-lane
 //    group reads ranks 4 c .. +3 of row s).  The sums are the same as with a,
 //    in the same order.
-//  * XF: x is fp32; each 8-value chunk is loaded as 32 bytes and rounded to
+//  * XM = 1: x is fp32; each 8-value chunk is loaded as 32 bytes and rounded to
 //    bf16 (RNE) before its MFMA, so z equals the bf16(x) launch's bit for bit.
+//  * XM = 2: fp32 x enters as two bf16 values, hi = bf16(x) and lo = bf16(x -
+//    hi) (16 significant bits), one MFMA each: z is that of the fp32 x within
+//    its own rounding to bf16 (an fp32 matmul with its casts took four torch
+//    launches, ~25 us of GPU time at M = 200, K = 768, rank 32; this 4-5 us).
 #include <mutex>
 
 #include "rq_common.h"
@@ -38,19 +42,20 @@ namespace {
 // hold more per k-step and batch 2 at rank 16).  Wave w sums k-steps w,
 // w + W, .. in order and the waves are summed in order, so the bits depend
 // on W alone: the forms of one rank share it.
-template <int RT, bool AT = false, bool XF = false> struct LoraShape {
+template <int RT, bool AT = false, int XM = 0> struct LoraShape {
     static constexpr int W = RT == 1 ? 16 : 8;
-    static constexpr int U = (RT == 1 && (AT || XF)) ? 2 : (RT <= 2 ? 4 : 2);
+    static constexpr int U = (RT == 1 && (AT || XM)) ? 2 : (RT <= 2 ? 4 : 2);
 };
 
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
-template <int RT, bool AT = false, bool XF = false>  // rank tiles of 16; AT: a given as
-                                                    // a^T [K, rank]; XF: fp32 x
-__global__ __launch_bounds__((64 * LoraShape<RT, AT, XF>::W)) void lora_down_kernel(
+template <int RT, bool AT = false, int XM = 0>  // rank tiles of 16; AT: a given as a^T
+                                               // [K, rank]; XM: 1, 2 for fp32 x
+__global__ __launch_bounds__((64 * LoraShape<RT, AT, XM>::W)) void lora_down_kernel(
     const void* __restrict__ x, int64_t M, int64_t K, const uint16_t* __restrict__ a,
     uint16_t* __restrict__ z) {
-    constexpr int kLoraWaves = LoraShape<RT, AT, XF>::W, U = LoraShape<RT, AT, XF>::U;
+    constexpr int kLoraWaves = LoraShape<RT, AT, XM>::W, U = LoraShape<RT, AT, XM>::U;
+    constexpr bool XF = XM != 0;
     constexpr int RANK = 16 * RT;
     __shared__ __attribute__((aligned(16))) float red[kLoraWaves][RT][4][64];
     __shared__ __attribute__((aligned(16))) uint8_t slab[AT ? kLoraWaves : 1][AT ? 64 * RANK : 16];
@@ -93,13 +98,21 @@ __global__ __launch_bounds__((64 * LoraShape<RT, AT, XF>::W)) void lora_down_ker
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (s0 + kLoraWaves * u < nsteps) {
-                u32x4_t xv = xa[b][u][0];
+                u32x4_t xv = xa[b][u][0], xl = {0u, 0u, 0u, 0u};
                 if constexpr (XF) {
                     const u32x4_t p = xa[b][u][0], q = xa[b][u][1];
                     xv = u32x4_t{pack_bf16x2(__uint_as_float(p[0]), __uint_as_float(p[1])),
                                  pack_bf16x2(__uint_as_float(p[2]), __uint_as_float(p[3])),
                                  pack_bf16x2(__uint_as_float(q[0]), __uint_as_float(q[1])),
                                  pack_bf16x2(__uint_as_float(q[2]), __uint_as_float(q[3]))};
+                    if constexpr (XM == 2) {
+                        auto rest = [](uint32_t h, uint32_t f0, uint32_t f1) {
+                            return pack_bf16x2(__uint_as_float(f0) - __uint_as_float(h << 16),
+                                               __uint_as_float(f1) - __uint_as_float(h & 0xffff0000u));
+                        };
+                        xl = u32x4_t{rest(xv[0], p[0], p[1]), rest(xv[1], p[2], p[3]),
+                                     rest(xv[2], q[0], q[1]), rest(xv[3], q[2], q[3])};
+                    }
                 }
                 const bf16x8_t av = __builtin_bit_cast(bf16x8_t, xv);
                 if constexpr (AT) {
@@ -125,6 +138,9 @@ __global__ __launch_bounds__((64 * LoraShape<RT, AT, XF>::W)) void lora_down_ker
                     } else {
                         bv = __builtin_bit_cast(bf16x8_t, wb[b][u][t]);
                     }
+                    if constexpr (XM == 2)
+                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            __builtin_bit_cast(bf16x8_t, xl), bv, acc[t], 0, 0, 0);
                     acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc[t], 0, 0, 0);
                 }
             }
@@ -482,24 +498,26 @@ hipError_t launch_lora_grads(const void* x, const void* u, const void* dy, const
 }
 
 hipError_t launch_lora_down(const void* x, int64_t m, int64_t k, const void* a, int rank, void* z,
-                            hipStream_t stream, bool a_t, bool x_f32) {
+                            hipStream_t stream, bool a_t, int x_mode) {
     const int blocks = (int)((m + 15) / 16);
     if (blocks == 0) return hipSuccess;
     const dim3 grid(blocks);
     const uint16_t* ap = (const uint16_t*)a;
     uint16_t* zp = (uint16_t*)z;
-#define RQ_DOWN_X(RT, ATV)                                                                         \
-    if (x_f32)                                                                                     \
-        hipLaunchKernelGGL((lora_down_kernel<RT, ATV, true>), grid,                                \
-                           dim3(64 * LoraShape<RT, ATV, true>::W), 0, stream, x, m, k, ap, zp);    \
-    else                                                                                           \
-        hipLaunchKernelGGL((lora_down_kernel<RT, ATV, false>), grid,                               \
-                           dim3(64 * LoraShape<RT, ATV, false>::W), 0, stream, x, m, k, ap, zp);
+#define RQ_DOWN_X(RT, ATV, XMV)                                                                    \
+    hipLaunchKernelGGL((lora_down_kernel<RT, ATV, XMV>), grid,                                     \
+                       dim3(64 * LoraShape<RT, ATV, XMV>::W), 0, stream, x, m, k, ap, zp)
+#define RQ_DOWN_A(RT, ATV)                                                                         \
+    switch (x_mode) {                                                                              \
+        case 0: RQ_DOWN_X(RT, ATV, 0); break;                                                      \
+        case 1: RQ_DOWN_X(RT, ATV, 1); break;                                                      \
+        default: RQ_DOWN_X(RT, ATV, 2); break;                                                     \
+    }
 #define RQ_DOWN(RT)                                                                                \
     if (a_t) {                                                                                     \
-        RQ_DOWN_X(RT, true)                                                                        \
+        RQ_DOWN_A(RT, true)                                                                        \
     } else {                                                                                       \
-        RQ_DOWN_X(RT, false)                                                                       \
+        RQ_DOWN_A(RT, false)                                                                       \
     }
     switch (rank) {
         case 16: RQ_DOWN(1) break;
@@ -509,6 +527,7 @@ hipError_t launch_lora_down(const void* x, int64_t m, int64_t k, const void* a, 
         default: return hipErrorInvalidValue;
     }
 #undef RQ_DOWN
+#undef RQ_DOWN_A
 #undef RQ_DOWN_X
     return hipGetLastError();
 }

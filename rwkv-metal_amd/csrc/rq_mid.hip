@@ -33,6 +33,7 @@
 #include "rq_common.h"
 #include "rq_dequant.h"
 #include "rq_launch.h"
+#include "rq_mid.h"
 
 #ifndef RQ_BITS
 #error "compile rq_mid.hip once per bit width with -DRQ_BITS=<bits>"
@@ -268,7 +269,8 @@ RQ_DEV void store_out4(const MidArgs& a, int64_t m, int64_t n, int64_t ld, f32x4
 }
 
 // The QLoRA low-rank term of one 16x16 tile (outputs n0 + 4 lg .. +3 of row
-// m0 + lr): v += scale * z . L^T, z [M, rank] and L [ncols, rank] bf16.
+// m0 + lr): v += scale * z . L^T, z [M, rank] and L [ncols, rank] bf16 (its
+// transpose [rank, l_ld] when stored).
 RQ_DEV f32x4_t add_lora(const rq::LoraArgs& lo, f32x4_t v, int64_t M, int64_t ncols, int64_t m0,
                         int64_t n0, int lane) {
     const int lg = lane >> 4, lr = lane & 15;
@@ -278,7 +280,17 @@ RQ_DEV f32x4_t add_lora(const rq::LoraArgs& lo, f32x4_t v, int64_t M, int64_t nc
         const int j = j0 + 8 * lg;
         u32x4_t zf = {0u, 0u, 0u, 0u}, lf = zf;
         if (j < lo.rank && m < M) zf = *(const u32x4_t*)((const uint16_t*)lo.z + m * lo.rank + j);
-        if (j < lo.rank && n < ncols) lf = *(const u32x4_t*)((const uint16_t*)lo.l + n * lo.rank + j);
+        if (j < lo.rank && n < ncols) {
+            const uint16_t* l = (const uint16_t*)lo.l;
+            if (lo.stored) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    lf[q] = (uint32_t)l[(j + 2 * q) * lo.l_ld + n] |
+                            ((uint32_t)l[(j + 2 * q + 1) * lo.l_ld + n] << 16);
+            } else {
+                lf = *(const u32x4_t*)(l + n * lo.rank + j);
+            }
+        }
         t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, lf),
                                                     __builtin_bit_cast(bf16x8_t, zf), t, 0, 0, 0);
     }
@@ -722,49 +734,19 @@ namespace rq {
 #define RQ_CAT2(a, b) a##b
 #define RQ_CAT(a, b) RQ_CAT2(a, b)
 
-// Tiles: 16*tm activation rows x 16*tn weight rows, `waves` at most, and the
-// measured time per 128-wide span of a CU that runs one block of it (us; 4-bit
-// codes, bf16 activations, from [2048, 2048] against [2048, 8192]).  A wave
-// dequantizes tn weight tiles and stages tm activation tiles per span, so wide
-// tiles do less per output, and small ones fill the chip.
-struct MidTile {
-    int tm, tn, waves;
-    double span_us;
-};
-static constexpr MidTile kMidTiles[] = {{1, 1, 16, 0.123}, {2, 1, 16, 0.177}, {3, 1, 16, 0.204},
-                                        {2, 2, 16, 0.233}, {4, 2, 8, 0.305},  {3, 4, 8, 0.43},
-                                        {4, 4, 8, 0.479}};
-
-// The tile with the least rounds x spans x time per span, plus the launch and
-// the sum over the waves (3 + 0.2 us per 16x16 tile of the block).
-static int mid_pick(int64_t m, int64_t n_out, int64_t k, double* us) {
-    int best = 0;
-    double bt = 1e30;
-    for (int i = 0; i < (int)(sizeof(kMidTiles) / sizeof(kMidTiles[0])); ++i) {
-        const MidTile& t = kMidTiles[i];
-        const int64_t blocks = ((m + 16 * t.tm - 1) / (16 * t.tm)) * ((n_out + 16 * t.tn - 1) / (16 * t.tn));
-        const double c = 3.0 + 0.2 * t.tm * t.tn +
-                         (double)((blocks + 255) / 256) * (double)((k + 127) / 128) * t.span_us;
-        if (c < bt) {
-            bt = c;
-            best = i;
-        }
-    }
-    if (us) *us = bt;
-    return best;
-}
-
 template <bool SB32, bool XF, int TM, int TN, int MAXW>
-static hipError_t launch_mid_t(MidArgs& a, hipStream_t stream) {
+static hipError_t launch_mid_t(MidArgs& a, const MidTile& plan, hipStream_t stream) {
     a.tiles_m = (int)((a.M + 16 * TM - 1) / (16 * TM));
     a.tiles_n = (int)((a.R + 16 * TN - 1) / (16 * TN));
     const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
     const int nspan = (int)((a.K + 127) / 128);
-    // about MAXW waves a CU, at least 4 a block ([16384, 4096] at M = 128, two
+    // about `waves` waves a CU, at least 4 a block ([16384, 4096] at M = 128, two
     // 4x4 blocks a CU: 38 us with 4 waves, 42 with 8; [8192, 2048] at M = 200
     // 21 against 25)
-    const int q = (int)((tiles + 255) / 256);
-    const int maxw = MAXW / q > 4 ? MAXW / q : 4;
+    const int64_t ptiles = ((a.M + 16 * plan.tm - 1) / (16 * plan.tm)) *
+                           ((a.R + 16 * plan.tn - 1) / (16 * plan.tn));
+    const int q = (int)((ptiles + 255) / 256);
+    const int maxw = plan.waves / q > 4 ? plan.waves / q : 4;
     a.spw = (nspan + maxw - 1) / maxw;
     const int nw = (nspan + a.spw - 1) / a.spw;
     // activations in flight: two halves of a span where the registers allow
@@ -777,14 +759,18 @@ static hipError_t launch_mid_t(MidArgs& a, hipStream_t stream) {
 
 template <bool SB32, bool XF>
 static hipError_t launch_mid_t_tile(MidArgs& a, int tile, hipStream_t stream) {
+    const MidTile& t = kMidTiles[tile];
     switch (tile) {
-        case 0: return launch_mid_t<SB32, XF, 1, 1, 16>(a, stream);
-        case 1: return launch_mid_t<SB32, XF, 2, 1, 16>(a, stream);
-        case 2: return launch_mid_t<SB32, XF, 3, 1, 16>(a, stream);
-        case 3: return launch_mid_t<SB32, XF, 2, 2, 16>(a, stream);
-        case 4: return launch_mid_t<SB32, XF, 4, 2, 8>(a, stream);
-        case 5: return launch_mid_t<SB32, XF, 3, 4, 8>(a, stream);
-        default: return launch_mid_t<SB32, XF, 4, 4, 8>(a, stream);
+        case 0: return launch_mid_t<SB32, XF, 1, 1, 16>(a, t, stream);
+        case 1: return launch_mid_t<SB32, XF, 2, 1, 16>(a, t, stream);
+        case 2: return launch_mid_t<SB32, XF, 3, 1, 16>(a, t, stream);
+        case 3: return launch_mid_t<SB32, XF, 2, 2, 16>(a, t, stream);
+        case 4: return launch_mid_t<SB32, XF, 4, 2, 8>(a, t, stream);
+        // 128 rows of fp32 activations in flight would spill: the same slices of
+        // the contraction (so the same sums as bf16(x)) on two 64-row tiles
+        case 5: return launch_mid_t<SB32, XF, XF ? 4 : 8, 2, 8>(a, t, stream);
+        case 6: return launch_mid_t<SB32, XF, 3, 4, 8>(a, t, stream);
+        default: return launch_mid_t<SB32, XF, 4, 4, 8>(a, t, stream);
     }
 }
 
@@ -815,7 +801,7 @@ hipError_t RQ_CAT(launch_qmm_t_mid_b, RQ_BITS)(const void* x, int x_dt, const ui
                                           int64_t m, int64_t rows, int64_t cols, int gs, void* y,
                                           int y_dt, hipStream_t stream, const LoraArgs* lora) {
     MidArgs a = mid_args(x, x_dt, wq, scales, biases, sb_dt, m, rows, cols, gs, y, y_dt, rows, lora);
-    const int tile = mid_pick(m, rows, cols, nullptr);
+    const int tile = mid_pick(m, rows, cols, RQ_BITS);
     if (sb_dt == RQ_F32)
         return x_dt == RQ_F32 ? launch_mid_t_tile<true, true>(a, tile, stream)
                               : launch_mid_t_tile<true, false>(a, tile, stream);

@@ -24,6 +24,7 @@
 #include "rq_common.h"
 #include "rq_dequant.h"
 #include "rq_launch.h"
+#include "rq_mid.h"
 
 #ifndef RQ_BITS
 #error "compile rq_qmm.hip once per bit width with -DRQ_BITS=<bits>"
@@ -1783,13 +1784,6 @@ hipError_t RQ_CAT(launch_qmm_t_b, RQ_BITS)(const void* x, int x_dt, const uint32
                                       const void* scales, const void* biases, int sb_dt,
                                       int64_t m, int64_t rows, int64_t cols, int gs, void* y,
                                       int y_dt, hipStream_t stream, const LoraArgs* lora) {
-    // Fewer than 256 rows: small tiles, the contraction split over the waves of
-    // a block.  (128 x 128 tiles of the same dequantization, one block walking
-    // all of K, took 58 us on [2048, 2048] and 220 on [2048, 8192] at M = 77,
-    // on 16 CUs; these take 7 and 17.)  Offsets inside a tile are 32-bit.
-    if (m < 256 && cols <= kMidMaxCols && !lora)
-        return RQ_CAT(launch_qmm_t_mid_b, RQ_BITS)(x, x_dt, wq, scales, biases, sb_dt, m, rows, cols,
-                                              gs, y, y_dt, stream, lora);
     const int gs_shift = __builtin_ctz(gs);
     const LoraArgs lo = lora ? *lora : LoraArgs{nullptr, nullptr, 0, 0.f};
     // bf16 or fp32 activations (fp32 rounded to bf16 as the producers stage them)
@@ -1797,6 +1791,30 @@ hipError_t RQ_CAT(launch_qmm_t_b, RQ_BITS)(const void* x, int x_dt, const uint32
                      sb_dt != RQ_F32 && cols % 64 == 0 && (cols / gs) % 8 == 0 &&
                      (((uintptr_t)x | (uintptr_t)scales | (uintptr_t)biases) & 15) == 0;
     const bool xf = x_dt == RQ_F32;
+    // Small tiles with the contraction split over the waves of a block: fewer
+    // than 256 rows (128 x 128 tiles of the same dequantization, one block
+    // walking all of K, took 58 us on [2048, 2048] and 220 on [2048, 8192] at
+    // M = 77, on 16 CUs; these take 7 and 17), and above where their estimate
+    // is the lower one.  Measured at 4 bits: [768, 768] (12 groups, no
+    // 64-wide stages) at M = 300 / 2048 26.2 / 27.3 -> 5.1 / 11.5 us, [1024,
+    // 1024] at M = 512 10.6 -> 6.8, [2048, 2048] at M = 512 16.2 -> 12.9, but
+    // [8192, 2048] 24 against 39.  The choice does not depend on x's type where
+    // the 64-wide stages apply: fp32 x gives the bits of bf16(x).  Offsets
+    // inside a tile are 32-bit.
+    if (cols <= kMidMaxCols && (!lora || (lora->mid && !lora->a))) {
+        bool mid = m < 256;
+        if (!mid) {
+            double us;
+            mid_pick(m, rows, cols, RQ_BITS, &us);
+            if (k64) mid = us < k64_us(m, rows, cols, RQ_BITS);
+            // fp32 tiles are re-read from L2 by every weight tile: [2048, 2048]
+            // at M = 2048 72 us against 40 with bf16 x
+            else mid = lora || (xf ? 1.5 * us : us) < wide_us(m, rows, cols, x_dt != RQ_BF16);
+        }
+        if (mid)
+            return RQ_CAT(launch_qmm_t_mid_b, RQ_BITS)(x, x_dt, wq, scales, biases, sb_dt, m, rows,
+                                                  cols, gs, y, y_dt, stream, lora);
+    }
     if (lora && lora->a) {
         // the fused QLoRA layer with its down-projection in the kernel: rank 16,
         // 4- or 8-bit codes, 128-column tiles (the 160-column ones have no
@@ -2036,7 +2054,7 @@ hipError_t RQ_CAT(launch_qmm_n_b, RQ_BITS)(const void* x, int x_dt, const uint32
         return hipGetLastError();
     }
 #undef RQ_NK64
-    if (lora) return hipErrorNotSupported;  // the low-rank term rides on the k64 kernels only
+    if (lora && !lora->mid) return hipErrorNotSupported;
     // Everything else: small tiles over wave slices of the contraction.  (128 x
     // 128 tiles, one block walking all weight rows, took 44 us on [768, 768] at
     // M = 200, on 12 CUs, and 3.6 us per 64 rows and round at any size; these
@@ -2044,7 +2062,8 @@ hipError_t RQ_CAT(launch_qmm_n_b, RQ_BITS)(const void* x, int x_dt, const uint32
     // are 32-bit.
     if (rows <= kMidMaxCols && cols <= kMidMaxCols)
         return RQ_CAT(launch_qmm_n_mid_b, RQ_BITS)(x, x_dt, wq, scales, biases, sb_dt, m, rows, cols,
-                                              gs, y, y_dt, stream, nullptr);
+                                              gs, y, y_dt, stream, lora);
+    if (lora) return hipErrorNotSupported;
     constexpr int BM = 128;
     const dim3 grid((unsigned)((cols + BN - 1) / BN), (unsigned)((m + BM - 1) / BM));
     const int gs_shift = __builtin_ctz(gs);

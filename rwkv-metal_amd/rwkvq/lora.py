@@ -50,11 +50,12 @@ class _QLoRAFunction(torch.autograd.Function):
     inside the transpose=True GEMM and adds z B^T in its output stage; dX is
     one launch (rq_qlora_dx) that computes u = dY B inside the
     transpose=False GEMM and adds scale * u A, reading A and B as stored; dA =
-    scale * u^T x and dB = scale * dY^T z are one rq_lora_grads launch.  Other ranks run z and u as rq_lora_down launches
-    and the term with rq_qmm_lora.  The frozen base gets no gradient.
+    scale * u^T x and dB = scale * dY^T z are one rq_lora_grads launch.  Other ranks and bit widths and
+    fewer than 256 rows run the same calls as two launches, z (or u) and the
+    GEMM with the term.  The frozen base gets no gradient.
 
-    fp32 x (the reference's default activations) is rounded to bf16 once, by
-    one cast, and so is fp32 dY: every kernel rounds its fp32 operands to bf16
+    fp32 x (the reference's default activations) is rounded to bf16 once for the
+    one-launch products, by one cast, and so is fp32 dY: every kernel rounds its fp32 operands to bf16
     as it stages them anyway (the results are the bits the fp32 inputs give),
     but the GEMMs re-read their activation tiles once per column tile, so
     twice the bytes per re-read cost more than the cast.  y and dX stay fp32,
@@ -65,10 +66,13 @@ class _QLoRAFunction(torch.autograd.Function):
         gs, bits = base.group_size, base.bits
         xdt = x2.dtype
         xb = x2.to(torch.bfloat16) if xdt == torch.float32 else x2
-        yz = ops.qlora_fused(xb, base.weight, base.scales, base.biases, lora_a, lora_b, scale,
-                             True, gs, bits, out_dtype=ops._promote(xdt, base.scales.dtype))
+        # one launch, z = x A^T inside the GEMM from bf16(x), or two, z from x
+        one = ops._one_launch(x2.shape[0], base.weight, lora_a.shape[0], bits, gs,
+                              base.scales.dtype, True)
+        yz = ops.qlora_product(xb if one else x2, base.weight, base.scales, base.biases, lora_a,
+                               lora_b, scale, True, gs, bits, ops._promote(xdt, base.scales.dtype))
         if yz is not None:
-            y, z = yz      # one launch: z = x A^T inside the GEMM
+            y, z = yz
         else:
             z = ops.lora_down(x2, lora_a)
             y = ops.quantized_matmul_lora(x2, base.weight, base.scales, base.biases, z, lora_b,
@@ -87,9 +91,12 @@ class _QLoRAFunction(torch.autograd.Function):
         dx = da = db = None
         dxu = None
         if ctx.needs_input_grad[0]:
-            # one launch from the adapters as stored: u = dY B inside the GEMM
-            dxu = ops.qlora_dx_fused(dyb, base.weight, base.scales, base.biases, lora_a, lora_b,
-                                     scale, gs, bits, out_dtype=ops._promote(xdt, base.scales.dtype))
+            # from the adapters as stored: u = dY B inside the GEMM, or as a launch of its own
+            one = ops._one_launch(dy.shape[0], base.weight, lora_a.shape[0], bits, gs,
+                                  base.scales.dtype, False)
+            dxu = ops.qlora_dx_product(dyb if one else dy, base.weight, base.scales, base.biases,
+                                       lora_a, lora_b, scale, gs, bits,
+                                       ops._promote(xdt, base.scales.dtype))
             if dxu is not None:
                 dx, u = dxu
             else:

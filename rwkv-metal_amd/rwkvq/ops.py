@@ -535,6 +535,33 @@ def qlora_fused(x: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor, a: Tenso
     fp32), else in MLX's promotion of x and the scales.  None where the fused
     kernels do not apply (see rq_qlora); no autograd (rwkvq.lora
     differentiates the layer)."""
+    if not (_lora_operands(x, a, lora) and
+            _one_launch(x.shape[0], w_q, a.shape[0], bits, group_size, scales.dtype, transpose)):
+        _qlora_check(x, w_q, scales, biases, a, lora, transpose, group_size, bits)
+        return None
+    return qlora_product(x, w_q, scales, biases, a, lora, scale, transpose, group_size, bits, out_dtype)
+
+
+def _lora_operands(x: Tensor, a: Tensor, b: Tensor) -> bool:
+    return x.dtype in (torch.bfloat16, torch.float32) and a.dtype == b.dtype == torch.bfloat16
+
+
+def _one_launch(m: int, w_q: Tensor, rank: int, bits: int, group_size: int, sdt: torch.dtype,
+                transpose: bool) -> bool:
+    """What the in-kernel down-projection covers (rq_qlora, rq_qlora_dx): rank 16
+    with 4- or 8-bit codes on the 64-wide-stage GEMMs.  The GEMM and z then
+    both read bf16(x), so fp32 x may be cast first; elsewhere z is made from
+    the fp32 x."""
+    if rank != 16 or m == 0:
+        return rank == 16
+    if m < 256 or bits not in (4, 8) or sdt == torch.float32:
+        return False
+    R, K = w_q.shape[0], w_q.shape[1] * 32 // bits
+    return (K % 64 == 0 and (K // group_size) % 8 == 0) if transpose else (R % 64 == 0 and K % 128 == 0)
+
+
+def _qlora_check(x, w_q, scales, biases, a, lora, transpose, group_size, bits):
+    """The packed words as int32, the weight's rows and columns."""
     _check_args(group_size, bits)
     w_q = _words(w_q)
     K = _check_packed(w_q, scales, biases, group_size, bits)
@@ -543,9 +570,17 @@ def qlora_fused(x: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor, a: Tenso
     if (x.dim() != 2 or x.shape[1] != n_in or tuple(a.shape) != (rank, n_in)
             or tuple(lora.shape) != (n_out, rank)):
         raise ValueError("qlora_fused: x, a and lora shapes do not agree")
-    if not (x.dtype in (torch.bfloat16, torch.float32) and a.dtype == lora.dtype == torch.bfloat16
-            and rank == 16):
-        return None
+    return w_q, K, n_out, rank
+
+
+def qlora_product(x: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor, a: Tensor,
+                  lora: Tensor, scale: float, transpose: bool = True, group_size: int = 64,
+                  bits: int = 4, out_dtype: torch.dtype | None = None):
+    """qlora_fused wherever rq_qlora runs it, in one launch or two (z, then the
+    GEMM with the term: any rank of 16 to 64, any bit width, any number of
+    rows; z is that of the fp32 x where x is fp32).  None elsewhere.  bf16
+    adapters, bf16 or fp32 x."""
+    w_q, K, n_out, rank = _qlora_check(x, w_q, scales, biases, a, lora, transpose, group_size, bits)
     _on_gpu(x, w_q, scales, biases, a, lora)
     x, w_q, scales, a, lora = _ready(x), _ready(w_q), _ready(scales), _ready(a), _ready(lora)
     biases = _ready(biases.to(scales.dtype))
@@ -575,6 +610,14 @@ def qlora_dx_fused(dy: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor, lora
     equal bit for bit to qlora_fused(dy, ..., lora_b^T, lora_a^T, scale,
     False), without the transposed copies.  dy is 2-D.  None where the fused
     kernels do not apply; no autograd."""
+    if not (_lora_operands(dy, lora_a, lora_b) and
+            _one_launch(dy.shape[0], w_q, lora_a.shape[0], bits, group_size, scales.dtype, False)):
+        _qlora_dx_check(dy, w_q, scales, biases, lora_a, lora_b, group_size, bits)
+        return None
+    return qlora_dx_product(dy, w_q, scales, biases, lora_a, lora_b, scale, group_size, bits, out_dtype)
+
+
+def _qlora_dx_check(dy, w_q, scales, biases, lora_a, lora_b, group_size, bits):
     _check_args(group_size, bits)
     w_q = _words(w_q)
     K = _check_packed(w_q, scales, biases, group_size, bits)
@@ -583,9 +626,15 @@ def qlora_dx_fused(dy: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor, lora
     if (dy.dim() != 2 or dy.shape[1] != R or tuple(lora_a.shape) != (rank, K)
             or tuple(lora_b.shape) != (R, rank)):
         raise ValueError("qlora_dx_fused: dy, lora_a and lora_b shapes do not agree")
-    if not (dy.dtype in (torch.bfloat16, torch.float32)
-            and lora_a.dtype == lora_b.dtype == torch.bfloat16 and rank == 16):
-        return None
+    return w_q, R, K, rank
+
+
+def qlora_dx_product(dy: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor, lora_a: Tensor,
+                     lora_b: Tensor, scale: float, group_size: int = 64, bits: int = 4,
+                     out_dtype: torch.dtype | None = None):
+    """qlora_dx_fused wherever rq_qlora_dx runs it, in one launch or two (as
+    qlora_product); None elsewhere."""
+    w_q, R, K, rank = _qlora_dx_check(dy, w_q, scales, biases, lora_a, lora_b, group_size, bits)
     _on_gpu(dy, w_q, scales, biases, lora_a, lora_b)
     dy, w_q, scales = _ready(dy), _ready(w_q), _ready(scales)
     lora_a, lora_b = lora_a.contiguous(), _ready(lora_b)

@@ -154,3 +154,51 @@ def test_mid_transposed_infinite_rows_stay_in_their_row(rq, dev):
     ref = x.to(dev).double() @ w
     assert torch.equal(torch.isinf(y), torch.isinf(ref))
     assert torch.isfinite(y[[i for i in range(m) if i != 3]]).all()
+
+
+@pytest.mark.parametrize("rank", [16, 32, 48, 64])
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m,R,K,bits,gs,sdt", [(17, 96, 160, 4, 32, torch.bfloat16),
+                                               (200, 3072, 768, 4, 64, torch.bfloat16),
+                                               (255, 256, 2048, 8, 128, torch.bfloat16),
+                                               (100, 352, 416, 5, 32, torch.float32),
+                                               (300, 320, 1024, 3, 64, torch.bfloat16),
+                                               (300, 96, 768, 4, 64, torch.bfloat16)])
+def test_qlora_two_launches(rq, dev, m, R, K, bits, gs, sdt, xdt, rank):
+    """rq_qlora / rq_qlora_dx outside the in-kernel down-projection: z (u) is that
+    of x (dY) itself, rounded once to bf16; the product gets the term of that
+    z before its one rounding."""
+    from rwkvq import ops
+    if rank == 16 and m >= 256 and bits in (4, 8) and (K // gs) % 8 == 0:
+        return
+    (wq, s, b), w = packed(rq, dev, R, K, gs, bits, sdt, m + R)
+    g = torch.Generator().manual_seed(rank)
+    A = (torch.randn(rank, K, generator=g) * K ** -0.5).bfloat16().to(dev)
+    B = (torch.randn(R, rank, generator=g) * 0.05).bfloat16().to(dev)
+    x = torch.randn(m, K, generator=g).to(xdt).to(dev)
+    dy = torch.randn(m, R, generator=g).to(xdt).to(dev)
+    odt = out_dtype(xdt, sdt)
+    print("qlora two launches", m, R, K, bits, rank, xdt, flush=True)
+    y, z = ops.qlora_product(x, wq, s, b, A, B, 2.0, True, gs, bits, odt)
+    assert y.dtype == odt
+    check(z, (x.double() @ A.double().t(), torch.bfloat16), K, "z")
+    check(y, (x.bfloat16().double() @ w.t() + 2.0 * z.double() @ B.double().t(), odt), K, "y")
+    dx, u = ops.qlora_dx_product(dy, wq, s, b, A, B, 2.0, gs, bits, odt)
+    check(u, (dy.double() @ B.double(), torch.bfloat16), R, "u")
+    check(dx, (dy.bfloat16().double() @ w + 2.0 * u.double() @ A.double(), odt), R, "dx")
+
+
+def test_fp32_down_projection_is_not_less_exact(rq, dev):
+    """z of fp32 x as two bf16 values per element: no further from float64 than
+    the fp32 product, both rounded once to bf16."""
+    from rwkvq import ops
+    (wq, s, b), _ = packed(rq, dev, 64, 4096, 64, 4, torch.bfloat16, 1)
+    g = torch.Generator().manual_seed(0)
+    x = torch.randn(128, 4096, generator=g).to(dev)
+    A = (torch.randn(32, 4096, generator=g) / 64).bfloat16().to(dev)
+    B = torch.zeros(64, 32, dtype=torch.bfloat16, device=dev)
+    _, z = ops.qlora_product(x, wq, s, b, A, B, 1.0, True, 64, 4, torch.float32)
+    ref = x.double() @ A.double().t()
+    old = (x @ A.float().t()).bfloat16()
+    err = lambda t: ((t.double() - ref).norm() / ref.norm()).item()  # noqa: E731
+    assert err(z) <= 1.01 * err(old), (err(z), err(old))
