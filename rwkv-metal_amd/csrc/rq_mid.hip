@@ -150,11 +150,8 @@ struct SpanRegs {
             }
         }
     }
-    // The weights as the fragments of four MFMAs: frag[2 h + j] holds, in lane
-    // (lg, lr), k = 64 h + 16 lg + 8 j .. +7 of row lr.
-    RQ_DEV void fragments(int gsh, int lg, bool f16, u32x4_t* frag) {
-        // the scales to every lane group, then the biases
-        uint32_t sv[NW], bv[NW];
+    // The scales to every lane group, and the biases.
+    RQ_DEV void spread_sb(uint32_t* sv, uint32_t* bv) const {
 #pragma unroll
         for (int i = 0; i < NW; ++i) {
             const auto r0 = __builtin_amdgcn_permlane32_swap(sb[i], sb[i], false, false);
@@ -162,6 +159,18 @@ struct SpanRegs {
             sv[i] = r1[0];
             bv[i] = r1[1];
         }
+    }
+    // Value of the span's group g.
+    RQ_DEV static float group_value(const uint32_t* v, int g, bool f16) {
+        if constexpr (SB32) return __uint_as_float(v[g]);
+        const uint32_t h = (v[g >> 1] >> (16 * (g & 1))) & 0xffffu;
+        return f16 ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
+    }
+    // The weights as the fragments of four MFMAs: frag[2 h + j] holds, in lane
+    // (lg, lr), k = 64 h + 16 lg + 8 j .. +7 of row lr.
+    RQ_DEV void fragments(int gsh, int lg, bool f16, u32x4_t* frag) {
+        uint32_t sv[NW], bv[NW];
+        spread_sb(sv, bv);
         if constexpr (BITS % 2 == 0) {
             // 16 codes are BITS / 2 whole words: spread the packed words, then
             // dequantize; group of the lane's codes of half h: (2 h + lg / 2) >> gsh
@@ -231,6 +240,23 @@ struct XPiece {
                           (2 * e + 1 < n ? (uint32_t)((ghalf_t)p)[2 * e + 1] << 16 : 0u);
             }
         }
+    }
+    // what bf16() leaves of fp32 or f16 values, rounded to bf16
+    RQ_DEV u32x4_t rest(u32x4_t hi) const {
+        u32x4_t r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float f0, f1;
+            if constexpr (XF) {
+                f0 = __uint_as_float(v[e >> 1][2 * (e & 1)]);
+                f1 = __uint_as_float(v[e >> 1][2 * (e & 1) + 1]);
+            } else {
+                f0 = f16_bits_to_f32(v[0][e] & 0xffffu);
+                f1 = f16_bits_to_f32(v[0][e] >> 16);
+            }
+            r[e] = pack_bf16x2(f0 - __uint_as_float(hi[e] << 16), f1 - __uint_as_float(hi[e] & 0xffff0000u));
+        }
+        return r;
     }
     RQ_DEV u32x4_t bf16(bool f16) const {
         if constexpr (XF) {
@@ -449,6 +475,203 @@ __global__ __launch_bounds__(64 * MAXW) void qmm_t_mid(const MidArgs a) {
                 store_out4(a, m + lr, n + 4 * lg, a.R, v);
             }
     }
+}
+
+// --------------------------------------------------------------- qmv_mid
+//
+// The decode GEMV of up to 16 activation rows for launches of few weight rows
+// (one projection, or the independent ones of a layer): one block per 16
+// weight rows, its waves over slices of the contraction as in qmm_t_mid.  The
+// weights are not rounded: the codes enter the MFMA as integers (exact in
+// bf16) and each group's scale and bias are applied to its sums in fp32, acc +=
+// s D + b X, X the group's activation sums from a second MFMA against ones.
+// The activations are the A operand, so an accumulator column is one weight
+// row and a lane needs one (scale, bias) per group.  An MFMA contracts 32
+// consecutive k, inside one group at every group size.  xsplit: rows m/2 .. m-1
+// hold what bf16 leaves of the fp32 or f16 activations of rows 0 .. m/2-1 (m at
+// most 4), and the two are added before the store.
+struct QmvMidArgs {
+    rq_problem p[RQ_MAX_GROUPED];
+    int block_start[RQ_MAX_GROUPED + 1];
+    int n, m, sb_f16, x_f16, y_dt, spw;
+    int xsplit;
+};
+
+// 4 x 4 transpose of (lane group, register): afterwards register j of lane
+// group g holds what register g of lane group j held.
+RQ_DEV void transpose_lane_groups(uint32_t& a, uint32_t& b, uint32_t& c, uint32_t& d) {
+    const auto r0 = __builtin_amdgcn_permlane32_swap(a, c, false, false);
+    const auto r1 = __builtin_amdgcn_permlane32_swap(b, d, false, false);
+    const auto r2 = __builtin_amdgcn_permlane16_swap(r0[0], r1[0], false, false);
+    const auto r3 = __builtin_amdgcn_permlane16_swap(r0[1], r1[1], false, false);
+    a = r2[0]; b = r2[1]; c = r3[0]; d = r3[1];
+}
+
+// A lane's run of codes -> the four fragments of the span as bf16 integers:
+// frag[j] holds, in lane (lg, lr), k = 32 j + 8 lg .. +7 of row lr.
+template <int BITS>
+RQ_DEV void code_fragments(const uint32_t* words, u32x4_t* frag) {
+    if constexpr (BITS == 4 || BITS == 8) {
+        // eight codes are whole words: spread the packed words
+        constexpr int HW = BITS / 4;
+        uint32_t w[4 * HW];
+#pragma unroll
+        for (int i = 0; i < 4 * HW; ++i) w[i] = words[i];
+#pragma unroll
+        for (int i = 0; i < HW; ++i) transpose_lane_groups(w[i], w[HW + i], w[2 * HW + i], w[3 * HW + i]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if constexpr (BITS == 4) {
+                typedef float f32x2_t __attribute__((ext_vector_type(2)));
+                const uint32_t lo = w[j] & 0x0F0F0F0Fu, hi = (w[j] >> 4) & 0x0F0F0F0Fu;
+                const f32x2_t l0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 512.f, false);
+                const f32x2_t l1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 512.f, true);
+                const f32x2_t h0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 512.f, false);
+                const f32x2_t h1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 512.f, true);
+                frag[j] = u32x4_t{pack_bf16x2(l0[0], h0[0]), pack_bf16x2(l0[1], h0[1]),
+                                  pack_bf16x2(l1[0], h1[0]), pack_bf16x2(l1[1], h1[1])};
+            } else {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    uint32_t v = w[2 * j + h];
+                    asm("" : "+v"(v));
+                    frag[j][2 * h] = pack_bf16x2((float)(uint8_t)v, (float)(uint8_t)(v >> 8));
+                    frag[j][2 * h + 1] = pack_bf16x2((float)(uint8_t)(v >> 16), (float)(uint8_t)(v >> 24));
+                }
+            }
+        }
+    } else {
+        uint32_t d[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            d[i] = pack_bf16x2((float)run_code<BITS>(words, 2 * i), (float)run_code<BITS>(words, 2 * i + 1));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) transpose_lane_groups(d[e], d[4 + e], d[8 + e], d[12 + e]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) frag[j] = u32x4_t{d[4 * j], d[4 * j + 1], d[4 * j + 2], d[4 * j + 3]};
+    }
+}
+
+template <int BITS, bool SB32, bool XF, int GSH>
+__global__ __launch_bounds__(1024) void qmv_mid(const QmvMidArgs a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // 2 KB per wave
+    constexpr int ES = XF ? 4 : 2, SBS = SB32 ? 4 : 2;
+    constexpr int gsh = GSH - 5, KG = 1 << gsh;  // 32-wide k-steps per group
+    const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lg = lane >> 4, lr = lane & 15;
+    int lo = 0, hi = a.n - 1;  // last problem whose first block is not past this one
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (a.block_start[mid] <= (int)blockIdx.x) lo = mid; else hi = mid - 1;
+    }
+    const rq_problem& P = a.p[lo];
+    const int64_t R = P.rows, K = P.cols;
+    const int64_t n0 = (int64_t)((int)blockIdx.x - a.block_start[lo]) * 16;
+    const int runs = (int)(K >> 5), nspan = (runs + 3) >> 2;
+    const int sp0 = wave * a.spw, sp1 = sp0 + a.spw < nspan ? sp0 + a.spw : nspan;
+    const int64_t wpr = (int64_t)runs * BITS, G = K >> GSH;
+
+    const uint8_t* wbase = (const uint8_t*)(P.w_q + n0 * wpr);
+    const int nr = R - n0 < 16 && lr >= (int)(R - n0) ? (int)(R - n0) - 1 : lr;
+    const uint32_t woff = (uint32_t)nr * (uint32_t)wpr * 4;
+    const gbyte_t sbp = (gbyte_t)((lg & 1) ? P.biases : P.scales) + ((n0 + nr) * G + ((4 * sp0) >> gsh)) * SBS;
+    SpanRegs<BITS, SB32> cur, nxt;
+    auto load_span = [&](SpanRegs<BITS, SB32>& r, int sp) {
+        // a run past the row's end reads the last one; its k-step is not run
+        const int run = 4 * sp + lg < runs ? 4 * sp + lg : runs - 1;
+        r.load_codes(wbase, woff + run * BITS * 4);
+        if (lg < 2) {
+            const int left = (runs - 4 * sp + KG - 1) >> gsh, ng = 4 >> gsh;
+            r.load_sb(sbp + (int64_t)((4 * (sp - sp0)) >> gsh) * SBS, gsh, left < ng ? left : ng);
+        }
+    };
+    // activations as in qmm_t_mid, one 16-row tile: rows past m repeat the last
+    const int xr = lane >> 3, xc = lane & 7;
+    const int xm = a.xsplit ? a.m >> 1 : a.m;
+    const bool xlo = a.xsplit && xr >= xm && xr < a.m;
+    uint32_t xoff[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int r = 8 * q + xr - (xlo && q == 0 ? xm : 0);
+        xoff[q] = (uint32_t)(r < xm ? r : xm - 1) * (uint32_t)K * ES;
+    }
+    XPiece<XF> xv[2][2];
+    auto load_x = [&](XPiece<XF>(&v)[2], int half) {
+        // a k past the row's end reads the half's first 32 (its k-step is not run)
+        const int c = 64 * half + 8 * xc < K ? xc : xc & 3;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) v[q].load((const uint8_t*)P.x, xoff[q] + (uint32_t)(64 * half + 8 * c) * ES);
+    };
+    uint8_t* xs = lds + wave * 2048;
+    uint8_t* xw = xs + xr * 128 + ((xc ^ xr) << 4);
+    const uint32_t xrd = wave * 2048 + lr * 128 + ((lg ^ (lr & 7)) << 4);
+
+    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, u32x4_t{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
+    f32x4_t acc = zero;
+    const int h1 = 2 * sp1 < (runs + 1) >> 1 ? 2 * sp1 : (runs + 1) >> 1;
+    load_span(cur, sp0);
+    load_x(xv[0], 2 * sp0);
+    if (2 * sp0 + 1 < h1) load_x(xv[1], 2 * sp0 + 1);
+    for (int sp = sp0; sp < sp1; ++sp) {
+        if (sp + 1 < sp1) load_span(nxt, sp + 1);
+        uint32_t sv[SpanRegs<BITS, SB32>::NW], bv[SpanRegs<BITS, SB32>::NW];
+        cur.spread_sb(sv, bv);
+        u32x4_t wf[4];
+        code_fragments<BITS>(cur.w, wf);
+        f32x4_t D = zero, X = zero;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int half = 2 * sp + h;
+            if (half < h1) {
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    u32x4_t v = xv[h][q].bf16(a.x_f16);
+                    if (xlo && q == 0) v = xv[h][q].rest(v);
+                    *(u32x4_t*)(xw + q * 1024) = v;
+                }
+                if (half + 2 < h1) load_x(xv[h], half + 2);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const int j = 2 * h + i;
+                    if (2 * half + i < runs) {
+                        const bf16x8_t xf =
+                            __builtin_bit_cast(bf16x8_t, *(const u32x4_t*)(lds + (xrd ^ (64 * i))));
+                        const bool first = j % KG == 0;
+                        D = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, __builtin_bit_cast(bf16x8_t, wf[j]),
+                                                                    first ? zero : D, 0, 0, 0);
+                        X = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, ones, first ? zero : X, 0, 0, 0);
+                        if (j % KG == KG - 1) {  // the group's last k-step (groups are whole)
+                            const float s = SpanRegs<BITS, SB32>::group_value(sv, j >> gsh, a.sb_f16);
+                            const float b = SpanRegs<BITS, SB32>::group_value(bv, j >> gsh, a.sb_f16);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) acc[e] = fmaf(s, D[e], fmaf(b, X[e], acc[e]));
+                        }
+                    }
+                }
+            }
+        }
+        cur = nxt;
+    }
+    if (nw > 1) {
+        *(f32x4_t*)(xs + lane * 16) = acc;
+        __syncthreads();
+        if (wave) return;
+        for (int w = 1; w < nw; ++w) {
+            const f32x4_t u = *(const f32x4_t*)(lds + w * 2048 + lane * 16);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] += u[e];
+        }
+    }
+    // lane (lg, lr): activation rows 4 lg + e, weight row lr
+    if (a.xsplit) {
+        acc[0] += xm == 1 ? acc[1] : acc[2];
+        acc[1] += acc[3];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (4 * lg + e < xm && n0 + lr < R) store_dt(P.y, a.y_dt, (4 * lg + e) * R + n0 + lr, acc[e]);
 }
 
 // ------------------------------------------------------------- qmm_n_mid
@@ -868,6 +1091,48 @@ hipError_t RQ_CAT(launch_qmm_n_mid_b, RQ_BITS)(const void* x, int x_dt, const ui
                               : launch_mid_n_tile<true, false>(a, tile, stream);
     return x_dt == RQ_F32 ? launch_mid_n_tile<false, true>(a, tile, stream)
                           : launch_mid_n_tile<false, false>(a, tile, stream);
+}
+
+// One launch of qmv_mid over n problems that share cols (n <= RQ_MAX_GROUPED); m
+// counts MFMA activation rows (twice the problems' with xsplit).
+hipError_t RQ_CAT(launch_qmv_mid_b, RQ_BITS)(const rq_problem* const* problems, int n, int x_dt,
+                                        int sb_dt, int y_dt, int64_t m, int gs, bool xsplit,
+                                        hipStream_t stream) {
+    QmvMidArgs a{};
+    int64_t blocks = 0;
+    for (int i = 0; i < n; ++i) {
+        a.p[i] = *problems[i];
+        a.block_start[i] = (int)blocks;
+        blocks += (problems[i]->rows + 15) / 16;
+    }
+    a.block_start[n] = (int)blocks;
+    if (blocks == 0) return hipSuccess;
+    a.n = n;
+    a.m = (int)m;
+    a.sb_f16 = sb_dt == RQ_F16;
+    a.x_f16 = x_dt == RQ_F16;
+    a.y_dt = y_dt;
+    a.xsplit = xsplit;
+    const int nspan = (int)((problems[0]->cols + 127) / 128);
+    const int q = (int)((blocks + 255) / 256), maxw = 16 / q > 4 ? 16 / q : 4;
+    a.spw = (nspan + maxw - 1) / maxw;
+    const int nw = (nspan + a.spw - 1) / a.spw;
+#define RQ_QMV_MID_G(SB, XFV, GSHV)                                                              \
+    hipLaunchKernelGGL((qmv_mid<RQ_BITS, SB, XFV, GSHV>), dim3((unsigned)blocks), dim3(64 * nw),  \
+                       nw * 2048, stream, a)
+#define RQ_QMV_MID_X(SB, XFV)                          \
+    switch (gs) {                                      \
+        case 32: RQ_QMV_MID_G(SB, XFV, 5); break;      \
+        case 64: RQ_QMV_MID_G(SB, XFV, 6); break;      \
+        default: RQ_QMV_MID_G(SB, XFV, 7); break;      \
+    }
+#define RQ_QMV_MID(SB) \
+    if (x_dt == RQ_F32) { RQ_QMV_MID_X(SB, true) } else { RQ_QMV_MID_X(SB, false) }
+    if (sb_dt == RQ_F32) { RQ_QMV_MID(true) } else { RQ_QMV_MID(false) }
+#undef RQ_QMV_MID
+#undef RQ_QMV_MID_X
+#undef RQ_QMV_MID_G
+    return hipGetLastError();
 }
 
 }  // namespace rq

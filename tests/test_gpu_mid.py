@@ -202,3 +202,50 @@ def test_fp32_down_projection_is_not_less_exact(rq, dev):
     old = (x @ A.float().t()).bfloat16()
     err = lambda t: ((t.double() - ref).norm() / ref.norm()).item()  # noqa: E731
     assert err(z) <= 1.01 * err(old), (err(z), err(old))
+
+
+@pytest.mark.parametrize("sdt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m", [3, 7, 9, 16])
+@pytest.mark.parametrize("groups", [1, 3, 5, 17])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("bits", [2, 3, 4, 5, 6, 8])
+def test_qmv_mid_groups(rq, dev, bits, gs, groups, m, sdt):
+    """The decode GEMV of any layout: weights unrounded, x rounded to bf16 once
+    (sums of K products: 2^-24 each)."""
+    R, K = 37, groups * gs
+    (wq, s, b), _ = packed(rq, dev, R, K, gs, bits, sdt, bits + groups)
+    w = rq.unpack_codes(wq, bits).double().reshape(R, -1, gs)
+    w = (w * s.double()[..., None] + b.double()[..., None]).reshape(R, K)
+    x = torch.randn(m, K, generator=torch.Generator().manual_seed(gs)).to(dev)
+    print("qmv mid", bits, gs, groups, m, sdt, flush=True)
+    y = rq.quantized_matmul(x, wq, s, b, True, gs, bits).double()
+    ref = x.bfloat16().double() @ w.t()
+    assert (y - ref).norm() <= 1e-5 * ref.norm() and (y - ref).abs().max() <= 3e-5 * ref.abs().max()
+
+
+@pytest.mark.parametrize("xdt", [torch.float32, torch.float16])
+@pytest.mark.parametrize("m", [1, 2])
+@pytest.mark.parametrize("R,K,gs,bits", [(50, 160, 32, 6), (2048, 2048, 32, 5), (33, 768 + 64, 64, 4),
+                                         (7, 10240, 32, 8)])
+def test_qmv_mid_split_activations(rq, dev, R, K, gs, bits, m, xdt):
+    """fp32 and f16 x at m <= 2 as two bf16 rows (16 significant bits), fp32
+    scales: within 2^-17 of the product of x itself, and its fp32 sums."""
+    (wq, s, b), _ = packed(rq, dev, R, K, gs, bits, torch.float32, R)
+    w = rq.unpack_codes(wq, bits).double().reshape(R, -1, gs)
+    w = (w * s.double()[..., None] + b.double()[..., None]).reshape(R, K)
+    x = torch.randn(m, K, generator=torch.Generator().manual_seed(m)).to(xdt).to(dev)
+    y = rq.quantized_matmul(x, wq, s, b, True, gs, bits).double()
+    ref = x.double() @ w.t()
+    assert (y - ref).norm() <= 1e-5 * ref.norm() and (y - ref).abs().max() <= 3e-5 * ref.abs().max()
+
+
+def test_qmv_mid_grouped_matches_single(rq, dev):
+    """Several problems of one launch, ragged rows, against their single ones."""
+    K, m = 2048, 11
+    ws = [packed(rq, dev, R, K, 64, 4, torch.bfloat16, R)[0] for R in (2048, 77, 2048, 16, 1)]
+    xs = [torch.randn(m, K, generator=torch.Generator().manual_seed(i)).bfloat16().to(dev) for i in range(5)]
+    ys = rq.grouped_qmv(xs, ws, 64, 4)
+    ref = [rq.quantized_matmul(x, *w, True, 64, 4) for x, w in zip(xs, ws)]
+    for y, r in zip(ys, ref):
+        err = ((y.double() - r.double()).norm() / r.double().norm()).item()
+        assert err <= 2.0 ** -8, err  # another split of K: outputs round either way
