@@ -29,6 +29,7 @@ from typing import List, Sequence, Tuple
 
 import torch
 from torch import Tensor
+from torch.autograd import forward_ad
 
 from . import _lib
 from ._lib import DTYPE_CODE, RQ_EUNSUPPORTED, RqGroupedPlan, RqProblem, check, lib
@@ -51,6 +52,13 @@ def _check_args(group_size: int, bits: int) -> None:
 def _on_gpu(*ts: Tensor) -> None:
     """Every operand on the same GPU: the kernels take raw pointers and run on
     the first operand's device."""
+    d = ts[0].device
+    if d.type == "cuda":
+        for t in ts:
+            if t.device != d:
+                break
+        else:
+            return
     for t in ts:
         if t.device.type != "cuda":
             raise RuntimeError(
@@ -68,8 +76,9 @@ def _float(t: Tensor, name: str) -> None:
 
 def _ready(t: Tensor) -> Tensor:
     """Contiguous and 16-byte aligned (the ABI's requirement)."""
-    t = t.contiguous()
-    if t.numel() and t.data_ptr() % 16:
+    if not t.is_contiguous():
+        t = t.contiguous()
+    if t.data_ptr() % 16 and t.numel():
         t = t.clone()
     return t
 
@@ -83,6 +92,8 @@ def _words(w_q: Tensor) -> Tensor:
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+# the operands are on the GPU, so CUDA is initialised: no lazy-init check per call
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 
 
 def _stream_on(device: torch.device) -> int:
@@ -109,7 +120,7 @@ class _DeviceGuard:
         self.prev = -1
 
     def __enter__(self):
-        cur = torch.cuda.current_device()
+        cur = _current_device()
         if cur != self.idx:
             self.prev = cur
             torch.cuda.set_device(self.idx)
@@ -129,6 +140,7 @@ def _ptr(t: Tensor) -> int:
 _dispatch_modes = torch._C._len_torch_dispatch_stack
 _function_modes = torch._C._len_torch_function_stack
 _functorch_active = torch._C._are_functorch_transforms_active
+_is_compiling = torch.compiler.is_compiling
 
 
 def _direct(*ts: Tensor) -> bool:
@@ -139,13 +151,23 @@ def _direct(*ts: Tensor) -> bool:
     dispatch, which is longer than the small launches take on the GPU.
     Anything else (torch.compile, meta and fake tensors, autograd, CPU
     tensors, which the op refuses) goes through the registered op."""
+    if not _eager(*ts):
+        return False
+    if torch.is_grad_enabled():
+        for t in ts:
+            if t.requires_grad:
+                return False
+    return True
+
+
+def _eager(*ts: Tensor) -> bool:
+    """_direct apart from autograd."""
     if _dispatch_modes() or _function_modes() or _functorch_active():
         return False
-    grad = torch.is_grad_enabled()
     for t in ts:
-        if type(t) is not Tensor or not t.is_cuda or (grad and t.requires_grad):
+        if type(t) is not Tensor or not t.is_cuda:
             return False
-    return not torch.compiler.is_compiling()
+    return not _is_compiling()
 
 
 # --------------------------------------------------------------- quantize
@@ -225,7 +247,7 @@ def _check_packed(w_q: Tensor, scales: Tensor, biases: Tensor, group_size: int, 
     if K % group_size:
         raise ValueError(f"unpacked width {K} is not divisible by group_size {group_size}")
     want = (*w_q.shape[:-1], K // group_size)
-    if tuple(scales.shape) != want or tuple(biases.shape) != want:
+    if scales.shape != want or biases.shape != want:
         raise ValueError(f"scales/biases must have shape {want} "
                          f"(got {tuple(scales.shape)} / {tuple(biases.shape)})")
     return K
@@ -294,34 +316,44 @@ def quantized_embedding(idx: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor
 def _qmm_impl(x: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor, transpose: bool,
             group_size: int, bits: int) -> Tensor:
     _on_gpu(x, w_q, scales, biases)
+    sdt, xdt = scales.dtype, x.dtype
     x, w_q, scales = _ready(x), _ready(w_q), _ready(scales)
-    biases = _ready(biases.to(scales.dtype))
-    R = w_q.shape[0]
-    K = w_q.shape[1] * 32 // bits
-    n_out = R if transpose else K
-    out_dtype = _promote(x.dtype, scales.dtype)
-    m = x.numel() // x.shape[-1] if x.shape[-1] else 0
-    y = torch.empty(*x.shape[:-1], n_out, dtype=out_dtype, device=x.device)
+    biases = _ready(biases if biases.dtype == sdt else biases.to(sdt))
+    R, words = w_q.shape
+    K = words * 32 // bits
+    shape = x.shape
+    out_dtype = xdt if xdt == sdt else torch.float32
+    n_in = shape[-1]
+    m = x.numel() // n_in if n_in else 0
+    y = torch.empty((*shape[:-1], R if transpose else K), dtype=out_dtype, device=x.device)
     if y.numel() == 0:
         return y
     L = lib()
-    with _DeviceGuard(x.device):
-        stream = _stream(x)
+    idx = x.get_device()
+    cur = _current_device()
+    if cur != idx:
+        torch.cuda.set_device(idx)
+    try:
+        stream = _raw_stream(idx) if _raw_stream is not None else _stream(x)
         # prefill batches with few output tiles over a long contraction split it
         # (rq_qmm_splitk, a per-stream workspace); everything else is rq_qmm
         nbytes = L.rq_qmm_splitk_workspace_bytes(m, R, K, group_size, bits) if (
             transpose and m >= 256) else 0
         if nbytes > 0:
             ws = _splitk_workspace(x.device, stream, nbytes)
-            rc = L.rq_qmm_splitk(_ptr(x), DTYPE_CODE[x.dtype], _ptr(w_q), _ptr(scales),
-                                 _ptr(biases), DTYPE_CODE[scales.dtype], m, R, K, group_size,
-                                 bits, _ptr(y), DTYPE_CODE[out_dtype], ws.data_ptr(), ws.numel(),
-                                 stream)
+            rc = L.rq_qmm_splitk(_ptr(x), DTYPE_CODE[xdt], _ptr(w_q), _ptr(scales),
+                                 _ptr(biases), DTYPE_CODE[sdt], m, R, K, group_size,
+                                 bits, y.data_ptr(), DTYPE_CODE[out_dtype], ws.data_ptr(),
+                                 ws.numel(), stream)
         else:
-            rc = L.rq_qmm(_ptr(x), DTYPE_CODE[x.dtype], _ptr(w_q), _ptr(scales), _ptr(biases),
-                          DTYPE_CODE[scales.dtype], m, R, K, group_size, bits,
-                          1 if transpose else 0, _ptr(y), DTYPE_CODE[out_dtype], stream)
-    check(rc, "quantized_matmul")
+            rc = L.rq_qmm(_ptr(x), DTYPE_CODE[xdt], _ptr(w_q), _ptr(scales), _ptr(biases),
+                          DTYPE_CODE[sdt], m, R, K, group_size, bits, 1 if transpose else 0,
+                          y.data_ptr(), DTYPE_CODE[out_dtype], stream)
+    finally:
+        if cur != idx:
+            torch.cuda.set_device(cur)
+    if rc:
+        check(rc, "quantized_matmul")
     return y
 
 
@@ -375,6 +407,28 @@ def _qmm_backward(ctx, grad):
 _qmm_op.register_autograd(_qmm_backward, setup_context=_qmm_setup)
 
 
+class _QmmFunction(torch.autograd.Function):
+    """The registered op's autograd formula without its dispatch: the same saved
+    tensors and the same products, for plain eager GPU tensors (_eager).  The op's
+    own eager autograd costs ~60 us of host time per call and again in the
+    backward, an eager Function ~15."""
+
+    @staticmethod
+    def forward(ctx, x, w_q, scales, biases, transpose, group_size, bits):
+        ctx.save_for_backward(w_q, scales, biases)
+        ctx.transpose, ctx.group_size, ctx.bits, ctx.x_dtype = transpose, group_size, bits, x.dtype
+        return _qmm_impl(x, w_q, scales, biases, transpose, group_size, bits)
+
+    @staticmethod
+    def backward(ctx, grad):
+        w_q, scales, biases = ctx.saved_tensors
+        dx = None
+        if ctx.needs_input_grad[0]:
+            dx = quantized_matmul(grad.contiguous(), w_q, scales, biases, not ctx.transpose,
+                                  ctx.group_size, ctx.bits).to(ctx.x_dtype)
+        return dx, None, None, None, None, None, None
+
+
 def quantized_matmul(x: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor,
                      transpose: bool = True, group_size: int = 64, bits: int = 4) -> Tensor:
     """mx.quantized_matmul.  transpose=True: x @ W^T ; transpose=False: x @ W."""
@@ -389,9 +443,14 @@ def quantized_matmul(x: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor,
     if x.shape[-1] != n_in:
         raise ValueError(f"x has inner dimension {x.shape[-1]} but the quantized weight expects "
                          f"{n_in} (transpose={transpose})")
-    if _direct(x, w_q, scales, biases):
-        return _qmm_impl(x, w_q, scales, biases, bool(transpose), group_size, bits)
-    return _qmm_op(x, w_q, scales, biases, bool(transpose), group_size, bits)
+    transpose = bool(transpose)
+    if _eager(x, w_q, scales, biases) and not (scales.requires_grad or biases.requires_grad):
+        if x.requires_grad and torch.is_grad_enabled():
+            if forward_ad._current_level >= 0:
+                return _qmm_op(x, w_q, scales, biases, transpose, group_size, bits)
+            return _QmmFunction.apply(x, w_q, scales, biases, transpose, group_size, bits)
+        return _qmm_impl(x, w_q, scales, biases, transpose, group_size, bits)
+    return _qmm_op(x, w_q, scales, biases, transpose, group_size, bits)
 
 
 def lora_down(x: Tensor, a: Tensor) -> Tensor:
