@@ -7,6 +7,7 @@
 // contiguous range of the dense side; dequantize stores that range 1 KB per
 // instruction after moving it through LDS.
 #include "rq_common.h"
+#include "rq_store.h"
 #include "rq_launch.h"
 
 namespace {
@@ -32,14 +33,14 @@ __global__ __launch_bounds__(kBlock) void quantize_kernel(
     // Threads past the end still take part in the shuffles (their lane group
     // is entirely past the end because total is a multiple of lpg).
     const bool live = t < total;
+    // runs and groups are numbered through the rows: no division for the row
+    // ([65536, 2048] at 4 bits 64.6 -> 62.9 us, 5.5 TB/s)
     const int64_t tt = live ? t : 0;
-    const int64_t row = tt / runs_per_row;
-    const int64_t run = tt - row * runs_per_row;
 
     // (Loading the wave's 2048 inputs 1 KB per instruction through LDS, the
     // way dequantize stores, measured slower here: 3.2 vs 3.8 TB/s at 4 bits.)
     float v[32];
-    load32_f32<WDT>(w, row * cols + run * 32, v);
+    load32_f32<WDT>(w, tt * 32, v);
 
     float w_min = v[0], w_max = v[0];
 #pragma unroll
@@ -86,9 +87,9 @@ __global__ __launch_bounds__(kBlock) void quantize_kernel(
     uint32_t words[BITS];
     run_pack<BITS>(codes, words);
     if (!live) return;
-    store_run<BITS>(wq + row * (runs_per_row * BITS) + run * BITS, words);
-    if ((run & (lpg - 1)) == 0) {
-        const int64_t gi = row * (cols >> gs_shift) + (run >> (gs_shift - 5));
+    store_run<BITS>(wq + tt * BITS, words);
+    if ((tt & (lpg - 1)) == 0) {
+        const int64_t gi = tt >> (gs_shift - 5);
         typedef typename dt_traits<WDT>::storage S;
         ((S*)scales)[gi] = dt_traits<WDT>::from_f32(scale);
         ((S*)biases)[gi] = dt_traits<WDT>::from_f32(bias);
@@ -100,79 +101,110 @@ __global__ __launch_bounds__(kBlock) void quantize_kernel(
 // mx.dequantize: ŵ = T(T(code*scale) + bias), T = the scales dtype (MLX
 // evaluates multiply and add as two ops in that dtype).  __fmul_rn/__fadd_rn
 // keep the two roundings separate when T is f32.
-template <int BITS, int ODT>
-// One thread per 32-code run.  With idx != NULL this is the embedding
-// lookup: output row r is table row idx[r] (rows = number of indices,
-// src_rows = table rows); an index outside the table gives a row of NaN and
-// reads nothing.
+//
+// The scales dtype is a template parameter: chosen at run time, every value's two
+// roundings were branches (816 VALU instructions and 370 branches a run at 6
+// bits, and a 64-bit division for the row; 294 and 4 now).  [10240, 2560] in bf16:
+// 19.6 -> 15.8 us at 6 bits (4.7 TB/s, the rate of a large copy), 16.4 -> 11.6 at
+// 4 bits; the [65536, 2048] head at 4 bits 72.5 -> 60.3.  What bounds it is HBM.
+
+// One code of a run as fp32; the four-bit pair conversion is that of
+// dequant_word4, the byte one that of dequant_run_fast.
+template <int BITS>
+RQ_DEV void run_values(const uint32_t* words, float* c) {
+    if constexpr (BITS == 4) {
+        typedef float f32x2_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const uint32_t lo = words[w] & 0x0F0F0F0Fu, hi = (words[w] >> 4) & 0x0F0F0F0Fu;
+            const f32x2_t l0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 512.f, false);
+            const f32x2_t l1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 512.f, true);
+            const f32x2_t h0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 512.f, false);
+            const f32x2_t h1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 512.f, true);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                c[8 * w + 2 * i] = l0[i];
+                c[8 * w + 2 * i + 1] = h0[i];
+                c[8 * w + 4 + 2 * i] = l1[i];
+                c[8 * w + 5 + 2 * i] = h1[i];
+            }
+        }
+    } else if constexpr (BITS == 8) {
+#pragma unroll
+        for (int w = 0; w < 8; ++w) {
+            uint32_t v = words[w];
+            asm("" : "+v"(v));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) c[4 * w + i] = (float)(uint8_t)(v >> (8 * i));
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 32; ++j) c[j] = (float)run_code<BITS>(words, j);
+    }
+}
+
+// Two values rounded to DT, back as fp32.
+template <int DT>
+RQ_DEV void round2(float& a, float& b) {
+    if constexpr (DT == RQ_BF16) {
+        const uint32_t v = pack_bf16x2(a, b);
+        a = __uint_as_float(v << 16);
+        b = __uint_as_float(v & 0xffff0000u);
+    } else if constexpr (DT == RQ_F16) {
+        a = f16_bits_to_f32(f32_to_f16_bits(a));
+        b = f16_bits_to_f32(f32_to_f16_bits(b));
+    }
+}
+
+// One thread per 32-code run.  IDX: the embedding lookup, output row r is table
+// row idx[r] (rows = number of indices, src_rows = table rows); an index
+// outside the table gives a row of NaN and reads nothing.
+template <int BITS, int SDT, int ODT, bool IDX>
 __global__ __launch_bounds__(kBlock) void dequantize_kernel(
     const uint32_t* __restrict__ wq, const void* __restrict__ scales,
-    const void* __restrict__ biases, int sb_dt, int64_t rows, int64_t cols, int gs_shift,
+    const void* __restrict__ biases, int64_t rows, int64_t cols, int gs_shift,
     void* __restrict__ out, const int64_t* __restrict__ idx, int64_t src_rows) {
-    // A lane's 32 outputs (64 or 128 B) are staged through LDS so that each
-    // store instruction of the wave writes 1 KB contiguous: the wave's 64
-    // runs are 2048 consecutive outputs (run t lands at t * 32).  Stored
-    // straight from registers, the four 16-B stores of a lane sat 64 B apart,
-    // one request per lane and instruction.  Lane L's chunk i sits at LDS
-    // chunk L*(NC+1) + i (the pad spreads the banks).
-    constexpr int NC = ODT == RQ_F32 ? 8 : 4;  // 16-byte chunks per lane
+    constexpr int NC = kRunChunks<ODT>;
     __shared__ __attribute__((aligned(16))) uint4 stg[kBlock / 64][64 * (NC + 1)];
     const int64_t runs_per_row = cols >> 5;
     const int64_t total = rows * runs_per_row;
     const int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    const int lane = threadIdx.x & 63;
-    const bool live = t < total;
-    const int64_t tt = live ? t : total - 1;
-    const int64_t row = tt / runs_per_row;
-    const int64_t run = tt - row * runs_per_row;
-    const int64_t src = idx ? idx[row] : row;
+    const int64_t tt = t < total ? t : total - 1;
+    int64_t src = tt;  // the run in the table; runs and groups are numbered through the rows
+    if constexpr (IDX) {
+        const int64_t row = total <= 0xffffffffll ? (int64_t)((uint32_t)tt / (uint32_t)runs_per_row)
+                                                  : tt / runs_per_row;
+        const int64_t r = idx[row];
+        src = r < 0 || r >= src_rows ? -1 : r * runs_per_row + (tt - row * runs_per_row);
+    }
     float vals[32];
-    if (src < 0 || src >= src_rows) {
+    if (IDX && src < 0) {
 #pragma unroll
         for (int j = 0; j < 32; ++j) vals[j] = __builtin_nanf("");
     } else {
-        const int64_t gi = src * (cols >> gs_shift) + (run >> (gs_shift - 5));
-        const float s = load_dt(scales, sb_dt, gi);
-        const float b = load_dt(biases, sb_dt, gi);
-
+        const int64_t gi = src >> (gs_shift - 5);
+        typedef typename dt_traits<SDT>::storage S;
+        const float s = dt_traits<SDT>::to_f32(((const S*)scales)[gi]);
+        const float b = dt_traits<SDT>::to_f32(((const S*)biases)[gi]);
         uint32_t words[BITS];
-        load_run<BITS>(wq + src * (runs_per_row * BITS) + run * BITS, words);
+        load_run<BITS>(wq + src * BITS, words);
+        run_values<BITS>(words, vals);
 #pragma unroll
-        for (int j = 0; j < 32; ++j) {
-            const float c = (float)run_code<BITS>(words, j);
-            const float p = round_to_dt(sb_dt, __fmul_rn(c, s));
-            vals[j] = round_to_dt(sb_dt, __fadd_rn(p, b));
-        }
-    }
-    uint4* line = stg[threadIdx.x >> 6];
-    if constexpr (ODT == RQ_F32) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            line[lane * (NC + 1) + i] =
-                make_uint4(__float_as_uint(vals[4 * i]), __float_as_uint(vals[4 * i + 1]),
-                           __float_as_uint(vals[4 * i + 2]), __float_as_uint(vals[4 * i + 3]));
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            uint32_t d[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t lo = dt_traits<ODT>::from_f32(vals[8 * i + 2 * j]);
-                const uint32_t hi = dt_traits<ODT>::from_f32(vals[8 * i + 2 * j + 1]);
-                d[j] = lo | (hi << 16);
+        for (int j = 0; j < 32; j += 2) {
+            float p0 = __fmul_rn(vals[j], s), p1 = __fmul_rn(vals[j + 1], s);
+            if constexpr (SDT == RQ_F32) {  // two roundings: the compiler would contract to fmas
+                asm("" : "+v"(p0));
+                asm("" : "+v"(p1));
             }
-            line[lane * (NC + 1) + i] = make_uint4(d[0], d[1], d[2], d[3]);
+            round2<SDT>(p0, p1);
+            p0 = __fadd_rn(p0, b);
+            p1 = __fadd_rn(p1, b);
+            if constexpr (SDT != ODT) round2<SDT>(p0, p1);  // else the store rounds
+            vals[j] = p0;
+            vals[j + 1] = p1;
         }
     }
-    __builtin_amdgcn_wave_barrier();  // LDS runs in order within the wave
-    const int64_t t0 = t - lane;      // the wave's first run
-    uint4* dst = (uint4*)((uint8_t*)out + t0 * (32 * (ODT == RQ_F32 ? 4 : 2)));
-#pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        const int c = lane + 64 * i;  // chunk c of the wave's output: lane c / NC, its chunk c % NC
-        const uint4 v = line[(c / NC) * (NC + 1) + c % NC];
-        if (t0 + c / NC < total) dst[c] = v;
-    }
+    store_runs<ODT>(vals, stg[threadIdx.x >> 6], t, total, out);
 }
 
 // ---------------------------------------------------------- pack / unpack
@@ -272,31 +304,33 @@ hipError_t launch_quantize(const void* w, int w_dt, int64_t rows, int64_t cols, 
     return hipGetLastError();
 }
 
+template <bool IDX>
+static hipError_t dequantize_launch(const int64_t* idx, int64_t n, const uint32_t* wq,
+                                    const void* scales, const void* biases, int sb_dt, int64_t rows,
+                                    int64_t cols, int gs, int bits, void* out, int out_dt,
+                                    hipStream_t stream) {
+    const int64_t threads = n * (cols / 32);
+    if (threads == 0) return hipSuccess;
+    const int gs_shift = __builtin_ctz(gs);
+    RQ_DISPATCH_BITS(bits, B, RQ_DISPATCH_DT(sb_dt, S, RQ_DISPATCH_DT(out_dt, D,
+        hipLaunchKernelGGL((dequantize_kernel<B, S, D, IDX>), dim3(grid_for(threads)), dim3(kBlock),
+                           0, stream, wq, scales, biases, n, cols, gs_shift, out, idx, rows))));
+    return hipGetLastError();
+}
+
 hipError_t launch_dequantize(const uint32_t* wq, const void* scales, const void* biases,
                              int sb_dt, int64_t rows, int64_t cols, int gs, int bits, void* out,
                              int out_dt, hipStream_t stream) {
-    const int64_t threads = rows * (cols / 32);
-    if (threads == 0) return hipSuccess;
-    const int gs_shift = __builtin_ctz(gs);
-    RQ_DISPATCH_BITS(bits, B, RQ_DISPATCH_DT(out_dt, D,
-        hipLaunchKernelGGL((dequantize_kernel<B, D>), dim3(grid_for(threads)), dim3(kBlock), 0,
-                           stream, wq, scales, biases, sb_dt, rows, cols, gs_shift, out,
-                           (const int64_t*)nullptr, rows)));
-    return hipGetLastError();
+    return dequantize_launch<false>(nullptr, rows, wq, scales, biases, sb_dt, rows, cols, gs, bits,
+                                    out, out_dt, stream);
 }
 
 hipError_t launch_embedding(const int64_t* idx, int64_t n, const uint32_t* wq,
                             const void* scales, const void* biases, int sb_dt, int64_t rows,
                             int64_t cols, int gs, int bits, void* out, int out_dt,
                             hipStream_t stream) {
-    const int64_t threads = n * (cols / 32);
-    if (threads == 0) return hipSuccess;
-    const int gs_shift = __builtin_ctz(gs);
-    RQ_DISPATCH_BITS(bits, B, RQ_DISPATCH_DT(out_dt, D,
-        hipLaunchKernelGGL((dequantize_kernel<B, D>), dim3(grid_for(threads)), dim3(kBlock), 0,
-                           stream, wq, scales, biases, sb_dt, n, cols, gs_shift, out, idx,
-                           rows)));
-    return hipGetLastError();
+    return dequantize_launch<true>(idx, n, wq, scales, biases, sb_dt, rows, cols, gs, bits, out,
+                                   out_dt, stream);
 }
 
 hipError_t launch_pack(const uint8_t* codes, int64_t rows, int64_t cols, int bits, uint32_t* wq,
