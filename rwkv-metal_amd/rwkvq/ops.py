@@ -313,6 +313,35 @@ def quantized_embedding(idx: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor
 
 # ------------------------------------------------------- quantized_matmul
 
+def _round_first(m: int, w_q: Tensor, sdt: torch.dtype, transpose: bool, group_size: int,
+                 bits: int) -> bool:
+    """Whether fp32 activations are rounded to bf16 by a pass of their own.  The
+    GEMMs of 256 rows and more round them as they stage them, with the same
+    result, but every output column tile reads (and rounds) the fp32 rows
+    again: the pass costs 6 bytes an element once and pays where many tiles
+    share it.  Measured in us, fp32 staged against the pass and bf16:
+    64-wide-stage GEMM at 4 bits, M = 1000 / 4096: [10240, 2560] 67.7 / 267.6
+    against 59.8 / 219.8, [2560, 10240] 74.3 / 265.3 against 73.5 / 220.2;
+    M = 512, [3072, 3072] 22.9 against 25.2 and [8192, 2048] 29.0 against 29.2
+    (1e10 multiply-adds are the line, above which every width won);  [2048,
+    8192] at M = 2048 6 bits 103 against 110, M = 4096 196 against 181;
+    narrower outputs lose ([1024, 4096], M = 4096, 51 against 61).  The 256-row
+    tiles of the other widths: [3072, 768] at M = 512 / 4096 16.1 / 170 against
+    15.0 / 87.  Transposed, where a stage's fp32 rows hold the producers up:
+    [2048, 2048] 46.5 against 37.0 at M = 256 and 51.7 against 51.3 at M =
+    4096, [10240, 2560] 203-299 against 151-237, but [1024, 1024] at M = 4096
+    28.3 against 32.1.  fp32 scales take other kernels."""
+    if m < 256 or sdt == torch.float32:
+        return False
+    R, K = w_q.shape[0], w_q.shape[1] * 32 // bits
+    if not transpose:
+        return R >= 1536 and R % 64 == 0 and K % 128 == 0
+    macs = m * R * K
+    if K % 64 == 0 and (K // group_size) % 8 == 0:
+        return (R >= 2560 and macs >= 10 ** 10) or (R >= 2048 and macs >= 6 * 10 ** 10)
+    return macs >= 1.2e9
+
+
 def _qmm_impl(x: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor, transpose: bool,
             group_size: int, bits: int) -> Tensor:
     _on_gpu(x, w_q, scales, biases)
@@ -325,6 +354,8 @@ def _qmm_impl(x: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor, transpose:
     out_dtype = xdt if xdt == sdt else torch.float32
     n_in = shape[-1]
     m = x.numel() // n_in if n_in else 0
+    if xdt == torch.float32 and m >= 256 and _round_first(m, w_q, sdt, transpose, group_size, bits):
+        x = x.to(torch.bfloat16)
     y = torch.empty((*shape[:-1], R if transpose else K), dtype=out_dtype, device=x.device)
     if y.numel() == 0:
         return y
@@ -341,12 +372,12 @@ def _qmm_impl(x: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor, transpose:
             transpose and m >= 256) else 0
         if nbytes > 0:
             ws = _splitk_workspace(x.device, stream, nbytes)
-            rc = L.rq_qmm_splitk(_ptr(x), DTYPE_CODE[xdt], _ptr(w_q), _ptr(scales),
+            rc = L.rq_qmm_splitk(_ptr(x), DTYPE_CODE[x.dtype], _ptr(w_q), _ptr(scales),
                                  _ptr(biases), DTYPE_CODE[sdt], m, R, K, group_size,
                                  bits, y.data_ptr(), DTYPE_CODE[out_dtype], ws.data_ptr(),
                                  ws.numel(), stream)
         else:
-            rc = L.rq_qmm(_ptr(x), DTYPE_CODE[xdt], _ptr(w_q), _ptr(scales), _ptr(biases),
+            rc = L.rq_qmm(_ptr(x), DTYPE_CODE[x.dtype], _ptr(w_q), _ptr(scales), _ptr(biases),
                           DTYPE_CODE[sdt], m, R, K, group_size, bits, 1 if transpose else 0,
                           y.data_ptr(), DTYPE_CODE[out_dtype], stream)
     finally:
