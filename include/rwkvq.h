@@ -281,9 +281,10 @@ int rq_lora_grads_noalloc(const void* x, const void* u, const void* dy, const vo
  * the 64-wide-stage GEMMs (the conditions of rq_qmm_lora).  Other ranks and bit
  * widths there, fewer than 256 rows, and every transposed product run two
  * launches, z and then the GEMM (z_out given, a contraction that is a multiple
- * of 32; fp32 x is not rounded for z).  Anything else returns RQ_EUNSUPPORTED
- * and the caller runs rq_lora_down and rq_qmm_lora.  a, lora and z_out 16-byte
- * aligned. */
+ * of 32; fp32 x is not rounded for z).  Anything else returns RQ_EUNSUPPORTED,
+ * as do forward products of at most 16 rows (rq_qmm multiplies the weights
+ * unrounded there), and the caller runs rq_lora_down and rq_qmm_lora or rq_qmm.
+ * a, lora and z_out 16-byte aligned. */
 int rq_qlora(const void* x, rq_dtype x_dt, const uint32_t* w_q, const void* scales,
              const void* biases, rq_dtype sb_dt, int64_t m, int64_t rows, int64_t cols,
              int group_size, int bits, int transpose, const void* a, const void* lora,

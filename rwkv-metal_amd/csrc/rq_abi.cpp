@@ -536,7 +536,9 @@ static bool qlora_two_launch(int x_dt, int bits, int64_t rank, int64_t m, int64_
 // Products that the in-kernel down-projection does not cover (fewer than 256
 // rows, other ranks and bit widths) as two launches where the GEMM takes the
 // term: z (fp32 x not rounded first), then the GEMM with the term in its output
-// stage.  `stored`: the adapters as rq_qlora_dx has them.
+// stage.  `stored`: the adapters as rq_qlora_dx has them.  Forward products of up
+// to 16 rows stay rq_qmm's: its GEMV multiplies the weights unrounded (and, at
+// one or two fp32 rows, x at 16 significant bits), which no GEMM here does.
 static hipError_t qlora_two_pass(int transpose, const void* x, int x_dt, const uint32_t* w_q,
                                  const void* scales, const void* biases, int sb_dt, int64_t m,
                                  int64_t rows, int64_t cols, int gs, int bits, const void* a,
@@ -544,6 +546,7 @@ static hipError_t qlora_two_pass(int transpose, const void* x, int x_dt, const u
                                  bool stored, hipStream_t stream) {
     const int64_t n_in = transpose ? cols : rows;
     if (!z || n_in % 32 || (x_dt != RQ_BF16 && x_dt != RQ_F32)) return hipErrorNotSupported;
+    if (transpose && m <= 16) return hipErrorNotSupported;
     if (cols > rq::kMidMaxCols || (!transpose && rows > rq::kMidMaxCols)) return hipErrorNotSupported;
     rq::LoraArgs lo{z, lora, rank, scale};
     lo.stored = stored;
@@ -594,8 +597,9 @@ int rq_qlora(const void* x, rq_dtype x_dt, const uint32_t* w_q, const void* scal
     if (e == hipErrorNotSupported)
         return fail(RQ_EUNSUPPORTED,
                     "rq_qlora: needs bf16 or fp32 x and, outside the in-kernel down-projection (rank 16, "
-                    "4- or 8-bit codes, m >= 256, the 64-wide-stage GEMMs), z_out and a contraction "
-                    "that is a multiple of 32; use rq_lora_down and rq_qmm_lora");
+                    "4- or 8-bit codes, m >= 256, the 64-wide-stage GEMMs), z_out, a contraction "
+                    "that is a multiple of 32 and, where transpose=1, m > 16; use rq_lora_down and "
+                    "rq_qmm or rq_qmm_lora");
     return launch_status(e, "rq_qlora");
 }
 

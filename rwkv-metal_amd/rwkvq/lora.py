@@ -53,7 +53,9 @@ class _QLoRAFunction(torch.autograd.Function):
     transpose=False GEMM and adds scale * u A, reading A and B as stored; dA =
     scale * u^T x and dB = scale * dY^T z are one rq_lora_grads launch.  Other ranks and bit widths and
     fewer than 256 rows run the same calls as two launches, z (or u) and the
-    GEMM with the term.  The frozen base gets no gradient.
+    GEMM with the term; the forward of 16 rows and fewer adds the term to
+    quantized_matmul, whose weights are not rounded there.  The frozen base
+    gets no gradient.
 
     fp32 x (the reference's default activations) is rounded to bf16 once for the
     one-launch products, by one cast, and so is fp32 dY: every kernel rounds its fp32 operands to bf16

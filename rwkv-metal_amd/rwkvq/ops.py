@@ -668,8 +668,9 @@ def qlora_product(x: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor, a: Ten
                   bits: int = 4, out_dtype: torch.dtype | None = None):
     """qlora_fused wherever rq_qlora runs it, in one launch or two (z, then the
     GEMM with the term: any rank of 16 to 64, any bit width, any number of
-    rows; z is that of the fp32 x where x is fp32).  None elsewhere.  bf16
-    adapters, bf16 or fp32 x."""
+    rows above the 16 that quantized_matmul multiplies with unrounded weights
+    (any at all where transpose is False); z is that of the fp32 x where x is
+    fp32).  None elsewhere.  bf16 adapters, bf16 or fp32 x."""
     w_q, K, n_out, rank = _qlora_check(x, w_q, scales, biases, a, lora, transpose, group_size, bits)
     _on_gpu(x, w_q, scales, biases, a, lora)
     x, w_q, scales, a, lora = _ready(x), _ready(w_q), _ready(scales), _ready(a), _ready(lora)

@@ -249,3 +249,30 @@ def test_qmv_mid_grouped_matches_single(rq, dev):
     for y, r in zip(ys, ref):
         err = ((y.double() - r.double()).norm() / r.double().norm()).item()
         assert err <= 2.0 ** -8, err  # another split of K: outputs round either way
+
+
+@pytest.mark.parametrize("rank", [16, 48])
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m", [1, 2, 3, 16])
+@pytest.mark.parametrize("R,K,bits,gs", [(768, 768, 4, 64), (96, 416, 3, 32)])
+def test_qlora_decode_rows_keep_the_unrounded_weights(rq, dev, R, K, bits, gs, m, xdt, rank):
+    """A LoRALinear step of up to 16 rows is quantized_matmul's product, whose
+    weights are not rounded, plus the term of the bf16 z: the bits of the two
+    composed, and for fp32 x their fp32 sums (2^-24 an addition)."""
+    from rwkvq import ops
+    (wq, s, b), _ = packed(rq, dev, R, K, gs, bits, torch.bfloat16, R)
+    base = rq.QuantizedLinear(K, R, bias=False, group_size=gs, bits=bits, device=dev)
+    base.weight, base.scales, base.biases = wq, s, b
+    lay = rq.LoRALinear(rank=rank, alpha=32.0, base_module=base)
+    g = torch.Generator().manual_seed(m)
+    with torch.no_grad():
+        lay.lora_b.copy_(torch.randn(R, rank, generator=g) * 0.05)
+    x = torch.randn(m, K, generator=g).to(xdt).to(dev)
+    print("qlora decode rows", m, R, K, bits, rank, xdt, flush=True)
+    A, B = lay.lora_a.detach(), lay.lora_b.detach()
+    z, y = ops.lora_down(x, A), lay(x)
+    assert torch.equal(y, ops.quantized_matmul_lora(x, wq, s, b, z, B, lay.scale, True, gs, bits))
+    ref = rq.quantized_matmul(x, wq, s, b, True, gs, bits).double() + lay.scale * (z.double() @ B.double().t())
+    assert y.dtype == xdt
+    if xdt == torch.float32:
+        assert (y.double() - ref).norm() <= 1e-6 * ref.norm()
