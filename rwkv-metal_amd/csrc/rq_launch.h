@@ -103,7 +103,7 @@ struct LoraArgs {
 // 16, 32, 48 or 64; k a multiple of 32).  a_t: the adapter is given as
 // a^T [k, rank] (row-major, 16-byte aligned) instead.  x_mode: 0 bf16 x; 1
 // fp32 x rounded to bf16 as it is read (z is then that of bf16(x)); 2 fp32 x as
-// the sum of two bf16 values.
+// the sum of three bf16 values, all its 24 significant bits.
 hipError_t launch_lora_down(const void* x, int64_t m, int64_t k, const void* a, int rank, void* z,
                             hipStream_t stream, bool a_t = false, int x_mode = 0);
 

@@ -25,10 +25,14 @@
 //    in the same order.
 //  * XM = 1: x is fp32; each 8-value chunk is loaded as 32 bytes and rounded to
 //    bf16 (RNE) before its MFMA, so z equals the bf16(x) launch's bit for bit.
-//  * XM = 2: fp32 x enters as two bf16 values, hi = bf16(x) and lo = bf16(x -
-//    hi) (16 significant bits), one MFMA each: z is that of the fp32 x within
-//    its own rounding to bf16 (an fp32 matmul with its casts took four torch
-//    launches, ~25 us of GPU time at M = 200, K = 768, rank 32; this 4-5 us).
+//  * XM = 2: fp32 x enters as three bf16 values that add up to it, its
+//    significand's 24 bits eight at a time, one MFMA each: z is that of the
+//    fp32 x, rounded once (an fp32 matmul with its casts took four torch
+//    launches, ~25 us of GPU time at M = 200, K = 768, rank 32; this 7.8 us
+//    with a and 6.8 with a^T in a kernel trace of the layers of width 768,
+//    0.3-0.4 more than two rounded pieces, which hold 16 bits).
+//    The pieces are truncated, not rounded: every remainder is then exact, and
+//    no finite x becomes an infinity.
 #include <mutex>
 
 #include "rq_common.h"
@@ -48,6 +52,17 @@ template <int RT, bool AT = false, int XM = 0> struct LoraShape {
 };
 
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+
+// The upper halves of two fp32 values, as a bf16 pair.
+RQ_DEV uint32_t trunc_bf16x2(float lo, float hi) {
+    return (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xffff0000u);
+}
+// What trunc_bf16x2 leaves of f: exact, and 0 of an infinity (a NaN stays one,
+// also where its upper half is that of an infinity).
+RQ_DEV float bf16_rest(float f) {
+    const float r = f - __uint_as_float(__float_as_uint(f) & 0xffff0000u);
+    return __builtin_fabsf(f) == __builtin_inff() ? 0.f : r;
+}
 
 template <int RT, bool AT = false, int XM = 0>  // rank tiles of 16; AT: a given as a^T
                                                // [K, rank]; XM: 1, 2 for fp32 x
@@ -98,20 +113,23 @@ __global__ __launch_bounds__((64 * LoraShape<RT, AT, XM>::W)) void lora_down_ker
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (s0 + kLoraWaves * u < nsteps) {
-                u32x4_t xv = xa[b][u][0], xl = {0u, 0u, 0u, 0u};
-                if constexpr (XF) {
+                u32x4_t xv = xa[b][u][0], xm = {0u, 0u, 0u, 0u}, xl = xm;
+                if constexpr (XM == 1) {
                     const u32x4_t p = xa[b][u][0], q = xa[b][u][1];
                     xv = u32x4_t{pack_bf16x2(__uint_as_float(p[0]), __uint_as_float(p[1])),
                                  pack_bf16x2(__uint_as_float(p[2]), __uint_as_float(p[3])),
                                  pack_bf16x2(__uint_as_float(q[0]), __uint_as_float(q[1])),
                                  pack_bf16x2(__uint_as_float(q[2]), __uint_as_float(q[3]))};
-                    if constexpr (XM == 2) {
-                        auto rest = [](uint32_t h, uint32_t f0, uint32_t f1) {
-                            return pack_bf16x2(__uint_as_float(f0) - __uint_as_float(h << 16),
-                                               __uint_as_float(f1) - __uint_as_float(h & 0xffff0000u));
-                        };
-                        xl = u32x4_t{rest(xv[0], p[0], p[1]), rest(xv[1], p[2], p[3]),
-                                     rest(xv[2], q[0], q[1]), rest(xv[3], q[2], q[3])};
+                } else if constexpr (XM == 2) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float f0 = __uint_as_float(xa[b][u][e >> 1][2 * (e & 1)]);
+                        float f1 = __uint_as_float(xa[b][u][e >> 1][2 * (e & 1) + 1]);
+                        xv[e] = trunc_bf16x2(f0, f1);
+                        f0 = bf16_rest(f0);
+                        f1 = bf16_rest(f1);
+                        xm[e] = trunc_bf16x2(f0, f1);
+                        xl[e] = trunc_bf16x2(bf16_rest(f0), bf16_rest(f1));
                     }
                 }
                 const bf16x8_t av = __builtin_bit_cast(bf16x8_t, xv);
@@ -138,9 +156,12 @@ __global__ __launch_bounds__((64 * LoraShape<RT, AT, XM>::W)) void lora_down_ker
                     } else {
                         bv = __builtin_bit_cast(bf16x8_t, wb[b][u][t]);
                     }
-                    if constexpr (XM == 2)
+                    if constexpr (XM == 2) {
                         acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                             __builtin_bit_cast(bf16x8_t, xl), bv, acc[t], 0, 0, 0);
+                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            __builtin_bit_cast(bf16x8_t, xm), bv, acc[t], 0, 0, 0);
+                    }
                     acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc[t], 0, 0, 0);
                 }
             }

@@ -276,3 +276,62 @@ def test_qlora_decode_rows_keep_the_unrounded_weights(rq, dev, R, K, bits, gs, m
     assert y.dtype == xdt
     if xdt == torch.float32:
         assert (y.double() - ref).norm() <= 1e-6 * ref.norm()
+
+
+def _z_and_u(rq, dev, x, A, transposed):
+    """z = x A^T of the two-launch forward, or u = dY B of the two-launch dX for
+    dY = x and B = A^T, through a weight that plays no part."""
+    from rwkvq import ops
+    rank, K = A.shape
+    if not transposed:
+        (wq, s, b), _ = packed(rq, dev, 32, K, 32, 4, torch.bfloat16, 1)
+        B = torch.zeros(32, rank, dtype=torch.bfloat16, device=dev)
+        return ops.qlora_product(x, wq, s, b, A, B, 1.0, True, 32, 4, torch.float32)[1]
+    (wq, s, b), _ = packed(rq, dev, K, 32, 32, 4, torch.bfloat16, 1)
+    A2 = torch.zeros(rank, 32, dtype=torch.bfloat16, device=dev)
+    return ops.qlora_dx_product(x, wq, s, b, A2, A.t().contiguous(), 1.0, 32, 4, torch.float32)[1]
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("rank", [16, 32, 48, 64])
+def test_fp32_down_projection_takes_all_24_bits(rq, dev, rank, transposed):
+    """Neighbouring elements of x, all 24 bits in use, that differ from the 17th on, against
+    adapter columns of opposite sign: z is the sum of the differences (each below
+    2^-16, K/2 of them), rounded to bf16 (half a unit in the last of 8
+    significant bits: 2^-8), its fp32 sums K additions of
+    partial sums below 2^4 (2^-24 each, of either sign)."""
+    K, m = 1024, 37
+    g = torch.Generator().manual_seed(rank)
+    v = 1.0 + torch.randint(0, 2 ** 22, (m, K // 2), generator=g).float() * 2.0 ** -23
+    x = torch.empty(m, K)
+    x[:, 0::2], x[:, 1::2] = v + torch.randint(0, 128, v.shape, generator=g) * 2.0 ** -23, v
+    A = torch.ones(rank, K)
+    A[:, 1::2] = -1.0
+    A = (A * torch.where(torch.arange(rank) % 2 == 0, 1.0, -2.0)[:, None]).bfloat16().to(dev)
+    z = _z_and_u(rq, dev, x.to(dev), A, transposed).double()
+    ref = x.double().to(dev) @ A.double().t()
+    sums = K ** 0.5 * 2.0 ** -24 * 2 ** 4
+    assert ((z - ref).abs() <= 2.0 ** -8 * ref.abs() + sums).all(), ((z - ref) / ref).abs().max()
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("rank", [16, 32, 48, 64])
+@pytest.mark.parametrize("val", [float("inf"), -float("inf"), float("nan"), 3.402e38, -3.4e38, 1e-40])
+def test_fp32_down_projection_special_values(rq, dev, val, rank, transposed):
+    """An infinity gives infinities of its sign times the adapter's, a finite value
+    above bf16's largest stays finite, a NaN stays in its row."""
+    K, m = 96, 20
+    g = torch.Generator().manual_seed(rank)
+    x = torch.randn(m, K, generator=g)
+    x[3, 41] = val
+    if val != val:  # payload in the lower half only
+        x.view(torch.int32)[3, 41] = 0x7f800001
+    A = ((torch.rand(rank, K, generator=g) + 0.5) / 64).bfloat16()
+    A[1::2] *= -1
+    z = _z_and_u(rq, dev, x.to(dev), A.to(dev), transposed).cpu().double()
+    ref = x.double() @ A.double().t()
+    assert torch.equal(z.isnan(), ref.isnan()) and torch.equal(z.isinf(), ref.isinf())
+    assert torch.equal(z.sign().nan_to_num(), ref.sign().nan_to_num())
+    ok = ref.isfinite()
+    # fp32 sums of K terms, rounded once to 8 significant bits (half a unit: 2^-8)
+    assert ((z - ref)[ok].abs() <= 2.0 ** -8 * ref[ok].abs() + K * 2.0 ** -24).all()
