@@ -144,6 +144,8 @@ class _LowRankFunction(torch.autograd.Function):
             z = x2 @ lora_a.to(ct).t()   # to be differentiated again: z as a function of x and A
 
         def scaled(p, q):
+            if ops._functorch_active():  # vmap multiplies addmm's first operand by beta
+                return scale * (p @ q)
             return torch.addmm(p.new_empty(p.shape[0], q.shape[1]), p, q, beta=0, alpha=scale)
 
         dx = da = db = None

@@ -80,3 +80,35 @@ def test_low_rank_term_over_sb6(rq, dev, xdt, backend):
             return base(t) + lay.scale * (z @ lay.lora_b.float().t())
         for p, q in zip(second(lay), second(composed)):
             assert (p.float() - q.float()).norm() <= 1e-2 * q.float().norm()
+
+
+def sb6_layer(rq, dev, R, K, r, backend="native", dropout=0.0):
+    import sb6_k3
+    arrays = sb6_k3.random_sb6(R, K, 1, 8, 5)
+    lin = rq.RwkvqLinear(*(t.to(dev) for t in sb6_k3.encode(*arrays, 1)), (R, K), 32, 8, 1)
+    base = {"native": rq.RwkvqNativeLinear, "hybrid": rq.RwkvqHybridLinear}[backend](lin)
+    lay = rq.LoRALinear(rank=r, alpha=32.0, base_module=base, dropout=dropout)
+    with torch.no_grad():
+        lay.lora_b.copy_(torch.randn(R, r, generator=torch.Generator().manual_seed(1)) * 0.05)
+    return lay, base
+
+
+def composed(lay, base, x):
+    """LoRALinear's term as separate ops."""
+    z = x @ lay.lora_a.to(x.dtype).t()
+    return base(x) + lay.scale * (z @ lay.lora_b.to(x.dtype).t())
+
+
+def test_low_rank_term_vmapped_backward(rq, dev, monkeypatch):
+    """Many incoming gradients at once, where memory that new_empty hands out holds
+    NaN.  bf16 adapters: their gradients round to bf16 (2^-8 between neighbours)."""
+    lay, base = sb6_layer(rq, dev, 256, 512, 16)
+    g = torch.Generator().manual_seed(2)
+    x, dys = torch.randn(6, 512, generator=g).to(dev), torch.randn(3, 6, 256, generator=g).to(dev)
+    new_empty = torch.Tensor.new_empty
+    monkeypatch.setattr(torch.Tensor, "new_empty", lambda t, *a, **k: new_empty(t, *a, **k).fill_(float("nan")))
+    out = []
+    for y in (lay(x), composed(lay, base, x)):
+        out.append(torch.vmap(lambda d: torch.autograd.grad(y, (lay.lora_a, lay.lora_b), d, retain_graph=True))(dys))
+    for p, q in zip(*out):
+        assert p.shape == q.shape and (p.float() - q.float()).norm() <= 2.0 ** -8 * q.float().norm()
