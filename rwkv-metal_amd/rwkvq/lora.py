@@ -213,9 +213,10 @@ class LoRALinear(nn.Module):
             return y.reshape(*lead, y.shape[-1])
         base = self.linear(x)
         ct = _promote(x.dtype, self.lora_a.dtype)
+        # autocast would round the base product with the term inside one node
         if (ct == x.dtype == base.dtype and (self.dropout is None or not self.training)
-                and not isinstance(self.linear, nn.Linear) and self.lora_a.is_cuda
-                and ops._eager(x, base) and forward_ad._current_level < 0):
+                and not isinstance(self.linear, nn.Linear) and ops._eager(x, base)
+                and not torch.is_autocast_enabled(x.device.type) and forward_ad._current_level < 0):
             return _LowRankFunction.apply(x.reshape(-1, x.shape[-1]), base.reshape(-1, base.shape[-1]),
                                           self.lora_a, self.lora_b, self.scale).reshape(base.shape)
         z = x.to(ct) @ self.lora_a.to(ct).t()

@@ -112,3 +112,28 @@ def test_low_rank_term_vmapped_backward(rq, dev, monkeypatch):
         out.append(torch.vmap(lambda d: torch.autograd.grad(y, (lay.lora_a, lay.lora_b), d, retain_graph=True))(dys))
     for p, q in zip(*out):
         assert p.shape == q.shape and (p.float() - q.float()).norm() <= 2.0 ** -8 * q.float().norm()
+
+
+@pytest.mark.parametrize("kind", ["native", "hybrid", "rank8"])
+def test_low_rank_term_under_autocast(rq, dev, kind):
+    """fp32 y, its base product not rounded, and gradients: the composed form's."""
+    R, K = 256, 512
+    if kind == "rank8":   # a QuantizedLinear whose term is not fused
+        base = rq.QuantizedLinear.from_linear(torch.nn.Linear(K, R, bias=False, device=dev).bfloat16(), 64, 4)
+        lay = rq.LoRALinear(rank=8, alpha=32.0, base_module=base)
+        with torch.no_grad():
+            lay.lora_b.copy_(torch.randn(R, 8, generator=torch.Generator().manual_seed(1)) * 0.05)
+    else:
+        lay, base = sb6_layer(rq, dev, R, K, 16, kind)
+    g = torch.Generator().manual_seed(2)
+    x = torch.randn(3, 20, K, generator=g).to(dev).requires_grad_(True)
+    dy = torch.randn(3, 20, R, generator=g).to(dev)
+    out = []
+    for f in (lay, lambda t: composed(lay, base, t)):
+        with torch.autocast("cuda", torch.bfloat16):
+            y = f(x)
+        assert y.dtype == torch.float32
+        out.append((y, *torch.autograd.grad(y, [x, lay.lora_a, lay.lora_b], dy)))
+    for p, q in zip(*out):
+        assert p.dtype == q.dtype
+        torch.testing.assert_close(p, q)
