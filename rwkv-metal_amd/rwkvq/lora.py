@@ -214,7 +214,7 @@ class LoRALinear(nn.Module):
         base = self.linear(x)
         ct = _promote(x.dtype, self.lora_a.dtype)
         # autocast would round the base product with the term inside one node
-        if (ct == x.dtype == base.dtype and (self.dropout is None or not self.training)
+        if (ct == x.dtype == base.dtype and (self.dropout is None or not self.dropout.training)
                 and not isinstance(self.linear, nn.Linear) and ops._eager(x, base)
                 and not torch.is_autocast_enabled(x.device.type) and forward_ad._current_level < 0):
             return _LowRankFunction.apply(x.reshape(-1, x.shape[-1]), base.reshape(-1, base.shape[-1]),

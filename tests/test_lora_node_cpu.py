@@ -99,3 +99,16 @@ def test_autocast_keeps_the_base_product(monkeypatch, backward_inside):
     for p, q in zip(*out):
         assert p.dtype == q.dtype
         torch.testing.assert_close(p, q)
+
+
+@pytest.mark.parametrize("training,dropping", [(True, True), (True, False), (False, True), (False, False)])
+def test_dropout_follows_its_own_module(monkeypatch, training, dropping):
+    """A dropout module switched by itself (sampling over masks at inference)."""
+    lay = layer(monkeypatch, dropout=0.5).train(training)
+    lay.dropout.train(dropping)
+    out = []
+    for f in (lay, lambda t: composed(lay, t)):
+        torch.manual_seed(0)
+        out.append(run(lay, f)())
+    for p, q in zip(*out):
+        torch.testing.assert_close(p, q)
