@@ -112,3 +112,17 @@ def test_dropout_follows_its_own_module(monkeypatch, training, dropping):
         out.append(run(lay, f)())
     for p, q in zip(*out):
         torch.testing.assert_close(p, q)
+
+
+def test_adapters_stepped_before_the_backward(monkeypatch):
+    """bf16 adapters under fp32 activations: an update in place between forward and
+    backward leaves the gradients those of the forward's adapters."""
+    lay = layer(monkeypatch)
+    assert lay.lora_a.dtype == torch.bfloat16
+    want = run(lay, lambda t: composed(lay, t))()
+    grads = run(lay, lay)
+    with torch.no_grad():
+        lay.lora_a.mul_(2.0)
+        lay.lora_b.add_(1.0)
+    for p, q in zip(grads(), want):
+        torch.testing.assert_close(p, q)
