@@ -141,6 +141,7 @@ _dispatch_modes = torch._C._len_torch_dispatch_stack
 _function_modes = torch._C._len_torch_function_stack
 _functorch_active = torch._C._are_functorch_transforms_active
 _is_compiling = torch.compiler.is_compiling
+_tracing = torch._C._get_tracing_state  # of torch.jit.trace, which records registered ops
 
 
 def _direct(*ts: Tensor) -> bool:
@@ -149,8 +150,8 @@ def _direct(*ts: Tensor) -> bool:
     dispatch or function mode and no functorch transform.  Such a call does
     exactly what the registered op would do and skips about 13 us of host
     dispatch, which is longer than the small launches take on the GPU.
-    Anything else (torch.compile, meta and fake tensors, autograd, CPU
-    tensors, which the op refuses) goes through the registered op."""
+    Anything else (torch.compile, torch.jit.trace, meta and fake tensors,
+    autograd, CPU tensors, which the op refuses) goes through the registered op."""
     if not _eager(*ts):
         return False
     if torch.is_grad_enabled():
@@ -162,7 +163,7 @@ def _direct(*ts: Tensor) -> bool:
 
 def _eager(*ts: Tensor) -> bool:
     """_direct apart from autograd."""
-    if _dispatch_modes() or _function_modes() or _functorch_active():
+    if _dispatch_modes() or _function_modes() or _functorch_active() or _tracing() is not None:
         return False
     for t in ts:
         if type(t) is not Tensor or not t.is_cuda:

@@ -137,3 +137,16 @@ def test_low_rank_term_under_autocast(rq, dev, kind):
     for p, q in zip(*out):
         assert p.dtype == q.dtype
         torch.testing.assert_close(p, q)
+
+
+@pytest.mark.parametrize("requires_grad", [True, False])
+def test_jit_trace_records_the_registered_op(rq, dev, tmp_path, requires_grad):
+    """A trace holds the op, not this call's result or a Python function: it runs
+    on other inputs and can be saved."""
+    g = torch.Generator().manual_seed(6)
+    wq, s, b = rq.quantize((torch.randn(64, 128, generator=g) * 0.02).bfloat16().to(dev), 32, 4)
+    x, x2 = (torch.randn(20, 128, generator=g).bfloat16().to(dev).requires_grad_(requires_grad) for _ in range(2))
+    f = torch.jit.trace(lambda t: rq.quantized_matmul(t, wq, s, b, True, 32, 4), x, check_trace=False)
+    f.save(str(tmp_path / "f.pt"))
+    want = rq.quantized_matmul(x2, wq, s, b, True, 32, 4)
+    assert torch.equal(f(x2), want) and torch.equal(torch.jit.load(str(tmp_path / "f.pt"))(x2), want)
