@@ -814,7 +814,7 @@ __global__ __launch_bounds__(64 * MAXW) void qmm_n_mid(const MidArgs a) {
         if (r0 + 32 <= a.R) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) c[i].load(wbase + (r0 + i) * wpr * 4, woff);
-        } else {  // rows past the end repeat the last one (x is 0 there)
+        } else {  // rows past the end repeat the last one's codes
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const int64_t r = r0 + 8 * lg + i < a.R ? r0 + 8 * lg + i : a.R - 1;
@@ -823,6 +823,11 @@ __global__ __launch_bounds__(64 * MAXW) void qmm_n_mid(const MidArgs a) {
         }
         const int64_t sr = r0 + (lane & 31) < a.R ? r0 + (lane & 31) : a.R - 1;
         sb.load_sb(sbp + sr * G * SBS, gst, ng);
+        if (r0 + 32 > a.R && r0 + (lane & 31) >= a.R) {
+            // and are 0, as x is there: an infinite weight times 0 would be NaN
+#pragma unroll
+            for (int i = 0; i < SpanRegs<BITS, SB32>::NW; ++i) sb.sb[i] = 0;
+        }
     };
     // activations: as in qmm_t_mid, k -> weight row
     const int qlast = (a.M - m0 < 16 * TM ? (int)(a.M - m0) - 1 : 16 * TM - 1) >> 3;

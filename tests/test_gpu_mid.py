@@ -335,3 +335,18 @@ def test_fp32_down_projection_special_values(rq, dev, val, rank, transposed):
     ok = ref.isfinite()
     # fp32 sums of K terms, rounded once to 8 significant bits (half a unit: 2^-8)
     assert ((z - ref)[ok].abs() <= 2.0 ** -8 * ref[ok].abs() + K * 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("sdt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("R", [1, 31, 45, 77, 96])
+@pytest.mark.parametrize("m", [3, 40, 300])
+def test_mid_transposed_infinite_weights_of_the_last_row(rq, dev, m, R, sdt):
+    """A contraction that ends inside a 32-row step pads with zeros of both
+    operands: infinite weights of the last row give infinities, no NaN."""
+    K, gs = 96, 32
+    (wq, s, b), w = packed(rq, dev, R, K, gs, 4, sdt, R)
+    b[R - 1, 1] = float("inf")
+    w[R - 1, gs:2 * gs] = float("inf")
+    x = torch.rand(m, R, generator=torch.Generator().manual_seed(1)).to(dev) + 0.1
+    y, ref = rq.quantized_matmul(x, wq, s, b, False, gs, 4), x.double() @ w
+    assert torch.equal(y.isinf(), ref.isinf()) and torch.equal(y.isfinite(), ref.isfinite())
