@@ -273,18 +273,20 @@ int rq_lora_grads_noalloc(const void* x, const void* u, const void* dy, const vo
  * [rows, rank], z_out = x . lora_a^T.  dX (transpose=0): a = lora_b^T
  * [rank, rows], lora = lora_a^T [cols, rank], z_out = u = dY . lora_b.
  * z is rounded once to bf16 before the term, as rq_lora_down + rq_qmm_lora
- * do.  Large problems (with z_out given) take two launches instead: z as its
- * own pass, which reads x once, then the GEMM with the term in its output
- * stage -- exactly rq_lora_down + rq_qmm_lora on bf16(x); recomputing z in
- * every output column tile costs more there: outputs at least 4096 wide and
- * twice the contraction.  One launch covers rank 16 with 4- or 8-bit codes on
- * the 64-wide-stage GEMMs (the conditions of rq_qmm_lora).  Other ranks and bit
- * widths there, fewer than 256 rows, and every transposed product run two
- * launches, z and then the GEMM (z_out given, a contraction that is a multiple
- * of 32; fp32 x is not rounded for z).  Anything else returns RQ_EUNSUPPORTED,
- * as do forward products of at most 16 rows (rq_qmm multiplies the weights
- * unrounded there), and the caller runs rq_lora_down and rq_qmm_lora or rq_qmm.
- * a, lora and z_out 16-byte aligned. */
+ * do.
+ * One launch: rank 16 with 4- or 8-bit codes on the 64-wide-stage GEMMs (the
+ * conditions of rq_qmm_lora; transpose=0: cols % 128 == 0).
+ * Two launches, both only with z_out given and a contraction that is a multiple
+ * of 32:
+ *  - of those, outputs at least 4096 wide and twice the contraction: z as its
+ *    own pass, which reads x once, then the GEMM with the term in its output
+ *    stage -- exactly rq_lora_down + rq_qmm_lora on bf16(x); recomputing z in
+ *    every output column tile costs more there;
+ *  - every other problem of bf16 or fp32 x, but for forward products of at most
+ *    16 rows (rq_qmm multiplies the weights unrounded there): z, of fp32 x
+ *    without rounding it, then the GEMM.
+ * Anything else returns RQ_EUNSUPPORTED, and the caller runs rq_lora_down and
+ * rq_qmm_lora or rq_qmm.  a, lora and z_out 16-byte aligned. */
 int rq_qlora(const void* x, rq_dtype x_dt, const uint32_t* w_q, const void* scales,
              const void* biases, rq_dtype sb_dt, int64_t m, int64_t rows, int64_t cols,
              int group_size, int bits, int transpose, const void* a, const void* lora,
@@ -299,9 +301,8 @@ int rq_qlora(const void* x, rq_dtype x_dt, const uint32_t* w_q, const void* scal
  * and u is stored to u_out [m, rank] bf16 (if not NULL) for the adapter
  * gradients.  The same product as rq_qlora with transpose=0, a = lora_b^T
  * and lora = lora_a^T, bit for bit, without the two transposed copies
- * (also where it takes two launches: cols >= 4096 and >= 2 rows, u_out
- * given).  Covers what rq_qlora's dX covers, in as many launches;
- * other problems return RQ_EUNSUPPORTED.  dy, w_q, lora_b and u_out 16-byte
+ * (also where it takes two launches).  Covers what rq_qlora's dX covers, in as
+ * many launches; other problems return RQ_EUNSUPPORTED.  dy, w_q, lora_b and u_out 16-byte
  * aligned, lora_a 2-byte aligned. */
 int rq_qlora_dx(const void* dy, rq_dtype dy_dt, const uint32_t* w_q, const void* scales,
                 const void* biases, rq_dtype sb_dt, int64_t m, int64_t rows, int64_t cols,

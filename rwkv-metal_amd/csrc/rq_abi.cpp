@@ -259,13 +259,6 @@ struct SplitKPlan {
     int bm = 256, splits = 1;
 };
 
-static bool splitk_applies(rq_dtype x_dt, rq_dtype sb_dt, int64_t m, int64_t cols, int gs,
-                           const void* x, const void* scales, const void* biases) {
-    return m >= 256 && (x_dt == RQ_BF16 || x_dt == RQ_F32) && sb_dt != RQ_F32 && cols % 64 == 0 &&
-           (cols / gs) % 8 == 0 &&
-           (((uintptr_t)x | (uintptr_t)scales | (uintptr_t)biases) & 15) == 0;
-}
-
 static SplitKPlan splitk_plan(int64_t m, int64_t rows, int64_t cols, int gs, int bits) {
     const int P = gs / 8;                            // 64-wide stages per 8-group period
     const int64_t nper = cols / (8 * (int64_t)gs);   // periods of the contraction
@@ -324,7 +317,7 @@ int rq_qmm_splitk(const void* x, rq_dtype x_dt, const uint32_t* w_q, const void*
     if (!valid_dt(x_dt) || !valid_dt(sb_dt) || !valid_dt(y_dt)) return fail(RQ_EINVAL, "unsupported dtype");
     if (m < 0) return fail(RQ_EINVAL, "negative m");
     SplitKPlan p;
-    if (splitk_applies(x_dt, sb_dt, m, cols, group_size, x, scales, biases))
+    if (rq::k64_t_covers(x_dt, sb_dt, m, cols, group_size, x, scales, biases))
         p = splitk_plan(m, rows, cols, group_size, bits);
     if (p.splits <= 1)  // not worth splitting (or not the 64-wide-stage GEMM): rq_qmm itself
         return rq_qmm(x, x_dt, w_q, scales, biases, sb_dt, m, rows, cols, group_size, bits, 1, y,
@@ -526,11 +519,16 @@ int rq_qmm_lora(const void* x, rq_dtype x_dt, const uint32_t* w_q, const void* s
 // 150-155 against 139 + 23), and the [2048, 2048] products +5 us fused
 // against +7.  bf16 or fp32 activations (the pass rounds fp32 ones to bf16
 // as the GEMM does, so either gives the bits of bf16(x)), rank 16, 4 or 8
-// bits, m >= 256: where the fused kernels apply.
-static bool qlora_two_launch(int x_dt, int bits, int64_t rank, int64_t m, int64_t n_in,
-                             int64_t n_out) {
-    return (x_dt == RQ_BF16 || x_dt == RQ_F32) && (bits == 4 || bits == 8) && rank == 16 &&
-           m >= 256 && n_in % 32 == 0 && n_out >= 4096 && n_out >= 2 * n_in;
+// bits, m >= 256: where the 64-wide-stage GEMMs run (elsewhere the pass would
+// be made again by qlora_two_pass, which does not round x).
+static bool qlora_two_launch(int transpose, const void* x, int x_dt, const void* scales,
+                             const void* biases, int sb_dt, int64_t m, int64_t rows, int64_t cols,
+                             int gs, int bits, int64_t rank) {
+    const int64_t n_in = transpose ? cols : rows, n_out = transpose ? rows : cols;
+    return (bits == 4 || bits == 8) && rank == 16 && n_in % 32 == 0 && n_out >= 4096 &&
+           n_out >= 2 * n_in &&
+           (transpose ? rq::k64_t_covers(x_dt, sb_dt, m, cols, gs, x, scales, biases)
+                      : rq::k64_n_covers(x_dt, sb_dt, m, rows, cols, bits, x, scales, biases));
 }
 
 // Products that the in-kernel down-projection does not cover (fewer than 256
@@ -576,7 +574,8 @@ int rq_qlora(const void* x, rq_dtype x_dt, const uint32_t* w_q, const void* scal
     if (!aligned16(x) || !aligned16(w_q) || !aligned16(a) || !aligned16(lora) || !aligned16(z_out))
         return fail(RQ_EALIGN, "rq_qlora: x, w_q, a, lora and z_out must be 16-byte aligned");
     hipError_t e;
-    if (z_out && qlora_two_launch(x_dt, bits, rank, m, n_in, n_out)) {
+    if (z_out && qlora_two_launch(transpose, x, x_dt, scales, biases, sb_dt, m, rows, cols,
+                                  group_size, bits, rank)) {
         e = rq::launch_lora_down(x, m, n_in, a, (int)rank, z_out, (hipStream_t)stream,
                                  /*a_t=*/false, x_dt == RQ_F32 ? 1 : 0);
         rq::LoraArgs lo{z_out, lora, (int)rank, scale};
@@ -624,7 +623,8 @@ int rq_qlora_dx(const void* dy, rq_dtype dy_dt, const uint32_t* w_q, const void*
     // u = dY . B from B [rows, rank] as stored; the term scale * u . A from A
     // [rank, cols] as stored
     hipError_t e;
-    if (u_out && qlora_two_launch(dy_dt, bits, rank, m, rows, cols)) {
+    if (u_out && qlora_two_launch(0, dy, dy_dt, scales, biases, sb_dt, m, rows, cols, group_size,
+                                  bits, rank)) {
         e = rq::launch_lora_down(dy, m, rows, lora_b, (int)rank, u_out, (hipStream_t)stream,
                                  /*a_t=*/true, dy_dt == RQ_F32 ? 1 : 0);
         rq::LoraArgs lo{u_out, lora_a, (int)rank, scale};

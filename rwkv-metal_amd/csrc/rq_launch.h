@@ -141,6 +141,24 @@ hipError_t launch_lora_grads(const void* x, const void* u, const void* dy, const
 // The short-batch GEMMs (rq_mid.hip) take weights of up to this many rows and columns.
 constexpr int64_t kMidMaxCols = 1 << 26;
 
+// What the 64-wide-stage GEMMs cover: 256 rows or more of bf16 or fp32
+// activations (fp32 rounded to bf16 as the producers stage them) and 16-bit
+// scales, aligned for whole-line loads.  Forward: whole 8-group chunks of the
+// contraction.
+inline bool k64_t_covers(int x_dt, int sb_dt, int64_t m, int64_t cols, int gs, const void* x,
+                         const void* scales, const void* biases) {
+    return m >= 256 && (x_dt == RQ_BF16 || x_dt == RQ_F32) && sb_dt != RQ_F32 && cols % 64 == 0 &&
+           (cols / gs) % 8 == 0 && (((uintptr_t)x | (uintptr_t)scales | (uintptr_t)biases) & 15) == 0;
+}
+// Transposed: whole stages of 64 weight rows and whole tiles of 128, or at 4 and
+// 8 bits 160, output columns.
+inline bool k64_n_covers(int x_dt, int sb_dt, int64_t m, int64_t rows, int64_t cols, int bits,
+                         const void* x, const void* scales, const void* biases) {
+    return m >= 256 && (x_dt == RQ_BF16 || x_dt == RQ_F32) && sb_dt != RQ_F32 && rows % 64 == 0 &&
+           (cols % 128 == 0 || ((bits == 4 || bits == 8) && cols % 160 == 0)) &&
+           ((uintptr_t)x & 15) == 0 && (((uintptr_t)scales | (uintptr_t)biases) & 7) == 0;
+}
+
 // MFMA GEMM, transpose=True: y[m, rows] = x[m, cols] . W^T.
 hipError_t launch_qmm_t(const void* x, int x_dt, const uint32_t* wq, const void* scales,
                         const void* biases, int sb_dt, int64_t m, int64_t rows, int64_t cols,

@@ -1786,10 +1786,7 @@ hipError_t RQ_CAT(launch_qmm_t_b, RQ_BITS)(const void* x, int x_dt, const uint32
                                       int y_dt, hipStream_t stream, const LoraArgs* lora) {
     const int gs_shift = __builtin_ctz(gs);
     const LoraArgs lo = lora ? *lora : LoraArgs{nullptr, nullptr, 0, 0.f};
-    // bf16 or fp32 activations (fp32 rounded to bf16 as the producers stage them)
-    const bool k64 = m >= 256 && (x_dt == RQ_BF16 || x_dt == RQ_F32) && RQ_GEMM_K64 &&
-                     sb_dt != RQ_F32 && cols % 64 == 0 && (cols / gs) % 8 == 0 &&
-                     (((uintptr_t)x | (uintptr_t)scales | (uintptr_t)biases) & 15) == 0;
+    const bool k64 = RQ_GEMM_K64 && k64_t_covers(x_dt, sb_dt, m, cols, gs, x, scales, biases);
     const bool xf = x_dt == RQ_F32;
     // Small tiles with the contraction split over the waves of a block: fewer
     // than 256 rows (128 x 128 tiles of the same dequantization, one block
@@ -1992,15 +1989,11 @@ hipError_t RQ_CAT(launch_qmm_n_b, RQ_BITS)(const void* x, int x_dt, const uint32
                                       int64_t m, int64_t rows, int64_t cols, int gs, void* y,
                                       int y_dt, hipStream_t stream, const LoraArgs* lora) {
     const LoraArgs lo = lora ? *lora : LoraArgs{nullptr, nullptr, 0, 0.f};
-    // warp-specialised transposed GEMM: bf16 dY, 16-bit aligned scales,
-    // whole stages of 64 weight rows and whole tiles of 128 or 160 output
-    // columns (160: 4- and 8-bit codes)
+    // warp-specialised transposed GEMM
     const bool can128 = cols % 128 == 0;
     const bool can160 = (RQ_BITS == 4 || RQ_BITS == 8) && RQ_GEMM_N160 && cols % 160 == 0;
-    // bf16 or fp32 dY (fp32 rounded to bf16 as the producers stage it)
-    const bool k64 = m >= 256 && (x_dt == RQ_BF16 || x_dt == RQ_F32) && RQ_GEMM_K64 &&
-                     sb_dt != RQ_F32 && rows % 64 == 0 && (can128 || can160) &&
-                     ((uintptr_t)x & 15) == 0 && (((uintptr_t)scales | (uintptr_t)biases) & 7) == 0;
+    const bool k64 = RQ_GEMM_K64 && (can128 || can160) &&
+                     k64_n_covers(x_dt, sb_dt, m, rows, cols, RQ_BITS, x, scales, biases);
     const bool xf = x_dt == RQ_F32;
 #define RQ_NK64(SD, BNV, FZV)                                                                       \
     do {                                                                                           \

@@ -254,3 +254,40 @@ def test_config4_qlora_layer_step_full_size(rq, dev):
         rel_check(dx.reshape(-1, K), xr.grad, what=f"{name} dX")
         rel_check(da, A.grad, what=f"{name} dA")
         rel_check(db, B.grad, what=f"{name} dB")
+
+
+def _launches(f):
+    """Kernels that f() enqueues: the nodes of its captured graph."""
+    import ctypes
+    f()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        f()
+    with open("/proc/self/maps") as maps:
+        path = next(ln.split()[-1] for ln in maps if "libamdhip64" in ln)
+    n = ctypes.c_size_t()
+    rc = ctypes.CDLL(path).hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n))
+    assert rc == 0
+    return n.value
+
+
+@pytest.mark.parametrize("transpose,M,R,K,rank,n", [
+    (True, 300, 2048, 2048, 16, 1), (False, 300, 2048, 2048, 16, 1),
+    (True, 300, 8192, 2048, 16, 2), (False, 300, 2048, 8192, 16, 2),    # much wider than the contraction
+    (True, 300, 5120, 1280, 16, 2), (False, 300, 1312, 5120, 16, 2),    # and no 64-wide stages
+    (True, 300, 2048, 2048, 32, 2), (False, 100, 768, 768, 16, 2)])
+def test_qlora_launch_counts(rq, dev, transpose, M, R, K, rank, n):
+    """The path is decided before anything is launched: no down-projection is made
+    and then made again."""
+    from rwkvq import ops
+    g = torch.Generator().manual_seed(0)
+    wq, s, b = rq.quantize((torch.randn(R, K, generator=g) * 0.02).bfloat16().to(dev), 64, 4)
+    A = torch.randn(rank, K, generator=g).bfloat16().to(dev)
+    B = torch.randn(R, rank, generator=g).bfloat16().to(dev)
+    x = torch.randn(M, K if transpose else R, generator=g).bfloat16().to(dev)
+    say(f"qlora launches {transpose} {M} {R} {K} {rank}")
+    if transpose:
+        assert _launches(lambda: ops.qlora_product(x, wq, s, b, A, B, 2.0, True, 64, 4)) == n
+    else:
+        assert _launches(lambda: ops.qlora_dx_product(x, wq, s, b, A, B, 2.0, 64, 4)) == n
