@@ -247,65 +247,16 @@ int rq_unpack(const uint32_t* w_q, int64_t rows, int64_t cols, int bits, uint8_t
     return launch_status(rq::launch_unpack(w_q, rows, cols, bits, codes, (hipStream_t)stream), "rq_unpack");
 }
 
-// Split-K plan for the 64-wide-stage transpose=1 GEMM.  A cost model over
-// measured per-stage times of one MI355X (1.13 us per 64-wide stage of a
-// 256-row tile, 0.875 us of a 128-row one, 0.43 us of a 64 x 96 one; 256
-// CUs, one block each) and the partial tiles' traffic (written and read once
-// at ~5 TB/s, plus ~3 us for the reduction launch): the split that beats the
-// unsplit launcher's own tile choice by 10 % or more, else none.  Splitting
-// pays where few tiles meet a long contraction (config 3's [2560, 10240] at
-// M = 512 / 2048), not where the partials cost as much as the work.
-struct SplitKPlan {
-    int bm = 256, splits = 1;
-};
-
-static SplitKPlan splitk_plan(int64_t m, int64_t rows, int64_t cols, int gs, int bits) {
-    const int P = gs / 8;                            // 64-wide stages per 8-group period
-    const int64_t nper = cols / (8 * (int64_t)gs);   // periods of the contraction
-    const int bn = (bits == 4 && rows % 160 == 0) ? 160 : 128;
-    const int64_t tn = (rows + bn - 1) / bn;
-    auto cost = [&](int bm, int64_t tiles, int64_t splits, double stage_us) {
-        const int64_t rounds = (tiles * splits + 255) / 256;
-        const int64_t periods = (nper + splits - 1) / splits;
-        double t = (double)rounds * (double)(periods * P) * stage_us;
-        if (splits > 1) t += 2.0 * (double)splits * (double)(m * rows) * 4.0 / 5e6 + 3.0;
-        (void)bm;
-        return t;
-    };
-    // the unsplit launcher's choice (launch_qmm_t_b*)
-    const int64_t t256 = ((m + 255) / 256) * tn, t128 = ((m + 127) / 128) * tn;
-    double plain;
-    if (t256 >= 200) plain = cost(256, t256, 1, 1.13);
-    else if (bits == 4 && t128 < 128) plain = cost(64, ((m + 63) / 64) * ((rows + 95) / 96), 1, 0.43);
-    else plain = cost(128, t128, 1, 0.875);
-    SplitKPlan best;
-    double bt = 0.9 * plain;
-    for (int bm : {256, 128}) {
-        const int64_t tiles = bm == 256 ? t256 : t128;
-        const double stage_us = bm == 256 ? 1.13 : 0.875;
-        for (int64_t s = 2; s <= nper && s <= 32 && tiles * s <= 1024; ++s) {
-            const double t = cost(bm, tiles, s, stage_us);
-            if (t < bt) {
-                bt = t;
-                best.bm = bm;
-                best.splits = (int)s;
-            }
-        }
-    }
-    // the short-batch tiles split the contraction inside a block ([768, 3072] at
-    // M = 512 15.3 -> 11.4 us; [2048, 8192] stays split, 33 against 36)
-    double mid;
-    rq::mid_pick(m, rows, cols, bits, &mid);
-    if (mid < 0.9 * (bt + 2.8)) best.splits = 1;
-    return best;
-}
-
+// Split-K of the 64-wide-stage transpose=1 GEMM, where gemm_plan estimates it
+// faster than both the whole contraction and the short-batch tiles: few tiles
+// and a long contraction ([2560, 10240] at M = 512 / 2048), not where the partials
+// cost as much as the work.
 int64_t rq_qmm_splitk_workspace_bytes(int64_t m, int64_t rows, int64_t cols, int group_size,
                                       int bits) {
     if (int rc = check_common(rows, cols, group_size, bits)) return rc;
     if (m < 0) return fail(RQ_EINVAL, "rq_qmm_splitk_workspace_bytes: negative m");
     if (m < 256 || cols % 64 || (cols / group_size) % 8) return 0;
-    const SplitKPlan p = splitk_plan(m, rows, cols, group_size, bits);
+    const rq::GemmPlan p = rq::gemm_plan(m, rows, cols, group_size, bits, /*may_split=*/true);
     return p.splits > 1 ? (int64_t)p.splits * m * rows * 4 : 0;
 }
 
@@ -316,9 +267,9 @@ int rq_qmm_splitk(const void* x, rq_dtype x_dt, const uint32_t* w_q, const void*
     if (int rc = check_common(rows, cols, group_size, bits)) return rc;
     if (!valid_dt(x_dt) || !valid_dt(sb_dt) || !valid_dt(y_dt)) return fail(RQ_EINVAL, "unsupported dtype");
     if (m < 0) return fail(RQ_EINVAL, "negative m");
-    SplitKPlan p;
+    rq::GemmPlan p;
     if (rq::k64_t_covers(x_dt, sb_dt, m, cols, group_size, x, scales, biases))
-        p = splitk_plan(m, rows, cols, group_size, bits);
+        p = rq::gemm_plan(m, rows, cols, group_size, bits, /*may_split=*/true);
     if (p.splits <= 1)  // not worth splitting (or not the 64-wide-stage GEMM): rq_qmm itself
         return rq_qmm(x, x_dt, w_q, scales, biases, sb_dt, m, rows, cols, group_size, bits, 1, y,
                       y_dt, stream);

@@ -1,10 +1,13 @@
 // rq_mid.h -- which tile the short-batch GEMMs (rq_mid.hip) take and what it
-// costs, for the launchers that choose between them and the large tiles.
+// costs, and the choice between them, the large tiles and a split contraction.
 #pragma once
 
 #include <stdint.h>
 
 namespace rq {
+
+// qmm_t_k64's tiles: 128 rows below this many of 256, 64 below this many of 128
+constexpr int kK64Bm128Below = 200, kK64Bm64Below = 128;
 
 // 16*tm activation rows x 16*tn weight rows, `waves` at most, and the measured
 // time per 128-wide span of a CU that runs one block of it (us; 4-bit codes,
@@ -45,23 +48,98 @@ inline int mid_pick(int64_t m, int64_t n_out, int64_t k, int bits, double* us = 
     return best;
 }
 
-// Estimated us of the 64-wide-stage GEMM (qmm_t_k64) on its own tile choice
-// (m >= 256): per 64-wide stage 0.43 us of a 64 x 96 tile, 0.7 (4 bits, 160
-// columns) or 0.5 of a 128-row one, 1.0 of a 256-row one.
-inline double k64_us(int64_t m, int64_t rows, int64_t cols, int bits) {
-    const int64_t bn = bits == 4 && rows % 160 == 0 ? 160 : 128;
-    const int64_t tn = (rows + bn - 1) / bn, t256 = ((m + 255) / 256) * tn, t128 = ((m + 127) / 128) * tn;
-    int64_t tiles = t256;
-    double stage = 1.0;
-    if (t256 < 200) {
-        tiles = t128;
-        stage = bn == 160 ? 0.7 : 0.5;
-        if (bits == 4 && t128 < 128) {
-            tiles = ((m + 63) / 64) * ((rows + 95) / 96);
-            stage = 0.43;
+// Estimates of the forward GEMMs where the 64-wide stages apply (m >= 256; us, one
+// MI355X), from both forms and the short-batch tiles timed over 17 weight
+// shapes of 0.8 M to 38 M elements at 13 row counts of 256 to 3072 and 3, 4, 6
+// and 8 bits: the plain ones are met within 2 % on average, the split ones
+// within 3 %.
+struct K64Tile {
+    int bm, bn;
+};
+
+// qmm_t_k64's tile for a whole contraction.
+inline K64Tile k64_tile(int64_t m, int64_t rows, int bits) {
+    // 160-row tiles (whole rounds over 256 CUs for the 2560-wide RWKV-7 shapes) split
+    // evenly into 8-code dequant jobs only at 4 bits
+    const int bn = bits == 4 && rows % 160 == 0 ? 160 : 128;
+    const int64_t tn = (rows + bn - 1) / bn;
+    if (((m + 255) / 256) * tn >= kK64Bm128Below) return {256, bn};
+    // 128-row tiles when 256-row ones leave most CUs idle (small M, narrow R), and at
+    // 4 bits 64 x 96 tiles when 128-row ones still leave half of them idle
+    // (M = 512 with 2560 outputs: 216 tiles instead of 64)
+    if (bits == 4 && ((m + 127) / 128) * tn < kK64Bm64Below) return {64, 96};
+    return {128, bn};
+}
+
+// us per 64-wide stage of a tile
+inline double k64_stage_us(K64Tile t, int bits) {
+    if (t.bm == 64) return 0.335;
+    if (t.bn == 160) return t.bm == 128 ? 0.70 : 1.02;
+    const bool small = t.bm == 128;
+    if (bits == 4) return small ? 0.54 : 0.88;
+    if (bits == 8) return small ? 0.59 : 0.92;
+    return bits < 4 ? (small ? 0.77 : 0.95) : (small ? 0.87 : 1.01);
+}
+
+// Launch (4.6 us on 64-row tiles, 3.6 on others, 6.5 with the reduction; 11.5 more
+// on 256-row tiles at the widths other than 4 and 8 bits), rounds over 256 CUs x
+// stages, and the output: one store, or `splits` fp32 partial tiles written and
+// read back by the reduction.
+inline double k64_us(int64_t m, int64_t rows, int64_t cols, int gs, int bits, K64Tile t, int64_t splits) {
+    const int64_t tiles = ((m + t.bm - 1) / t.bm) * ((rows + t.bn - 1) / t.bn) * splits;
+    const int64_t nper = cols / (8 * (int64_t)gs);  // a split is of whole 8-group periods
+    const int64_t stages = ((nper + splits - 1) / splits) * (gs / 8);
+    const double mouts = 1e-6 * (double)(m * rows);
+    double us = splits == 1 ? (t.bm == 64 ? 4.6 : 3.6) + 0.8 * mouts : 6.5 + 1.6 * (double)splits * mouts;
+    if (t.bm == 256 && bits != 4 && bits != 8) us += 11.5;
+    // measured 6 % longer on the smaller tiles of a split
+    const double stage = k64_stage_us(t, bits) * (splits > 1 && t.bm == 128 ? 1.06 : 1.0);
+    return us + (double)((tiles + 255) / 256) * (double)stages * stage;
+}
+
+// The short-batch tiles at 256 rows and more: beside mid_pick's estimate the
+// output and what the tiles re-read from L2.
+inline double mid_us(int64_t m, int64_t rows, int64_t cols, int bits) {
+    double us;
+    mid_pick(m, rows, cols, bits, &us);
+    const double mouts = 1e-6 * (double)(m * rows);
+    if (bits < 4) us *= 1.08;  // measured at 3 bits
+    return us * (1.0 + 4e-6 * mouts * (double)cols) + 0.9 * mouts;
+}
+
+// The form with the least estimate.  Timed over those shapes at 2 to 5 bits it is
+// 6.8 % faster on average than the plain and split forms alone ([1024, 4096] at
+// M = 512, 4 bits, 17.3 -> 14.6 us, [768, 3072] 14.9 -> 11.9); the largest loss is
+// [1536, 1536] at M = 512, 4 bits, 13.0 -> 13.9.  One estimator for all three:
+// with another for the split, [3072, 3072] at M = 640 left its split (26 us) for
+// short-batch tiles (30) and [12288, 3072] its large tiles (93) for them (106).
+struct GemmPlan {
+    bool mid = false;
+    int bm = 0, splits = 1;  // > 1: qmm_t_k64 on bm-row tiles into partial tiles
+};
+inline GemmPlan gemm_plan(int64_t m, int64_t rows, int64_t cols, int gs, int bits, bool may_split) {
+    GemmPlan p;
+    const K64Tile t = k64_tile(m, rows, bits);
+    double best = k64_us(m, rows, cols, gs, bits, t, 1);
+    p.bm = t.bm;
+    const int bn = bits == 4 && rows % 160 == 0 ? 160 : 128;
+    const int64_t nper = cols / (8 * (int64_t)gs);
+    for (int bm = 256; may_split && bm >= 128; bm /= 2) {
+        const int64_t tiles = ((m + bm - 1) / bm) * ((rows + bn - 1) / bn);
+        for (int64_t s = 2; s <= nper && s <= 32 && tiles * s <= 1024; ++s) {
+            const double us = 1.02 * k64_us(m, rows, cols, gs, bits, {bm, bn}, s);  // not for a tie
+            if (us < best) {
+                best = us;
+                p.bm = bm;
+                p.splits = (int)s;
+            }
         }
     }
-    return 2.8 + (double)((tiles + 255) / 256) * (double)(cols / 64) * stage;
+    if (mid_us(m, rows, cols, bits) < best) {
+        p.mid = true;
+        p.splits = 1;
+    }
+    return p;
 }
 
 // Estimated us of the 32-wide-stage GEMMs that take what qmm_t_k64 does not:

@@ -401,12 +401,6 @@ constexpr int kWsBlock = 512;
 #ifndef RQ_K64_PPRIO
 #define RQ_K64_PPRIO 2  // qmm_t_k64: wave priority of the producer waves (0-3; 2 measured +4-6%)
 #endif
-#ifndef RQ_K64_BM128_BELOW
-#define RQ_K64_BM128_BELOW 200  // qmm_t_k64: 128-row tiles when 256-row ones number fewer
-#endif
-#ifndef RQ_K64_BM64_BELOW
-#define RQ_K64_BM64_BELOW 128  // qmm_t_k64, 4 bits: 64 x 96 tiles when 128-row ones number fewer
-#endif
 #ifndef RQ_K64_CPRIO
 #define RQ_K64_CPRIO 0  // qmm_t_k64: wave priority of the MFMA waves (0-3)
 #endif
@@ -1794,19 +1788,20 @@ hipError_t RQ_CAT(launch_qmm_t_b, RQ_BITS)(const void* x, int x_dt, const uint32
     // M = 77, on 16 CUs; these take 7 and 17), and above where their estimate
     // is the lower one.  Measured at 4 bits: [768, 768] (12 groups, no
     // 64-wide stages) at M = 300 / 2048 26.2 / 27.3 -> 5.1 / 11.5 us, [1024,
-    // 1024] at M = 512 10.6 -> 6.8, [2048, 2048] at M = 512 16.2 -> 12.9, but
-    // [8192, 2048] 24 against 39.  The choice does not depend on x's type where
+    // 1024] at M = 512 10.5 -> 7.1, [2048, 2048] at M = 512 16.3 -> 14.6, but
+    // [8192, 2048] 24 against 41.  The choice does not depend on x's type where
     // the 64-wide stages apply: fp32 x gives the bits of bf16(x).  Offsets
     // inside a tile are 32-bit.
     if (cols <= kMidMaxCols && (!lora || (lora->mid && !lora->a))) {
         bool mid = m < 256;
-        if (!mid) {
-            double us;
-            mid_pick(m, rows, cols, RQ_BITS, &us);
-            if (k64) mid = us < k64_us(m, rows, cols, RQ_BITS);
+        if (!mid && k64) {
+            mid = gemm_plan(m, rows, cols, gs, RQ_BITS, /*may_split=*/false).mid;
+        } else if (!mid) {
             // fp32 tiles are re-read from L2 by every weight tile: [2048, 2048]
             // at M = 2048 72 us against 40 with bf16 x
-            else mid = lora || (xf ? 1.5 * us : us) < wide_us(m, rows, cols, x_dt != RQ_BF16);
+            double us;
+            mid_pick(m, rows, cols, RQ_BITS, &us);
+            mid = lora || (xf ? 1.5 * us : us) < wide_us(m, rows, cols, x_dt != RQ_BF16);
         }
         if (mid)
             return RQ_CAT(launch_qmm_t_mid_b, RQ_BITS)(x, x_dt, wq, scales, biases, sb_dt, m, rows,
@@ -1819,7 +1814,7 @@ hipError_t RQ_CAT(launch_qmm_t_b, RQ_BITS)(const void* x, int x_dt, const uint32
 #if RQ_BITS == 4 || RQ_BITS == 8
         if (!k64 || lora->rank != 16) return hipErrorNotSupported;
         const int tn = (int)((rows + 127) / 128);
-        const int bm = ((m + 255) / 256) * tn < RQ_K64_BM128_BELOW ? 128 : 256;
+        const int bm = ((m + 255) / 256) * tn < kK64Bm128Below ? 128 : 256;
         const int tm = (int)((m + bm - 1) / bm);
         const int blocks = ((tm * tn + 7) / 8) * 8;
 #define RQ_FZ_BMX(SD, GSHV, BMV, XFV)                                                             \
@@ -1848,19 +1843,9 @@ hipError_t RQ_CAT(launch_qmm_t_b, RQ_BITS)(const void* x, int x_dt, const uint32
     }
     // 64-wide stages: 16-bit 16-byte aligned scales, whole 8-group chunks
     if (k64) {
-        // 160-row tiles (whole rounds over 256 CUs for the 2560-wide RWKV-7 shapes) split
-        // evenly into 8-code dequant jobs only at 4 bits
-        int bn = (RQ_BITS == 4 && rows % 160 == 0) ? 160 : 128;
-        int tn = (int)((rows + bn - 1) / bn);
-        // 128-row tiles when 256-row ones leave most CUs idle (small M, narrow R)
-        int bm = ((m + 255) / 256) * tn < RQ_K64_BM128_BELOW ? 128 : 256;
-        // and at 4 bits 64 x 96 tiles when 128-row ones still leave half of them idle
-        // (M = 512 with 2560 outputs: 216 tiles instead of 64)
-        if (RQ_BITS == 4 && bm == 128 && ((m + 127) / 128) * tn < RQ_K64_BM64_BELOW) {
-            bm = 64;
-            bn = 96;
-            tn = (int)((rows + bn - 1) / bn);
-        }
+        const K64Tile t = k64_tile(m, rows, RQ_BITS);
+        const int bm = t.bm, bn = t.bn;
+        const int tn = (int)((rows + bn - 1) / bn);
         const int tm = (int)((m + bm - 1) / bm);
         const int blocks = ((tm * tn + 7) / 8) * 8;
 #define RQ_K64_BMX(SD, BNV, GSHV, BMV, XFV)                                                       \

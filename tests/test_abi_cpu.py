@@ -218,6 +218,21 @@ def test_qmm_splitk_plan_and_rejections(L):
                            None) == -2
 
 
+@pytest.mark.parametrize("m,rows,cols,bits,split", [
+    # us measured split / short-batch tiles / whole contraction
+    (640, 3072, 3072, 4, True),     # 26 / 30 / 40
+    (640, 1536, 6144, 4, True),     # 26 / 30 / 38
+    (1024, 1024, 4096, 8, True),    # 23 / 26 / 39
+    (512, 768, 3072, 4, False),     # 15 / 12 / 21
+    (512, 1024, 4096, 4, False),    # 17 / 15 / 27
+    (512, 1024, 1024, 8, False),    # 13 / 7 / 14
+    (640, 2048, 2048, 4, False),    # 22 / 19 / 17
+    (2048, 4096, 4096, 4, False)])  # 95 / 160 / 69
+def test_splitk_plan_against_the_other_forms(L, m, rows, cols, bits, split):
+    """A contraction is split where that is the fastest of the three forms."""
+    assert (L.rq_qmm_splitk_workspace_bytes(m, rows, cols, 64, bits) > 0) == split
+
+
 def test_qlora_dx_rejections_before_any_device_work(L):
     """rq_qlora_dx validates before it launches: the rank, NULL adapters,
     alignment (16 bytes for dy, lora_b and u_out, which are read or written
