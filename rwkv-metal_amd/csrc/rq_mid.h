@@ -48,6 +48,27 @@ inline int mid_pick(int64_t m, int64_t n_out, int64_t k, int bits, double* us = 
     return best;
 }
 
+// Fewer than 256 rows: the short-batch tiles with their output, and qmm_t_kernel's
+// 128 x 128 tiles, two blocks a CU (us per 64 columns of a round of 512 tiles, and
+// of 256 or fewer).  Over 7 weight shapes of 10240 to 65536 rows, 8 row counts, all
+// six bit widths, bf16 and fp32 x, the form with the lower estimate is the faster
+// one or within 6 % in 670 of 674, and within 11 % in the others.  One choice for
+// both types of x: fp32 x gives the bits of bf16(x).
+inline double mid_short_us(int64_t m, int64_t rows, int64_t cols, int bits) {
+    double us;
+    mid_pick(m, rows, cols, bits, &us);
+    // fp32 x costs them more than the large tiles at 5 and 6 bits, where bf16 x is even
+    return (bits == 5 || bits == 6 ? 1.05 : 1.0) * (us + 2.4e-6 * (double)(m * rows));
+}
+inline double t128_us(int64_t m, int64_t rows, int64_t cols, int bits) {
+    const int64_t tiles = ((m + 127) / 128) * ((rows + 127) / 128), rest = tiles % 512;
+    const bool odd = bits != 4 && bits != 8;
+    const double two = bits == 4 ? 2.0 : (bits == 8 ? 2.4 : (bits < 4 ? 1.9 : 2.43));
+    const double one = bits == 4 ? 1.63 : (bits == 8 ? 1.88 : (bits < 4 ? 1.39 : 1.73));
+    const double round = (double)(tiles / 512) * two + (rest == 0 ? 0.0 : (rest <= 256 ? one : two));
+    return (odd ? 10.0 : 1.5) + round * (double)((cols + 63) / 64) + 1.25e-6 * (double)(m * rows);
+}
+
 // Estimates of the forward GEMMs where the 64-wide stages apply (m >= 256; us, one
 // MI355X), from both forms and the short-batch tiles timed over 17 weight
 // shapes of 0.8 M to 38 M elements at 13 row counts of 256 to 3072 and 3, 4, 6

@@ -8,7 +8,8 @@
 // w.r.t. x, which MLX autograd emits for the QLoRA backward
 // (rwkv_metal/lora/finetune.py:141).
 //
-// Fewer than 256 activation rows of a forward product run rq_mid.hip.
+// Fewer than 256 activation rows of a forward product run rq_mid.hip, or against
+// many weight rows qmm_t (qmm_t_kernel below).
 //
 // qmm_n (qmm_n_kernel) covers the transposed products outside the 64-wide-stage
 // kernels below: block tile BM x 128 outputs, 64 weight rows per stage, 4 waves
@@ -79,6 +80,120 @@ RQ_DEV void store_16dw(uint16_t* lds, const uint32_t* d) {
     u32x4_t* p = (u32x4_t*)lds;
 #pragma unroll
     for (int q = 0; q < 4; ++q) p[q] = u32x4_t{d[4 * q], d[4 * q + 1], d[4 * q + 2], d[4 * q + 3]};
+}
+
+// ----------------------------------------------------------------- qmm_t
+//
+// 17 to 255 activation rows against many weight rows (t128_us): block tile 128 x
+// 128 outputs, 64 contraction elements per stage, 4 waves in a 2 x 2 arrangement.
+// A thread dequantizes one 32-code run of the tile per stage and converts one of
+// activations, so a code and an activation are converted once per 128 x 128
+// outputs; the short-batch tiles convert them once per 64 at most, which is what
+// bounds them there ([65536, 768] at M = 200, 4 bits: bf16 x 63 us against 87, fp32
+// 80 against 116), and have the shorter chains ([10240, 2560] 68 against 40).
+
+template <int BITS, int XDT, int BM>
+__global__ __launch_bounds__(kBlock) void qmm_t_kernel(
+    const void* __restrict__ x, const uint32_t* __restrict__ wq, const void* __restrict__ scales,
+    const void* __restrict__ biases, int sb_dt, int64_t M, int64_t R, int64_t K, int gs_shift,
+    void* __restrict__ y, int y_dt) {
+    constexpr int TM = BM / 32;  // 16-row MFMA tiles per wave along m (wave covers BM/2)
+    constexpr int TN = 4;        // wave covers 64 output columns
+    constexpr int AR = BM / 128; // activation rows loaded per thread per stage
+    __shared__ __attribute__((aligned(16))) uint16_t As[2][BM * LDS_LD];
+    __shared__ __attribute__((aligned(16))) uint16_t Bs[2][BN * LDS_LD];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = wave >> 1, wn = wave & 1;
+    const int lg = lane >> 4, lr = lane & 15;
+    const int64_t m0 = (int64_t)blockIdx.y * BM, n0 = (int64_t)blockIdx.x * BN;
+    const int64_t runs_per_row = K >> 5, wpr = runs_per_row * BITS, G = K >> gs_shift;
+    const int nst = (int)((runs_per_row + 1) >> 1);
+    const int half = tid & 1;           // which run of the stage this thread loads
+    const int64_t brow = n0 + (tid >> 1);
+
+    uint32_t cw[BITS];
+    float sc = 0.f, bi = 0.f;
+    uint32_t xa[AR][16];
+
+    auto gload = [&](int st) {
+        const int64_t run = 2 * (int64_t)st + half;
+        const bool run_ok = run < runs_per_row;
+        if (run_ok && brow < R) {
+            load_run<BITS>(wq + brow * wpr + run * BITS, cw);
+            const int64_t gi = brow * G + (run >> (gs_shift - 5));
+            sc = load_dt(scales, sb_dt, gi);
+            bi = load_dt(biases, sb_dt, gi);
+        } else {
+#pragma unroll
+            for (int w = 0; w < BITS; ++w) cw[w] = 0u;
+            sc = 0.f;
+            bi = 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < AR; ++i) {
+            const int64_t arow = m0 + (tid >> 1) + 128 * i;
+            if (run_ok && arow < M) {
+                load_act_run<XDT>(x, arow, K, run * 32, K, true, xa[i]);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 16; ++q) xa[i][q] = 0u;
+            }
+        }
+    };
+    auto swrite = [&](int buf) {
+        uint32_t d[16];
+        dequant_run_bf16<BITS>(cw, sc, bi, d);
+        store_16dw(&Bs[buf][(tid >> 1) * LDS_LD + half * 32], d);
+#pragma unroll
+        for (int i = 0; i < AR; ++i)
+            store_16dw(&As[buf][((tid >> 1) + 128 * i) * LDS_LD + half * 32], xa[i]);
+    };
+
+    f32x4_t acc[TM][TN];
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b) acc[a][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    gload(0);
+    swrite(0);
+    __syncthreads();
+    for (int st = 0; st < nst; ++st) {
+        const int buf = st & 1;
+        if (st + 1 < nst) gload(st + 1);
+#pragma unroll
+        for (int ks = 0; ks < BK / 32; ++ks) {
+            bf16x8_t af[TM], bf[TN];
+#pragma unroll
+            for (int a = 0; a < TM; ++a)
+                af[a] = lds_frag(&As[buf][(wm * (BM / 2) + a * 16 + lr) * LDS_LD + ks * 32 + lg * 8]);
+#pragma unroll
+            for (int b = 0; b < TN; ++b)
+                bf[b] = lds_frag(&Bs[buf][(wn * 64 + b * 16 + lr) * LDS_LD + ks * 32 + lg * 8]);
+#pragma unroll
+            for (int a = 0; a < TM; ++a)
+#pragma unroll
+                for (int b = 0; b < TN; ++b)
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bf[b], acc[a][b],
+                                                                        0, 0, 0);
+        }
+        if (st + 1 < nst) swrite(buf ^ 1);
+        __syncthreads();
+    }
+
+    // D[4*lg + i][lr] of each 16x16 tile: rows are m, columns are n.
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b) {
+            const int64_t n = n0 + wn * 64 + b * 16 + lr;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int64_t m = m0 + wm * (BM / 2) + a * 16 + 4 * lg + i;
+                if (m < M && n < R) store_dt(y, y_dt, m * R + n, acc[a][b][i]);
+            }
+        }
 }
 
 // ----------------------------------------------------------------- qmm_n
@@ -1782,8 +1897,8 @@ hipError_t RQ_CAT(launch_qmm_t_b, RQ_BITS)(const void* x, int x_dt, const uint32
     const LoraArgs lo = lora ? *lora : LoraArgs{nullptr, nullptr, 0, 0.f};
     const bool k64 = RQ_GEMM_K64 && k64_t_covers(x_dt, sb_dt, m, cols, gs, x, scales, biases);
     const bool xf = x_dt == RQ_F32;
-    // Small tiles with the contraction split over the waves of a block: fewer
-    // than 256 rows (128 x 128 tiles of the same dequantization, one block
+    // Small tiles with the contraction split over the waves of a block: most
+    // products of fewer than 256 rows (128 x 128 tiles of the same dequantization, one block
     // walking all of K, took 58 us on [2048, 2048] and 220 on [2048, 8192] at
     // M = 77, on 16 CUs; these take 7 and 17), and above where their estimate
     // is the lower one.  Measured at 4 bits: [768, 768] (12 groups, no
@@ -1793,10 +1908,11 @@ hipError_t RQ_CAT(launch_qmm_t_b, RQ_BITS)(const void* x, int x_dt, const uint32
     // the 64-wide stages apply: fp32 x gives the bits of bf16(x).  Offsets
     // inside a tile are 32-bit.
     if (cols <= kMidMaxCols && (!lora || (lora->mid && !lora->a))) {
-        bool mid = m < 256;
-        if (!mid && k64) {
+        bool mid = m < 256 && (lora || mid_short_us(m, rows, cols, RQ_BITS) <=
+                                           t128_us(m, rows, cols, RQ_BITS));
+        if (k64) {
             mid = gemm_plan(m, rows, cols, gs, RQ_BITS, /*may_split=*/false).mid;
-        } else if (!mid) {
+        } else if (m >= 256) {
             // fp32 tiles are re-read from L2 by every weight tile: [2048, 2048]
             // at M = 2048 72 us against 40 with bf16 x
             double us;
@@ -1909,6 +2025,14 @@ hipError_t RQ_CAT(launch_qmm_t_b, RQ_BITS)(const void* x, int x_dt, const uint32
             if (bn == 160) { RQ_DMA(160, false); } else { RQ_DMA(128, false); }
         }
 #undef RQ_DMA
+        return hipGetLastError();
+    }
+    if (m < 256) {
+        constexpr int BM = 128;
+        const dim3 grid((unsigned)((rows + BN - 1) / BN), (unsigned)((m + BM - 1) / BM));
+        RQ_DISPATCH_DT(x_dt, XD,
+            hipLaunchKernelGGL((qmm_t_kernel<RQ_BITS, XD, BM>), grid, dim3(kBlock), 0, stream, x, wq,
+                               scales, biases, sb_dt, m, rows, cols, gs_shift, y, y_dt));
         return hipGetLastError();
     }
     {

@@ -350,3 +350,18 @@ def test_mid_transposed_infinite_weights_of_the_last_row(rq, dev, m, R, sdt):
     x = torch.rand(m, R, generator=torch.Generator().manual_seed(1)).to(dev) + 0.1
     y, ref = rq.quantized_matmul(x, wq, s, b, False, gs, 4), x.double() @ w
     assert torch.equal(y.isinf(), ref.isinf()) and torch.equal(y.isfinite(), ref.isfinite())
+
+
+@pytest.mark.parametrize("xdt,sdt", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32),
+                                     (torch.float16, torch.float16), (torch.float32, torch.bfloat16)])
+@pytest.mark.parametrize("m,R,K,bits,gs", [(255, 65537, 64, 4, 64), (129, 60001, 96, 8, 32), (200, 65536, 160, 3, 32),
+                                           (130, 65530, 128, 5, 128), (255, 65500, 384, 6, 64), (255, 65536, 256, 2, 32)])
+def test_forward_128_tiles_of_many_weight_rows(rq, dev, m, R, K, bits, gs, xdt, sdt):
+    """Rows and columns past a tile, contractions that end inside a 64-wide stage."""
+    (wq, s, b), w = packed(rq, dev, R, K, gs, bits, sdt, m + K)
+    x = torch.randn(m, K, generator=torch.Generator().manual_seed(m)).to(xdt).to(dev)
+    print("forward 128 tiles", m, R, K, bits, xdt, sdt, flush=True)
+    y = rq.quantized_matmul(x, wq, s, b, True, gs, bits)
+    check(y, (x.bfloat16().double() @ w.t(), out_dtype(xdt, sdt)), K, "128 tiles")
+    if xdt == torch.float32 and sdt == torch.float32:
+        assert torch.equal(y, rq.quantized_matmul(x.bfloat16(), wq, s, b, True, gs, bits))
