@@ -282,9 +282,10 @@ int rq_lora_grads_noalloc(const void* x, const void* u, const void* dy, const vo
  *    own pass, which reads x once, then the GEMM with the term in its output
  *    stage -- exactly rq_lora_down + rq_qmm_lora on bf16(x); recomputing z in
  *    every output column tile costs more there;
- *  - every other problem of bf16 or fp32 x, but for forward products of at most
- *    16 rows (rq_qmm multiplies the weights unrounded there): z, of fp32 x
- *    without rounding it, then the GEMM.
+ *  - every other problem of bf16 or fp32 x: z, of fp32 x without rounding it,
+ *    then the GEMM; but for forward products of at most 16 rows (rq_qmm
+ *    multiplies the weights unrounded there) and those of 256 and more outside
+ *    the 64-wide stages that the large tiles run faster, term and all.
  * Anything else returns RQ_EUNSUPPORTED, and the caller runs rq_lora_down and
  * rq_qmm_lora or rq_qmm.  a, lora and z_out 16-byte aligned. */
 int rq_qlora(const void* x, rq_dtype x_dt, const uint32_t* w_q, const void* scales,

@@ -496,6 +496,9 @@ static hipError_t qlora_two_pass(int transpose, const void* x, int x_dt, const u
     const int64_t n_in = transpose ? cols : rows;
     if (!z || n_in % 32 || (x_dt != RQ_BF16 && x_dt != RQ_F32)) return hipErrorNotSupported;
     if (transpose && m <= 16) return hipErrorNotSupported;
+    const bool k64 = rq::k64_t_covers(x_dt, sb_dt, m, cols, gs, x, scales, biases);
+    if (transpose && !k64 && !rq::forward_takes_mid(x_dt, false, true, m, rows, cols, gs, bits))
+        return hipErrorNotSupported;
     if (cols > rq::kMidMaxCols || (!transpose && rows > rq::kMidMaxCols)) return hipErrorNotSupported;
     rq::LoraArgs lo{z, lora, rank, scale};
     lo.stored = stored;

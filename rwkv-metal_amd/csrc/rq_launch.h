@@ -138,9 +138,6 @@ hipError_t launch_lora_grads(const void* x, const void* u, const void* dy, const
                              void* db, const LoraGradPlan& p, void* work, hipStream_t stream,
                              bool xdy_f32 = false);
 
-// The short-batch GEMMs (rq_mid.hip) take weights of up to this many rows and columns.
-constexpr int64_t kMidMaxCols = 1 << 26;
-
 // What the 64-wide-stage GEMMs cover: 256 rows or more of bf16 or fp32
 // activations (fp32 rounded to bf16 as the producers stage them) and 16-bit
 // scales, aligned for whole-line loads.  Forward: whole 8-group chunks of the

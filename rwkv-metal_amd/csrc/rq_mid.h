@@ -4,6 +4,8 @@
 
 #include <stdint.h>
 
+#include "../../include/rwkvq.h"
+
 namespace rq {
 
 // qmm_t_k64's tiles: 128 rows below this many of 256, 64 below this many of 128
@@ -163,13 +165,45 @@ inline GemmPlan gemm_plan(int64_t m, int64_t rows, int64_t cols, int gs, int bit
     return p;
 }
 
-// Estimated us of the 32-wide-stage GEMMs that take what qmm_t_k64 does not:
-// 256-row tiles, 1.05 us per stage (qmm_t_ws), 2.0 with fp32 activations
-// (qmm_t_big).
-inline double wide_us(int64_t m, int64_t rows, int64_t cols, bool x32) {
-    const int64_t bn = rows % 160 == 0 ? 160 : 128;
+// 256 rows and more where the 64-wide stages do not apply (fp32 scales, groups that
+// are no multiple of 8, f16 x): the 32-wide-stage GEMMs, 256-row tiles
+// (qmm_t_ws, and with fp32 or f16 x qmm_t_big), against the short-batch tiles, whose
+// fp32 rows are read again from L2 by every weight tile.  Both timed alone over 25
+// weight shapes of 0.5 M to 67 M elements, M = 256 to 4096, 4, 5, 6 and 8 bits: of 924
+// products 30 lose more than 5 % to the other form, most of them fp32 x at M = 4096.
+inline double wide_us(int64_t m, int64_t rows, int64_t cols, int bits, bool x16) {
+    const bool w160 = rows % 160 == 0;
+    const int64_t bn = w160 ? 160 : 128;
     const int64_t tiles = ((m + 255) / 256) * ((rows + bn - 1) / bn);
-    return 3.0 + (double)((tiles + 255) / 256) * (double)((cols + 31) / 32) * (x32 ? 2.0 : 1.05);
+    const double stages = (double)((tiles + 255) / 256) * (double)((cols + 31) / 32);
+    const double mouts = 1e-6 * (double)(m * rows);
+    if (!x16) return stages * (w160 ? 2.75 : 2.1) + 2.5 * mouts;
+    const double stage = bits == 4 || bits == 8 ? (w160 ? 0.62 : 0.53) : (w160 ? 1.27 : 1.05);
+    return 13.0 + stages * stage + 1.5 * mouts;
+}
+inline double mid_wide_us(int64_t m, int64_t rows, int64_t cols, int bits, bool x32) {
+    double us;
+    mid_pick(m, rows, cols, bits, &us);
+    const double mouts = 1e-6 * (double)(m * rows);
+    return us * (1.0 + (x32 ? 55e-6 : 7e-6) * mouts * (double)cols) + (x32 ? 4.8 : 2.2) * mouts;
+}
+
+// The short-batch GEMMs take weights of up to this many rows and columns (offsets
+// inside a tile are 32-bit).
+constexpr int64_t kMidMaxCols = 1 << 26;
+
+// Whether a forward product runs the short-batch tiles.  k64: the 64-wide stages
+// apply.  lora: with the low-rank term in its output stage, which of the others
+// only the 64-wide stages can add; elsewhere it takes launches of its own, ~15 us and
+// 24 bytes an output.
+inline bool forward_takes_mid(int x_dt, bool k64, bool lora, int64_t m, int64_t rows, int64_t cols,
+                              int gs, int bits) {
+    if (cols > kMidMaxCols) return false;
+    if (k64) return gemm_plan(m, rows, cols, gs, bits, /*may_split=*/false).mid;
+    if (m < 256) return lora || mid_short_us(m, rows, cols, bits) <= t128_us(m, rows, cols, bits);
+    const double term = lora ? 15.0 + 4.8e-6 * (double)(m * rows) : 0.0;
+    return mid_wide_us(m, rows, cols, bits, x_dt == RQ_F32) <
+           wide_us(m, rows, cols, bits, x_dt == RQ_BF16) + term;
 }
 
 }  // namespace rq

@@ -1898,31 +1898,18 @@ hipError_t RQ_CAT(launch_qmm_t_b, RQ_BITS)(const void* x, int x_dt, const uint32
     const bool k64 = RQ_GEMM_K64 && k64_t_covers(x_dt, sb_dt, m, cols, gs, x, scales, biases);
     const bool xf = x_dt == RQ_F32;
     // Small tiles with the contraction split over the waves of a block: most
-    // products of fewer than 256 rows (128 x 128 tiles of the same dequantization, one block
-    // walking all of K, took 58 us on [2048, 2048] and 220 on [2048, 8192] at
-    // M = 77, on 16 CUs; these take 7 and 17), and above where their estimate
-    // is the lower one.  Measured at 4 bits: [768, 768] (12 groups, no
+    // products of fewer than 256 rows (128 x 128 tiles of the same
+    // dequantization, one block walking all of K, took 58 us on [2048, 2048] and
+    // 220 on [2048, 8192] at M = 77, on 16 CUs; these take 7 and 17), and above
+    // where their estimate is the lower one.  Measured at 4 bits: [768, 768] (12 groups, no
     // 64-wide stages) at M = 300 / 2048 26.2 / 27.3 -> 5.1 / 11.5 us, [1024,
     // 1024] at M = 512 10.5 -> 7.1, [2048, 2048] at M = 512 16.3 -> 14.6, but
     // [8192, 2048] 24 against 41.  The choice does not depend on x's type where
-    // the 64-wide stages apply: fp32 x gives the bits of bf16(x).  Offsets
-    // inside a tile are 32-bit.
-    if (cols <= kMidMaxCols && (!lora || (lora->mid && !lora->a))) {
-        bool mid = m < 256 && (lora || mid_short_us(m, rows, cols, RQ_BITS) <=
-                                           t128_us(m, rows, cols, RQ_BITS));
-        if (k64) {
-            mid = gemm_plan(m, rows, cols, gs, RQ_BITS, /*may_split=*/false).mid;
-        } else if (m >= 256) {
-            // fp32 tiles are re-read from L2 by every weight tile: [2048, 2048]
-            // at M = 2048 72 us against 40 with bf16 x
-            double us;
-            mid_pick(m, rows, cols, RQ_BITS, &us);
-            mid = lora || (xf ? 1.5 * us : us) < wide_us(m, rows, cols, x_dt != RQ_BF16);
-        }
-        if (mid)
-            return RQ_CAT(launch_qmm_t_mid_b, RQ_BITS)(x, x_dt, wq, scales, biases, sb_dt, m, rows,
-                                                  cols, gs, y, y_dt, stream, lora);
-    }
+    // the 64-wide stages apply: fp32 x gives the bits of bf16(x).
+    if ((!lora || (lora->mid && !lora->a)) &&
+        forward_takes_mid(x_dt, k64, lora != nullptr, m, rows, cols, gs, RQ_BITS))
+        return RQ_CAT(launch_qmm_t_mid_b, RQ_BITS)(x, x_dt, wq, scales, biases, sb_dt, m, rows, cols, gs,
+                                              y, y_dt, stream, lora);
     if (lora && lora->a) {
         // the fused QLoRA layer with its down-projection in the kernel: rank 16,
         // 4- or 8-bit codes, 128-column tiles (the 160-column ones have no

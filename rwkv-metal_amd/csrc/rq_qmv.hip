@@ -62,6 +62,7 @@
 
 #include "rq_common.h"
 #include "rq_launch.h"
+#include "rq_mid.h"
 
 #include <cstring>
 #include <vector>
