@@ -192,6 +192,24 @@ inline double mid_wide_us(int64_t m, int64_t rows, int64_t cols, int bits, bool 
 // inside a tile are 32-bit).
 constexpr int64_t kMidMaxCols = 1 << 26;
 
+// Whether a small launch that the split GEMV does not take (fp32 scales, group counts
+// that rule out whole-line loads) runs qmv_kernel with its waves splitting K, rather
+// than qmv_mid: bf16 x of up to 3 rows, where qmv_mid's 16-row MFMA tile is mostly
+// padding and its per-wave staging costs more than the weights.  fp32 scales, one
+// row, qmv_kernel / qmv_mid in us: 4 bits, group size 64, [2048, 2048] 4.3 / 5.1, [8192,
+// 2048] 6.3 / 8.7, [16384, 4096] 14.1 / 23.0 (3 rows 17.5 / 23.5, 4 rows 28.6 / 22.8); 8
+// bits [16384, 4096] 19.9 / 27.5, [16384, 1024] 9.5 / 9.1; 3 bits [16384, 4096] 22.5 /
+// 27.1, [10240, 2560] 14.9 / 13.5; group size 32, 4 bits, [8192, 2048] 7.2 / 8.2, [4096,
+// 4096] 8.9 / 8.3.  5 and 6 bits never, nor fp32 x, which qmv_kernel converts again
+// in every block, nor rows too long for its LDS ([2560, 10240], 3 rows, 17.8 / 12.8).
+inline bool qmv_splits_k(int x_dt, int64_t m, int64_t cols, int gs, int bits, int64_t rowblocks) {
+    if (x_dt != RQ_BF16 || m > 3 || bits == 5 || bits == 6 || m * cols > 12288) return false;
+    if (gs == 32) return m <= 2 && rowblocks >= (bits == 2 || bits == 4 ? 512 : 1024);
+    if (bits == 3) return m <= 2 && rowblocks >= 768 && cols >= 2048;
+    if (bits == 8) return m <= 2 && rowblocks >= (m == 1 ? 128 : 256) && cols >= 1280;
+    return rowblocks >= (m == 1 ? 128 : (m == 2 ? 256 : 512)) && (m < 3 || cols >= 2048);
+}
+
 // Whether a forward product runs the short-batch tiles.  k64: the 64-wide stages
 // apply.  lora: with the low-rank term in its output stage, which of the others
 // only the 64-wide stages can add; elsewhere it takes launches of its own, ~15 us and

@@ -41,8 +41,9 @@
 //    i < MI can be a real activation row (MI = min(M, 4) rounded up to a
 //    power of two), so only those are updated and stored.
 //  * Work unit ("task") = 16*RB rows of one problem.  A block of 4 waves
-//    takes 4 consecutive tasks of one problem; each wave walks every span of
-//    K for its own rows.
+//    takes 4 consecutive tasks of one problem (KS = 1, each wave walks every
+//    span of K for its own rows) or, for small launches, one task whose spans
+//    the 4 waves split and sum in LDS (KS = 4).
 //  * The activation rows x[0..M) of the block's problem are staged once in
 //    LDS as bf16; A operands are read from there for every span, so only
 //    packed codes (and their scales) live in registers: a wave issues the
@@ -56,9 +57,9 @@
 // streamed qmv_stream_* (m <= 4) and qmv_wide_* (4 < m <= 16) for launches
 // that fill the GPU with rows, and qmv_split for small launches (m <= 8; one
 // memory round trip per launch); each is described where it is defined.
-// qmv_mid (rq_mid.hip: any layout, m <= 16) takes the other small launches,
-// and the large ones that would cost qmv_kernel several passes; launch_bucket
-// draws the lines.
+// qmv_mid (rq_mid.hip: any layout, m <= 16) takes most of the other small
+// launches, and the large ones that would cost qmv_kernel several passes;
+// launch_bucket draws the lines.
 
 #include "rq_common.h"
 #include "rq_launch.h"
@@ -271,7 +272,7 @@ constexpr int kLdsBudget = rq::kQmvLdsBudget;  // bytes of LDS staging per block
 // first).  In both, loads are never predicated: out-of-range rows and runs
 // read clamped, in-bounds addresses and are neutralised at compute time by a
 // zero scale and bias (s*D + (b/128 - s)*O = 0).
-template <int BITS, int SDT, int NMC, int MI, int RB, int NS, bool SLDS>
+template <int BITS, int SDT, int NMC, int MI, int RB, int KS, int NS, bool SLDS>
 __global__ __launch_bounds__(kBlock) RQ_QMV_OCC void qmv_kernel(const QmvArgs args) {
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
     typedef typename SBPair<SDT>::type sbp_t;
@@ -295,9 +296,9 @@ __global__ __launch_bounds__(kBlock) RQ_QMV_OCC void qmv_kernel(const QmvArgs ar
     const int gsh = args.gs_shift;
     const int64_t G = K >> gsh;
     const int64_t lblock = bid - args.block_start[p];
-    constexpr int kRowsPerBlock = kWaves * 16 * RB;
+    constexpr int kRowsPerBlock = (KS == 1 ? kWaves : 1) * 16 * RB;
     const int64_t blk_row0 = lblock * kRowsPerBlock;
-    const int64_t row0 = blk_row0 + wave * 16 * RB;
+    const int64_t row0 = blk_row0 + (KS == 1 ? wave * 16 * RB : 0);
 
     const int lg = lane >> 4;  // lane group: run inside the span / k-slice
     const int lr = lane & 15;  // A row m' / weight row inside a 16-row block
@@ -346,11 +347,12 @@ __global__ __launch_bounds__(kBlock) RQ_QMV_OCC void qmv_kernel(const QmvArgs ar
     // The first NS-1 stages of packed codes are requested before the LDS
     // staging below, so their latency overlaps it.  (A wave past the end of
     // its problem loads clamped rows and leaves after the barrier.)
+    const int s0 = KS == 1 ? 0 : wave;
     Stage<BITS, RB> st[NS];
     if constexpr (SLDS) {
 #pragma unroll
         for (int i = 0; i < NS - 1; ++i) {
-            load(i, st[i]);
+            load(s0 + i * KS, st[i]);
             __builtin_amdgcn_sched_barrier(0);  // stage 0 must be the oldest load
         }
     }
@@ -583,12 +585,12 @@ __global__ __launch_bounds__(kBlock) RQ_QMV_OCC void qmv_kernel(const QmvArgs ar
     };
 
     if constexpr (SLDS) {
-        // Rolling pipeline: span s+NS-1 is loaded while span s is computed.
-        for (int s = 0; s < nspans; s += NS) {
+        // Rolling pipeline: span s+(NS-1)*KS is loaded while span s is computed.
+        for (int s = s0; s < nspans; s += NS * KS) {
 #pragma unroll
             for (int i = 0; i < NS; ++i) {
-                load(s + i + NS - 1, st[(i + NS - 1) % NS]);
-                compute(s + i, st[i]);
+                load(s + (i + NS - 1) * KS, st[(i + NS - 1) % NS]);
+                compute(s + i * KS, st[i]);
                 // keep the loads in issue order: the memory counter retires in
                 // order, so a stage loaded late would make its compute drain
                 // every younger load
@@ -597,12 +599,35 @@ __global__ __launch_bounds__(kBlock) RQ_QMV_OCC void qmv_kernel(const QmvArgs ar
         }
     } else {
         // Batches of NS spans: all loads first, then consume in order.
-        for (int s = 0; s < nspans; s += NS) {
+        for (int s = s0; s < nspans; s += NS * KS) {
 #pragma unroll
-            for (int i = 0; i < NS; ++i) load(s + i, st[i]);
+            for (int i = 0; i < NS; ++i) load(s + i * KS, st[i]);
 #pragma unroll
-            for (int i = 0; i < NS; ++i) compute(s + i, st[i]);
+            for (int i = 0; i < NS; ++i) compute(s + i * KS, st[i]);
         }
+    }
+
+    if constexpr (KS > 1) {
+        __shared__ float red[KS][RB][NMC][4][64];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int c = 0; c < NMC; ++c)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) red[wave][rb][c][i][lane] = acc[rb][c][i];
+        __syncthreads();
+        if (wave != 0) return;
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int c = 0; c < NMC; ++c)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    float v = red[0][rb][c][i][lane];
+#pragma unroll
+                    for (int w = 1; w < KS; ++w) v += red[w][rb][c][i][lane];
+                    acc[rb][c][i] = v;
+                }
     }
 
     // Slot combine: D row m' = slot*MC + mm lives in lane group (m'/4), so the
@@ -642,12 +667,28 @@ __global__ __launch_bounds__(kBlock) RQ_QMV_OCC void qmv_kernel(const QmvArgs ar
     }
 }
 
-template <int SDT, int NMC, int MI, int RB, bool XLDS>
+template <int SDT, int NMC, int MI, int RB, int KS, bool XLDS>
 hipError_t launch_one(const QmvArgs& a, int blocks, size_t lds, hipStream_t stream) {
     constexpr int NS = XLDS ? RQ_QMV_NS : RQ_QMV_BATCH;
-    hipLaunchKernelGGL((qmv_kernel<RQ_BITS, SDT, NMC, MI, RB, NS, XLDS>), dim3(blocks),
+    hipLaunchKernelGGL((qmv_kernel<RQ_BITS, SDT, NMC, MI, RB, KS, NS, XLDS>), dim3(blocks),
                        dim3(kBlock), lds, stream, a);
     return hipGetLastError();
+}
+
+// The waves of a block split K: at most 3 activation rows (NMC = 1).
+hipError_t launch_ksplit(const QmvArgs& a, int sb_dt, bool xlds, int blocks, size_t lds,
+                         hipStream_t stream) {
+    hipError_t e = hipErrorInvalidValue;
+#define RQ_QMV_KS(SD, XL)                                                                \
+    switch (a.m) {                                                                       \
+        case 1: e = launch_one<SD, 1, 1, 1, kWaves, XL>(a, blocks, lds, stream); break;   \
+        case 2: e = launch_one<SD, 1, 2, 1, kWaves, XL>(a, blocks, lds, stream); break;   \
+        case 3: e = launch_one<SD, 1, 4, 1, kWaves, XL>(a, blocks, lds, stream); break;   \
+        default: break;                                                                  \
+    }
+    RQ_DISPATCH_DT(sb_dt, SD, if (xlds) { RQ_QMV_KS(SD, true) } else { RQ_QMV_KS(SD, false) });
+#undef RQ_QMV_KS
+    return e;
 }
 
 template <int RB>
@@ -658,11 +699,11 @@ hipError_t launch_cfg(const QmvArgs& a, int sb_dt, int nmc, bool xlds, int block
     const int mi = a.m >= 3 ? 4 : a.m;
 #define RQ_QMV_NMC(SD, XL)                                                                \
     switch (nmc * 8 + (nmc == 1 ? mi : 4)) {                                              \
-        case 9: e = launch_one<SD, 1, 1, RB, XL>(a, blocks, lds, stream); break;       \
-        case 10: e = launch_one<SD, 1, 2, RB, XL>(a, blocks, lds, stream); break;      \
-        case 12: e = launch_one<SD, 1, 4, RB, XL>(a, blocks, lds, stream); break;      \
-        case 20: e = launch_one<SD, 2, 4, RB, XL>(a, blocks, lds, stream); break;      \
-        case 36: e = launch_one<SD, 4, 4, RB, XL>(a, blocks, lds, stream); break;      \
+        case 9: e = launch_one<SD, 1, 1, RB, 1, XL>(a, blocks, lds, stream); break;       \
+        case 10: e = launch_one<SD, 1, 2, RB, 1, XL>(a, blocks, lds, stream); break;      \
+        case 12: e = launch_one<SD, 1, 4, RB, 1, XL>(a, blocks, lds, stream); break;      \
+        case 20: e = launch_one<SD, 2, 4, RB, 1, XL>(a, blocks, lds, stream); break;      \
+        case 36: e = launch_one<SD, 4, 4, RB, 1, XL>(a, blocks, lds, stream); break;      \
         default: break;                                                                   \
     }
     RQ_DISPATCH_DT(sb_dt, SD, if (xlds) { RQ_QMV_NMC(SD, true) } else { RQ_QMV_NMC(SD, false) });
@@ -2200,7 +2241,7 @@ static hipError_t launch_bucket(const rq_problem* const* probs, int n, int x_dt,
         }
         return hipSuccess;
     }
-    // Everything else that is small (more than 8 rows: [2048, 2048] at m = 12
+    // Most of what else is small (more than 8 rows: [2048, 2048] at m = 12
     // 11.7 us on qmv_kernel with the waves splitting K, 5.6 here, [8192, 2048] 13.6
     // -> 8.3, [2048, 8192] 19 -> 10.9; fp32 scales at 6 bits and m = 1, fp32 x,
     // [2048, 2048] 11.4 -> 7.2), and of the large launches those whose activation rows
@@ -2210,7 +2251,8 @@ static hipError_t launch_bucket(const rq_problem* const* probs, int n, int x_dt,
     // than 4 and 8 bits ([65536, 2048], 3 bits, m = 8 56 -> 50, m = 5 41 against
     // 49; [65536, 768], m = 1 21.8 -> 20.7).
     const bool odd_bits = RQ_BITS != 4 && RQ_BITS != 8;
-    if (K <= kMidMaxCols &&
+    const bool ksplit = cfg == 0 && qmv_splits_k(x_dt, m, K, gs, RQ_BITS, rowblocks);
+    if (K <= kMidMaxCols && !ksplit &&
         (cfg == 0 || m > 8 || sb_dt == RQ_F32 || (odd_bits && (m == 8 || K % 512 != 0)))) {
         for (int base = 0; base < n; base += RQ_MAX_GROUPED) {
             const int cnt = (n - base) < RQ_MAX_GROUPED ? (n - base) : RQ_MAX_GROUPED;
@@ -2221,7 +2263,7 @@ static hipError_t launch_bucket(const rq_problem* const* probs, int n, int x_dt,
         return hipSuccess;
     }
     const int RB = cfg == 2 ? RQ_QMV_BIG_RB : 1;
-    const int rows_per_block = 16 * RB * kWaves;
+    const int rows_per_block = ksplit ? 16 : 16 * RB * kWaves;
     // LDS staging: a zero line, activations [m][K] as bf16, their group sums
     // [m][K/gs] fp32, then the block's (scale, bias) pairs.
     const size_t sbsz = sb_dt == RQ_F32 ? 8 : 4;
@@ -2253,7 +2295,8 @@ static hipError_t launch_bucket(const rq_problem* const* probs, int n, int x_dt,
             a.sb_vec &= (((uintptr_t)a.p[i].scales | (uintptr_t)a.p[i].biases) & 15) == 0;
         if (blocks == 0) continue;
         hipError_t e;
-        if (cfg == 2) e = launch_cfg<RQ_QMV_BIG_RB>(a, sb_dt, nmc, xlds, (int)blocks, dyn, stream);
+        if (ksplit) e = launch_ksplit(a, sb_dt, xlds, (int)blocks, dyn, stream);
+        else if (cfg == 2) e = launch_cfg<RQ_QMV_BIG_RB>(a, sb_dt, nmc, xlds, (int)blocks, dyn, stream);
         else e = launch_cfg<1>(a, sb_dt, nmc, xlds, (int)blocks, dyn, stream);
         if (e != hipSuccess) return e;
     }

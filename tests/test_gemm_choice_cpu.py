@@ -15,6 +15,9 @@ extern "C" int short_takes_128(long m, long rows, long cols, int bits) {
 extern "C" int takes_mid(int x_dt, int k64, int lora, long m, long rows, long cols, int gs, int bits) {
     return rq::forward_takes_mid(x_dt, k64, lora, m, rows, cols, gs, bits);
 }
+extern "C" int splits_k(int x_dt, long m, long cols, int gs, int bits, long rowblocks) {
+    return rq::qmv_splits_k(x_dt, m, cols, gs, bits, rowblocks);
+}
 """
 BF16, F32 = 0, 2
 
@@ -30,6 +33,7 @@ def choice(tmp_path_factory):
     lib = ctypes.CDLL(so)
     lib.short_takes_128.argtypes = [ctypes.c_long] * 3 + [ctypes.c_int]
     lib.takes_mid.argtypes = [ctypes.c_int] * 3 + [ctypes.c_long] * 3 + [ctypes.c_int] * 2
+    lib.splits_k.argtypes = [ctypes.c_int] + [ctypes.c_long] * 2 + [ctypes.c_int] * 2 + [ctypes.c_long]
     return lib
 
 
@@ -63,3 +67,22 @@ def test_fewer_than_256_rows(choice, m, rows, cols, bits, big):
     (F32, 1, 100, 65536, 768, 4, True)])
 def test_256_rows_outside_the_64_wide_stages(choice, x_dt, lora, m, rows, cols, bits, mid):
     assert bool(choice.takes_mid(x_dt, 0, lora, m, rows, cols, 32, bits)) == mid
+
+
+@pytest.mark.parametrize("x_dt,m,rows,cols,gs,bits,ks", [
+    # us measured qmv_kernel splitting K / qmv_mid, fp32 scales
+    (BF16, 1, 16384, 4096, 64, 4, True),     # 14.1 / 23.0
+    (BF16, 3, 16384, 4096, 64, 4, True),     # 17.5 / 23.5
+    (BF16, 4, 16384, 4096, 64, 4, False),    # 28.6 / 22.8
+    (F32, 1, 16384, 4096, 64, 4, False),
+    (BF16, 1, 2048, 2048, 64, 4, True),      # 4.3 / 5.1
+    (BF16, 1, 4096, 4096, 32, 4, False),     # 8.9 / 8.3
+    (BF16, 1, 8192, 2048, 32, 4, True),      # 7.2 / 8.2
+    (BF16, 2, 16384, 4096, 128, 8, True),    # 20.2 / 26.5
+    (BF16, 1, 10240, 2560, 64, 3, False),    # 14.9 / 13.5
+    (BF16, 2, 16384, 4096, 128, 3, True),    # 21.4 / 22.9
+    (BF16, 1, 12288, 3072, 128, 2, True),    # 10.2 / 14.5
+    (BF16, 1, 16384, 4096, 32, 6, False),
+    (BF16, 3, 10240, 10240, 64, 4, False)])
+def test_small_decode_launches_outside_the_split_gemv(choice, x_dt, m, rows, cols, gs, bits, ks):
+    assert bool(choice.splits_k(x_dt, m, cols, gs, bits, (rows + 15) // 16)) == ks

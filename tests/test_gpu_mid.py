@@ -365,3 +365,24 @@ def test_forward_128_tiles_of_many_weight_rows(rq, dev, m, R, K, bits, gs, xdt, 
     check(y, (x.bfloat16().double() @ w.t(), out_dtype(xdt, sdt)), K, "128 tiles")
     if xdt == torch.float32 and sdt == torch.float32:
         assert torch.equal(y, rq.quantized_matmul(x.bfloat16(), wq, s, b, True, gs, bits))
+
+
+@pytest.mark.parametrize("m", [1, 2, 3])
+@pytest.mark.parametrize("R,K,gs,bits,sdt", [(8200, 2048, 64, 4, torch.float32), (12290, 2080, 32, 4, torch.float32),
+                                             (16380, 2176, 128, 8, torch.float32), (12300, 2112, 64, 3, torch.float32),
+                                             (8193, 2144, 32, 2, torch.float32), (24000, 1344, 64, 4, torch.bfloat16),
+                                             (8200, 1344, 64, 2, torch.float16)])
+def test_qmv_waves_splitting_k(rq, dev, R, K, gs, bits, sdt, m):
+    """Few bf16 rows against fp32 scales or odd group counts: ragged rows, spans
+    that end inside the contraction; weights unrounded, sums of K products
+    (2^-24 each), a 16-bit y rounded once."""
+    (wq, s, b), _ = packed(rq, dev, R, K, gs, bits, sdt, bits)
+    w = rq.unpack_codes(wq, bits).double().reshape(R, -1, gs)
+    w = (w * s.double()[..., None] + b.double()[..., None]).reshape(R, K)
+    x = torch.randn(m, K, generator=torch.Generator().manual_seed(gs)).bfloat16().to(dev)
+    print("qmv ksplit", R, K, gs, bits, sdt, m, flush=True)
+    y = rq.quantized_matmul(x, wq, s, b, True, gs, bits)
+    ref = x.double() @ w.t()
+    out = 2.0 ** -8 if y.dtype == torch.bfloat16 else 0.0
+    assert (y.double() - ref).norm() <= (1e-5 + out) * ref.norm()
+    assert ((y.double() - ref).abs() <= 3e-5 * ref.abs().max() + 1.01 * out * ref.abs()).all()
