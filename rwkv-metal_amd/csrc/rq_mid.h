@@ -192,6 +192,48 @@ inline double mid_wide_us(int64_t m, int64_t rows, int64_t cols, int bits, bool 
 // inside a tile are 32-bit).
 constexpr int64_t kMidMaxCols = 1 << 26;
 
+// The decode GEMVs; m counts MFMA rows (two for each of fp32 or f16 x at one or two).
+
+// Whether qmv_mid takes a small launch of more than 4 rows from the split GEMV,
+// which makes two passes: few blocks of short rows, and at 7 and 8 rows (at 4 bits
+// from 5, where long enough) more than two blocks a CU; slower between.  Split /
+// qmv_mid in us: m = 8, 4 bits, [768, 768] 5.5 / 4.1, [2560, 2560] 7.5 / 6.6, [10240,
+// 2560] 14.3 / 11.2, [8192, 2048] 8.1 / 8.3; m = 5 [16384, 768] 7.0 / 7.5, and at 6
+// bits [2048, 2048] 7.4 / 8.3, at 2 [16384, 4096] 19.0 / 22.3.
+inline bool qmv_mid_over_split(int x_dt, int64_t m, int64_t cols, int bits, int64_t rowblocks) {
+    if (m <= 4) return false;
+    if (m >= 7)
+        return (rowblocks <= 192 && cols <= 4096) ||
+               (rowblocks > 512 && !(bits == 5 && x_dt == RQ_F32));  // [10240, 2560] 17.4 / 20.0
+    if (bits == 4) return (rowblocks <= 192 && cols <= 4096) || (rowblocks > 512 && cols >= 2048);
+    return rowblocks <= 192 && cols < 2048;
+}
+
+// Whether qmv_mid takes a large launch (2048 blocks of 16 rows and more) that the
+// streamed GEMVs do not cover from qmv_kernel.  Above 8 rows always ([65536, 768] at m
+// = 12, 4 bits, 26 -> 17.6 us).  Below, qmv_kernel / qmv_mid in us:
+//  * 16-bit scales: 3, 5 and 6 bits at 8 rows ([65536, 2048], 3 bits, 55.6 / 51.2) and
+//    in rows of no whole 512 codes ([65536, 768], 6 bits, 35.9 / 30.0; 3 bits at m = 1
+//    17.7 / 18.9); at 2 bits from 5 fp32 rows ([65536, 768], m = 8, 23.2 / 18.5, bf16
+//    14.4 / 17.2).
+//  * fp32 scales: 3, 5 and 6 bits but for up to 4 long rows in groups of 64 and more
+//    ([65536, 2048], m = 1, 3 bits, group size 64, 42.1 / 50.0, 32 51 / 37); the other
+//    widths in groups of 32 but for one or two short bf16 rows (4 bits, [65536, 2048],
+//    m = 1 27.7 / 37.9, m = 8 57 / 40), in groups of 64 from 5 rows where x is fp32 or
+//    long (m = 8, [49152, 3072] 47 / 43; m = 1 26.9 / 41.0, [65536, 768] 10.1 / 16.6).
+inline bool qmv_large_takes_mid(int x_dt, int sb_dt, int64_t m, int64_t cols, int gs, int bits) {
+    if (m > 8) return true;
+    const bool odd = bits == 3 || bits == 5 || bits == 6;
+    if (sb_dt != RQ_F32) {
+        if (bits == 2) return x_dt == RQ_F32 && m >= 5 && (m == 8 || cols % 512 != 0);
+        return odd && (m == 8 || (cols % 512 != 0 && !(bits == 3 && m == 1)));
+    }
+    if (odd) return gs == 32 || cols < 2048 || m > 4;
+    if (gs == 32) return x_dt != RQ_BF16 || m > (bits == 8 ? 1 : 2) || cols > 2048;
+    if (m <= 4) return bits == 8 && m >= 3 && cols < 2048;
+    return x_dt == RQ_F32 || cols > 2048;
+}
+
 // Whether a small launch that the split GEMV does not take (fp32 scales, group counts
 // that rule out whole-line loads) runs qmv_kernel with its waves splitting K, rather
 // than qmv_mid: bf16 x of up to 3 rows, where qmv_mid's 16-row MFMA tile is mostly

@@ -2184,12 +2184,7 @@ static hipError_t launch_bucket(const rq_problem* const* probs, int n, int x_dt,
     const int split_budget = rowblocks <= kSplitOneBlockMax ? kSplitLdsOneBlock : kLdsBudget;
     for (int i = 0; i < n && split && !fold; ++i)
         split = split_covers(*probs[i], sb_dt, m, gs, split_budget);
-    // At 5 to 8 rows the split GEMV takes two passes: qmv_mid is faster on few
-    // blocks of short rows and on more than two blocks a CU, slower between
-    // (m = 8: [768, 768] 5.3 -> 3.8 us, [2560, 2560] 7.4 -> 6.3, [10240, 2560]
-    // 14.9 -> 11.4, but [8192, 2048] 8.1 against 8.3, [2048, 8192] at m = 5 9.7
-    // against 10.9).
-    if (split && m > 4 && !fold && ((rowblocks <= 192 && K <= 4096) || rowblocks > 512)) split = false;
+    if (split && !fold && qmv_mid_over_split(x_dt, m, K, RQ_BITS, rowblocks)) split = false;
     if (split) {
         for (int base = 0; base < n; base += RQ_MAX_GROUPED) {
             const int cnt = (n - base) < RQ_MAX_GROUPED ? (n - base) : RQ_MAX_GROUPED;
@@ -2241,19 +2236,9 @@ static hipError_t launch_bucket(const rq_problem* const* probs, int n, int x_dt,
         }
         return hipSuccess;
     }
-    // Most of what else is small (more than 8 rows: [2048, 2048] at m = 12
-    // 11.7 us on qmv_kernel with the waves splitting K, 5.6 here, [8192, 2048] 13.6
-    // -> 8.3, [2048, 8192] 19 -> 10.9; fp32 scales at 6 bits and m = 1, fp32 x,
-    // [2048, 2048] 11.4 -> 7.2), and of the large launches those whose activation rows
-    // or scales cost qmv_kernel more: above 8 rows ([65536, 768] at m = 12 26 -> 17.6
-    // us, at m = 8 14.7 against 17.3), fp32 scales ([65536, 2048], 6 bits, m = 4
-    // 102 -> 78), and 8 rows, or rows of no whole 512 codes, at the widths other
-    // than 4 and 8 bits ([65536, 2048], 3 bits, m = 8 56 -> 50, m = 5 41 against
-    // 49; [65536, 768], m = 1 21.8 -> 20.7).
-    const bool odd_bits = RQ_BITS != 4 && RQ_BITS != 8;
     const bool ksplit = cfg == 0 && qmv_splits_k(x_dt, m, K, gs, RQ_BITS, rowblocks);
     if (K <= kMidMaxCols && !ksplit &&
-        (cfg == 0 || m > 8 || sb_dt == RQ_F32 || (odd_bits && (m == 8 || K % 512 != 0)))) {
+        (cfg == 0 || qmv_large_takes_mid(x_dt, sb_dt, m, K, gs, RQ_BITS))) {
         for (int base = 0; base < n; base += RQ_MAX_GROUPED) {
             const int cnt = (n - base) < RQ_MAX_GROUPED ? (n - base) : RQ_MAX_GROUPED;
             const hipError_t e = RQ_CAT(launch_qmv_mid_b, RQ_BITS)(probs + base, cnt, x_dt, sb_dt, y_dt,

@@ -18,6 +18,12 @@ extern "C" int takes_mid(int x_dt, int k64, int lora, long m, long rows, long co
 extern "C" int splits_k(int x_dt, long m, long cols, int gs, int bits, long rowblocks) {
     return rq::qmv_splits_k(x_dt, m, cols, gs, bits, rowblocks);
 }
+extern "C" int over_split(int x_dt, long m, long cols, int bits, long rowblocks) {
+    return rq::qmv_mid_over_split(x_dt, m, cols, bits, rowblocks);
+}
+extern "C" int large_mid(int x_dt, int sb_dt, long m, long cols, int gs, int bits) {
+    return rq::qmv_large_takes_mid(x_dt, sb_dt, m, cols, gs, bits);
+}
 """
 BF16, F32 = 0, 2
 
@@ -34,6 +40,8 @@ def choice(tmp_path_factory):
     lib.short_takes_128.argtypes = [ctypes.c_long] * 3 + [ctypes.c_int]
     lib.takes_mid.argtypes = [ctypes.c_int] * 3 + [ctypes.c_long] * 3 + [ctypes.c_int] * 2
     lib.splits_k.argtypes = [ctypes.c_int] + [ctypes.c_long] * 2 + [ctypes.c_int] * 2 + [ctypes.c_long]
+    lib.over_split.argtypes = [ctypes.c_int] + [ctypes.c_long] * 2 + [ctypes.c_int, ctypes.c_long]
+    lib.large_mid.argtypes = [ctypes.c_int] * 2 + [ctypes.c_long] * 2 + [ctypes.c_int] * 2
     return lib
 
 
@@ -86,3 +94,42 @@ def test_256_rows_outside_the_64_wide_stages(choice, x_dt, lora, m, rows, cols, 
     (BF16, 3, 10240, 10240, 64, 4, False)])
 def test_small_decode_launches_outside_the_split_gemv(choice, x_dt, m, rows, cols, gs, bits, ks):
     assert bool(choice.splits_k(x_dt, m, cols, gs, bits, (rows + 15) // 16)) == ks
+
+
+@pytest.mark.parametrize("x_dt,m,rows,cols,bits,mid", [
+    # us measured split GEMV / qmv_mid
+    (BF16, 8, 768, 768, 4, True),        # 5.5 / 4.1
+    (BF16, 5, 10240, 2560, 4, True),     # 12.8 / 11.2
+    (BF16, 5, 16384, 768, 4, False),     # 7.0 / 7.5
+    (BF16, 5, 2048, 2048, 6, False),     # 7.4 / 8.3
+    (BF16, 6, 16384, 4096, 2, False),    # 19.1 / 22.2
+    (F32, 5, 10240, 2560, 8, False),     # 12.8 / 13.7
+    (BF16, 8, 10240, 2560, 6, True),     # 20.1 / 17.5
+    (F32, 8, 10240, 2560, 5, False),     # 17.4 / 20.0
+    (BF16, 5, 1024, 1024, 3, True),      # 5.6 / 4.8
+    (BF16, 4, 768, 768, 4, False)])
+def test_5_to_8_decode_rows(choice, x_dt, m, rows, cols, bits, mid):
+    assert bool(choice.over_split(x_dt, m, cols, bits, (rows + 15) // 16)) == mid
+
+
+@pytest.mark.parametrize("x_dt,sb_dt,m,cols,gs,bits,mid", [
+    # us measured qmv_kernel / qmv_mid, 65536 rows unless noted; fp32 x at 1 and 2 rows
+    # counts twice
+    (BF16, BF16, 1, 768, 64, 2, False),    # 11.8 / 16.3
+    (BF16, BF16, 8, 2048, 64, 2, False),   # 28.6 / 38.9
+    (F32, BF16, 8, 768, 64, 2, True),      # 23.2 / 18.5
+    (BF16, BF16, 1, 768, 64, 3, False),    # 17.7 / 18.9
+    (BF16, BF16, 2, 768, 64, 6, True),     # 36.4 / 30.1
+    (BF16, BF16, 8, 2048, 64, 5, True),    # 82 / 70
+    (BF16, BF16, 9, 2048, 64, 4, True),
+    (BF16, F32, 1, 768, 64, 4, False),     # 10.1 / 16.6
+    (BF16, F32, 4, 2048, 64, 4, False),    # 26.7 / 38.8
+    (F32, F32, 4, 3072, 64, 4, False),     # 42 / 49 (49152 rows)
+    (BF16, F32, 8, 2048, 64, 4, False),    # 36.9 / 40.1
+    (F32, F32, 8, 2048, 64, 4, True),
+    (BF16, F32, 1, 2048, 32, 4, False),    # 27.7 / 37.9
+    (F32, F32, 4, 2048, 32, 4, True),
+    (BF16, F32, 1, 2048, 64, 6, False),    # 70 / 77
+    (BF16, F32, 2, 2048, 32, 6, True)])
+def test_large_decode_launches_outside_the_streamed_gemv(choice, x_dt, sb_dt, m, cols, gs, bits, mid):
+    assert bool(choice.large_mid(x_dt, sb_dt, m, cols, gs, bits)) == mid
