@@ -245,6 +245,9 @@ inline bool qmv_large_takes_mid(int x_dt, int sb_dt, int64_t m, int64_t cols, in
 // 4096] 8.9 / 8.3.  5 and 6 bits never, nor fp32 x, which qmv_kernel converts again
 // in every block, nor rows too long for its LDS ([2560, 10240], 3 rows, 17.8 / 12.8).
 inline bool qmv_splits_k(int x_dt, int64_t m, int64_t cols, int gs, int bits, int64_t rowblocks) {
+    // one long 8-bit form: [2560, 10240], bf16 scales, 2 rows, 13.7 / 15.8
+    if (x_dt == RQ_BF16 && bits == 8 && m == 2 && gs >= 64 && cols >= 8192 && cols <= 10240)
+        return rowblocks >= 128;
     if (x_dt != RQ_BF16 || m > 3 || bits == 5 || bits == 6 || m * cols > 12288) return false;
     if (gs == 32) return m <= 2 && rowblocks >= (bits == 2 || bits == 4 ? 512 : 1024);
     if (bits == 3) return m <= 2 && rowblocks >= 768 && cols >= 2048;

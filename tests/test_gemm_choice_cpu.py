@@ -91,6 +91,8 @@ def test_256_rows_outside_the_64_wide_stages(choice, x_dt, lora, m, rows, cols, 
     (BF16, 2, 16384, 4096, 128, 3, True),    # 21.4 / 22.9
     (BF16, 1, 12288, 3072, 128, 2, True),    # 10.2 / 14.5
     (BF16, 1, 16384, 4096, 32, 6, False),
+    (BF16, 2, 2560, 10240, 64, 8, True),     # 13.7 / 15.8, bf16 scales
+    (BF16, 2, 2560, 10240, 32, 8, False),    # 23.0 / 17.1
     (BF16, 3, 10240, 10240, 64, 4, False)])
 def test_small_decode_launches_outside_the_split_gemv(choice, x_dt, m, rows, cols, gs, bits, ks):
     assert bool(choice.splits_k(x_dt, m, cols, gs, bits, (rows + 15) // 16)) == ks
