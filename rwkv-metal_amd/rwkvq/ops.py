@@ -674,6 +674,8 @@ def qlora_product(x: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor, a: Ten
     fp32).  None elsewhere.  bf16 adapters, bf16 or fp32 x."""
     w_q, K, n_out, rank = _qlora_check(x, w_q, scales, biases, a, lora, transpose, group_size, bits)
     _on_gpu(x, w_q, scales, biases, a, lora)
+    if transpose and 0 < x.shape[0] <= 16:
+        return None   # what rq_qlora answers, without the buffers and the call
     x, w_q, scales, a, lora = _ready(x), _ready(w_q), _ready(scales), _ready(a), _ready(lora)
     biases = _ready(biases.to(scales.dtype))
     m = x.shape[0]
@@ -766,7 +768,7 @@ def quantized_matmul_lora(x: Tensor, w_q: Tensor, scales: Tensor, biases: Tensor
     lead = x.shape[:-1]
     x2, z2 = x.reshape(-1, n_in), z.reshape(-1, z.shape[-1])
     y = None
-    if z2.shape[-1] in (16, 32, 48, 64) and x2.shape[0] > 0:
+    if z2.shape[-1] in (16, 32, 48, 64) and x2.shape[0] >= 256:  # the 64-wide-stage kernels
         y = _qmm_lora_fused(x2, w_q, scales, biases, z2, lora, scale, transpose, group_size, bits)
     if y is None:
         y = quantized_matmul(x2, w_q, scales, biases, transpose, group_size, bits)

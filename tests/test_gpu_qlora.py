@@ -291,3 +291,27 @@ def test_qlora_launch_counts(rq, dev, transpose, M, R, K, rank, n):
         assert _launches(lambda: ops.qlora_product(x, wq, s, b, A, B, 2.0, True, 64, 4)) == n
     else:
         assert _launches(lambda: ops.qlora_dx_product(x, wq, s, b, A, B, 2.0, 64, 4)) == n
+
+
+@pytest.mark.parametrize("m", [1, 16])
+def test_decode_rows_make_no_call_that_declines(rq, dev, m, monkeypatch):
+    """Up to 16 forward rows: the library is not asked for products that it does not
+    fuse at that size."""
+    from rwkvq import _lib, ops
+    L = _lib.lib()
+
+    class Counting:
+        calls = []
+
+        def __getattr__(self, name):
+            self.calls.append(name)
+            return getattr(L, name)
+
+    g = torch.Generator().manual_seed(0)
+    lin = torch.nn.Linear(768, 512, bias=False, device=dev, dtype=torch.bfloat16)
+    lay = rq.LoRALinear(rank=32, base_module=rq.QuantizedLinear.from_linear(lin, 64, 4))
+    x = torch.randn(m, 768, generator=g).bfloat16().to(dev)
+    monkeypatch.setattr(ops, "lib", lambda: Counting())
+    with torch.no_grad():
+        lay(x)
+    assert Counting.calls == ["rq_lora_down", "rq_qmm"]
