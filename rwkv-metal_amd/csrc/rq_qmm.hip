@@ -11,15 +11,16 @@
 // Fewer than 256 activation rows of a forward product run rq_mid.hip, or against
 // many weight rows qmm_t (qmm_t_kernel below).
 //
-// qmm_n (qmm_n_kernel) covers the transposed products outside the 64-wide-stage
-// kernels below: block tile BM x 128 outputs, 64 weight rows per stage, 4 waves
-// in a 2x2 arrangement, v_mfma_f32_16x16x32_bf16 with fp32 accumulators.  Packed
-// weights are dequantized once per block per stage in registers (ŵ =
-// bf16(fma(scale, code, bias))) and written to LDS as bf16, transposed ([k][r]):
-// the contraction runs over the weight rows, and a thread dequantizes the same
-// run of two adjacent rows and writes (row, row+1) pairs as one dword per k.
-// LDS is double buffered and the next stage's global loads are issued before
-// the current stage's MFMAs.
+// qmm_n (qmm_n_kernel) covers transposed products of more than 2^26 weight rows
+// or columns, which neither the 64-wide-stage kernels below nor the short-batch
+// tiles (32-bit offsets inside a tile) take: block tile BM x 128 outputs, 64
+// weight rows per stage, 4 waves in a 2x2 arrangement,
+// v_mfma_f32_16x16x32_bf16 with fp32 accumulators.  Packed weights are
+// dequantized once per block per stage in registers (ŵ = bf16(fma(scale, code,
+// bias))) and written to LDS as bf16, transposed ([k][r]): the contraction runs
+// over the weight rows, and a thread dequantizes the same run of two adjacent
+// rows and writes (row, row+1) pairs as one dword per k.  LDS is double buffered
+// and the next stage's global loads are issued before the current stage's MFMAs.
 #include <type_traits>
 
 #include "rq_common.h"
